@@ -12,12 +12,12 @@
 // Jobs and their order. The top level of a pyramid comes first; the level
 // below it reads the top level's unsmoothed flow of the same frame
 // (flowfilter.cu:663-672), so its tiles wait, after their propagation
-// phase and before the update, until every tile of the top level has
-// signalled completion (a counter in device memory). Blocks are dispatched
-// in order on each XCD and producers never wait, so every producer a
-// consumer waits for is running or finished; the wait is also bounded by a
-// spin limit. Lower levels read the previous frame's flow of the level
-// above (the reference's ascending update order) and do not wait.
+// phase and before the update, until the few top-level tiles that cover
+// them have signalled completion (flags in device memory, wait_upper). Blocks
+// are dispatched in order on each XCD and producers never wait, so every
+// producer a consumer waits for is running or finished; the wait is also
+// bounded by a spin limit. Lower levels read the previous frame's flow of the level above (the
+// reference's ascending update order) and do not wait.
 //
 // Tile geometry: a workgroup is nw waves stacked vertically (nw is a launch
 // parameter, picked by timing the candidates); lane l of every wave owns
@@ -95,15 +95,25 @@ struct LevelJob {
     int W, H, Hu, Hsrc;  // level size, upper level height, image height
     int N, K, border, h0, TW, TH, tiles_x, tiles_y;
     int delta, img_mode, first_block;
-    // completion counters: wait until counter wait_idx has counted
-    // wait_target more tiles in this launch than before it; signal counter
-    // signal_idx. frame_slot >= 0: the level's image is a filter's input
-    // frame, which a launch may pass in place as its frame frame_slot (read
-    // where the caller keeps it).
-    int wait_idx, wait_target, frame_slot, signal_idx;
+    // wait_job >= 0: wait for tiles of that job of the table, which has
+    // wait_tx tiles across and its first tile's flags at wait_flags. Which
+    // of them: the first and last row (low and high half of the word
+    // wait_rows + r of the block map) for this job's tile row r, and the
+    // columns (word wait_rows + tiles_y + c) for its tile column c. flags
+    // >= 0: the job's tiles are waited for; tile t's flags are at flags + t.
+    // frame_slot >= 0: the level's image is a filter's input frame, which a
+    // launch may pass in place as its frame frame_slot (read where the
+    // caller keeps it).
+    int wait_job, wait_tx, wait_flags, wait_rows, flags, frame_slot;
     float dt, gamma, maxflow;
-    int pad_;
 };
+
+__device__ __forceinline__ int lane_id() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
+// A job in the constant address space: its fields are read with scalar loads
+// wherever they are used.
+#define FF_CONSTANT __attribute__((address_space(4)))
 
 // ------------------------------------------------------------ buffer access
 
@@ -212,49 +222,63 @@ __device__ __forceinline__ int xcd_tile(int b, int nt) {
     return (b % 8) * q + b / 8;
 }
 
-// ------------------------------------------------- completion counters
+// --------------------------------------------------- tiles waited for
 
-// Wait until the producer job's tiles have all signalled. The counters
-// only grow: a launch with sequence number `epoch` (1, 2, ... since the host
-// last cleared them) waits for epoch * wait_target, compared modulo 2^32.
-// Nothing is reset in the kernel, so the wait costs one relaxed load when the
-// producer is done (a returning atomic here would put a device-scope round
-// trip on every consumer tile's critical path). The data the producers
-// published (the unsmoothed flow) is read with device-coherent loads after
-// the wait, so no cache invalidation is needed; the workgroup barrier
-// orders every wave's loads after the polling thread saw the count.
-// The wait gives up after `spin_limit` polls and counts a timeout (the host
-// reports it as an error); `bias` is added to the target (0, or a count no
-// launch reaches, which a test uses to make the wait give up).
-__device__ __forceinline__ void wait_upper(const LevelJob& p, unsigned* counters, int timeout_idx, unsigned epoch,
-                                           int spin_limit, unsigned bias) {
-    if (threadIdx.x == 0) {
-        const unsigned* done = counters + 2 * p.wait_idx;
-        const unsigned target = epoch * (unsigned)p.wait_target + bias;
-        int spins = 0;
-        while ((int)(__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {
-            __builtin_amdgcn_s_sleep(8);
-            if (++spins > spin_limit) {
-                __hip_atomic_fetch_add(counters + timeout_idx, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                break;
-            }
-        }
-    }
-    __syncthreads();
+// Flags of the top-level tiles that a launch's other tiles wait for: a word
+// each, which the launch sets to its sequence number `epoch` (1, 2, ... since
+// the host last cleared the flags) when the tile is done, so that nothing is
+// reset in the kernel. `started` (may be null) counts all such tiles of all
+// launches on the device as they start (WaitingLaunch).
+struct TileFlags {
+    unsigned* done;
+    unsigned* timeouts;  // count of the waits that gave up
+    unsigned* started;
+    unsigned epoch;
+};
+
+// Blocks are grouped by tile body: top levels with float, u8, reduced u8
+// and twice-reduced u8 images, then delta levels with float, u8 and reduced
+// u8 images; ends[i] is the first block after group i. (Selecting the body
+// from the block index rather than from a job field also keeps the
+// compiler's register allocation of each body as tight as in a kernel of
+// its own.)
+struct GroupEnds {
+    int e[6];
+};
+
+// Arguments of the frame kernel, in one struct that any place reads from the
+// kernel's argument segment (launch_args).
+struct WaitArgs {
+    int spin_limit;
+    unsigned bias;
+};
+struct FrameArgs {
+    const unsigned char* ptr[kMaxLaunchFrames];
+    int pitch[kMaxLaunchFrames];
+};
+struct LaunchArgs {
+    const LevelJob* jobs;
+    const int* block_job;
+    TileFlags fl;
+    GroupEnds ends;
+    int nw;
+    WaitArgs wa;
+    FrameArgs frames;
+};
+__device__ __forceinline__ const LaunchArgs& launch_args() {
+    auto* q = (const FF_CONSTANT LaunchArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    return *(const LaunchArgs*)q;
 }
 
-// Count this tile as done once its device-coherent stores have completed:
-// every wave waits for its outstanding stores (vmcnt 0; the immediate
-// leaves the other counters unwaited), the barrier joins the waves, and one
-// thread increments the counter.
-__device__ __forceinline__ void signal_done(const LevelJob& p, unsigned* counters) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (threadIdx.x == 0)
-        __hip_atomic_fetch_add(counters + 2 * p.signal_idx, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ unsigned flag_load(const unsigned* f) {
+    return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-// ------------------------------------------------------------ tile body
+__device__ __forceinline__ void flag_store(unsigned* f, unsigned v) {
+    __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void flag_add(unsigned* f) {
+    __hip_atomic_fetch_add(f, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Per-thread view of the tile.
 struct Geo {
@@ -264,6 +288,72 @@ struct Geo {
     bool xin;      // column strictly inside the propagation border
     bool wave_in;  // every pixel of the wave strictly inside the border
 };
+
+// The tiles of the upper level that tile t waits for: first, first + 1, ..,
+// nx of them across, n in all.
+struct UpperTiles {
+    int first, nx, n;
+    // the i-th of them
+    __device__ __forceinline__ int tile(int i, const LevelJob& p) const { return first + i / nx * p.wait_tx + i % nx; }
+};
+__device__ __forceinline__ UpperTiles upper_tiles(const LevelJob& p, int t) {
+    const int ty = t / p.tiles_x, tx = t - ty * p.tiles_x;
+    const auto* w = (const FF_CONSTANT unsigned*)launch_args().block_job + p.wait_rows;
+    const unsigned rows = w[ty], cols = w[p.tiles_y + tx];
+    const int ty0 = (int)(rows & 0xffffu), tx0 = (int)(cols & 0xffffu);
+    const int nx = (int)(cols >> 16) - tx0 + 1;
+    return UpperTiles{ty0 * p.wait_tx + tx0, nx, ((int)(rows >> 16) - ty0 + 1) * nx};
+}
+
+// Wait for the tiles u of the upper level. Waiting for these few alone lets a
+// tile go on as soon as they are there, whatever the rest of the level does
+// (a 2048x1088 two-level launch took 54.6 us when every tile waited for the
+// whole level, 52.2 us so). The first wave polls, a lane per tile, with
+// relaxed loads (the flow the producers published is read with
+// device-coherent loads after the wait, so no cache needs invalidating), and
+// the barrier holds the others. The wait gives up after `spin_limit` polls
+// and counts a timeout (the host reports it as an error). `bias` is added to
+// the number waited for (0, or what no launch writes, which a test uses to
+// make the wait give up).
+__device__ __forceinline__ void wait_upper(const LevelJob& p, const UpperTiles& u, const Geo& g) {
+    if (g.wave == 0) {
+        const TileFlags& fl = launch_args().fl;
+        const int spin_limit = launch_args().wa.spin_limit;
+        const unsigned bias = launch_args().wa.bias;
+        int spins = 0;
+        for (int first = 0; first < u.n; first += LANES) {
+            const unsigned* done = fl.done + p.wait_flags + u.tile(min(first + g.lane, u.n - 1), p);
+            while (__ballot(flag_load(done) != fl.epoch + bias)) {
+                __builtin_amdgcn_s_sleep(8);
+                if (++spins > spin_limit) {
+                    if (g.lane == 0) flag_add(fl.timeouts);
+                    first = u.n;
+                    break;
+                }
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// Count an awaited tile as started.
+__device__ __forceinline__ void signal_started(const Geo& g) {
+    unsigned* started = launch_args().fl.started;
+    if (started && g.wave == 0 && g.lane == 0) flag_add(started);
+}
+
+// Mark tile t as done once its device-coherent stores have completed: every
+// wave waits for its outstanding stores (vmcnt 0; the immediate leaves the
+// other counters unwaited), the barrier joins the waves, and one thread
+// writes the flag.
+__device__ __forceinline__ void signal_done(const LevelJob& p, int t, const Geo& g) {
+    const TileFlags& fl = launch_args().fl;
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if (g.wave == 0 && g.lane == 0) flag_store(fl.done + p.flags + t, fl.epoch);
+}
+
+// ------------------------------------------------------------ tile body
 
 // Registers of the level state: flow (fu, fv) and, on delta levels, the
 // scalar (old brightness) and vector (delta flow) payloads.
@@ -645,16 +735,6 @@ __device__ __forceinline__ float* xrow(float* xch, int nw, int slot, int wave) {
     return xch + ((slot * nw + wave) * 10) * LANES;
 }
 
-// Per-launch arguments of the frame kernel besides the job table.
-struct WaitArgs {
-    int spin_limit;
-    unsigned bias;
-};
-struct FrameArgs {
-    const unsigned char* ptr[kMaxLaunchFrames];
-    int pitch[kMaxLaunchFrames];
-};
-
 // INNER: a tile whose every pixel lies inside the border, away from the
 // image edges (every wave inside, no edge lanes, no clamped rows, no
 // column or row beyond the image): one straight-line body with no per-wave
@@ -663,15 +743,20 @@ struct FrameArgs {
 // ALLOW_INNER: interior tiles take that body (a kernel instantiation of
 // its own, since the second body changes the register allocation of the
 // first). Other tiles choose per wave.
+// t: the tile, row by row from the top.
 template <bool DELTA, int MODE, int R, bool ALLOW_INNER, bool INNER = false>
-__device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* xch, int nw, unsigned* counters, unsigned epoch,
-                                           int timeout_idx, const WaitArgs& wa, ImgSrc frame) {
+__device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch, int nw,
+                                           ImgSrc frame) {
+    
     Geo g;
-    g.lane = threadIdx.x & (LANES - 1);
-    g.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int t = xcd_tile(tile, p.tiles_x * p.tiles_y);
-    const int tyi = t / p.tiles_x, txi = t - tyi * p.tiles_x;
+    // the lane from the hardware's count, so that threadIdx.x takes no
+    // register beyond the next line
+    g.lane = lane_id();
+    g.wave = wave_id();
+    if constexpr (!DELTA && !INNER)
+        if (p.flags >= 0) signal_started(g);
     // output range of the tile and the buffer around it, clamped into the image
+    const int tyi = t / p.tiles_x, txi = t - tyi * p.tiles_x;
     const int ox0 = txi * p.TW, ox1 = min(ox0 + p.TW, p.W);
     const int oy0 = tyi * p.TH, oy1 = min(oy0 + p.TH, p.H);
     const int x0 = clampi(ox0 - p.h0, 0, p.W - LANES);
@@ -681,7 +766,7 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* x
         // propagation border is 0
         const int bb = max(p.border, 1);
         if (x0 >= bb && x0 + LANES - 1 < p.W - bb && y0 >= bb && y0 + nw * R - 1 < p.H - bb) {
-            level_tile<DELTA, MODE, R, true, true>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, frame);
+            level_tile<DELTA, MODE, R, true, true>(p, t, xch, nw, frame);
             return;
         }
     }
@@ -710,8 +795,10 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* x
 
     const Rsrc rfi = rsrc(p.flow_in, p.flow_in_pitch * p.H);
     const Rsrc rai = rsrc(p.a0_in, p.a0_in_pitch * p.H);
-    const Rsrc rfo = rsrc(p.flow_out, p.flow_out_pitch * p.H);
-    const Rsrc rao = rsrc(p.a0_out, p.a0_out_pitch * p.H);
+
+    // (looked up here, so that the wait is one load from the flags)
+    UpperTiles u{0, 1, 0};
+    if (DELTA && p.wait_job >= 0) u = upper_tiles(p, t);
 
     State<DELTA, R> s;
 
@@ -734,6 +821,7 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* x
 
     int slot = 0;
 
+    {
     // ---------------------------------------------------------- propagation
     // N iterations of an X and a Y pass; the last one separately, since on
     // a delta level part of its flow output is dead
@@ -795,11 +883,15 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* x
     for (int it = 0; it + 1 < p.N; ++it) iteration(std::false_type{});
     iteration(std::true_type{});
 
+    }
     // ------------------------------------------------ image model + update
-    if (DELTA && p.wait_idx >= 0) wait_upper(p, counters, timeout_idx, epoch, wa.spin_limit, wa.bias);
+    {
+    if (DELTA && p.wait_job >= 0) wait_upper(p, u, g);
     float aold[R];  // unused (and removed) on delta levels
     float2 up[R];
     int offa[R], offf[R];
+    const Rsrc rai = rsrc(p.a0_in, p.a0_in_pitch * p.H);
+    const Rsrc rao = rsrc(p.a0_out, p.a0_out_pitch * p.H);
     const Rsrc rdf = rsrc(p.dflow_out, p.dflow_out_pitch * p.H);
     const Rsrc rfu = rsrc(p.flow_upd, p.flow_upd_pitch * p.H);
     const int xmx = DELTA ? p.xmap[g.xl] : 0;
@@ -825,6 +917,7 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* x
     if (!INNER && xedge) model_update<DELTA, true, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf);
     else model_update<DELTA, false, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf);
 
+    }
     // ------------------------------------------------------------ smoothing
     // flowSmoothX_k / flowSmoothY_k (flowsmoothing_k.cu:21-87), K times.
     for (int it = 0; it < p.K; ++it) {
@@ -865,6 +958,8 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* x
         else smooth_y<false, R>(s.fu, s.fv, a2u, a2v, a1u, a1v, b1u, b1v, b2u, b2v, rlast);
     }
 
+    {
+    const Rsrc rfo = rsrc(p.flow_out, p.flow_out_pitch * p.H);
     // ------------------------------------------------- write the new state
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -872,18 +967,9 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int tile, float* x
         const bool out = out_x && y >= oy0 && y < oy1;
         st2(rfo, out ? y * p.flow_out_pitch + g.x * 8 : OOB, s.fu[r], s.fv[r]);
     }
-    if (!DELTA && p.signal_idx >= 0) signal_done(p, counters);
+    if (!DELTA && p.flags >= 0) signal_done(p, t, g);
+    }
 }
-
-// Blocks are grouped by tile body: top levels with float, u8, reduced u8
-// and twice-reduced u8 images, then delta levels with float, u8 and reduced
-// u8 images; ends[i] is the first block after group i. (Selecting the body
-// from the block index rather than from a job field also keeps the
-// compiler's register allocation of each body as tight as in a kernel of
-// its own.)
-struct GroupEnds {
-    int e[6];
-};
 
 // Rows per thread of a tile body: RLOW, except for top levels reduced on
 // load (the top level of a pyramid, which the level below waits for), which
@@ -904,29 +990,46 @@ struct TileShape {
 };
 constexpr TileShape kShapes[] = {{4, 8, false}, {8, 8, false}, {4, 4, false}, {4, 4, true}};
 
-template <int RTOP, int RLOW = kRows, bool INNER = false>
-__global__ void __launch_bounds__(1024, RLOW == 4 ? 8 : 1)
-    k_fused_frame(const LevelJob* __restrict__ jobs, const int* __restrict__ block_job, unsigned* counters,
-                  unsigned epoch, int timeout_idx, GroupEnds ends, int nw, WaitArgs wa, FrameArgs frames) {
-    // row exchange between the waves of the workgroup (2 * nw * 10 * LANES floats)
-    extern __shared__ float xch[];
-    const LevelJob& p = jobs[block_job[blockIdx.x]];
-    const int tile = (int)blockIdx.x - p.first_block;
-    const unsigned b = blockIdx.x;
-    // the job's input frame passed in place, if any (frame_slot is
-    // uniform, so is the selection)
-    ImgSrc fr{nullptr, 0};
-    if (p.frame_slot >= 0) fr = ImgSrc{frames.ptr[p.frame_slot], frames.pitch[p.frame_slot]};
-    if (b < (unsigned)ends.e[0]) level_tile<false, IMG_F32, RLOW, INNER>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, fr);
-    else if (b < (unsigned)ends.e[1]) level_tile<false, IMG_U8, RLOW, INNER>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, fr);
-    else if (b < (unsigned)ends.e[2]) level_tile<false, IMG_U8_DOWN, RTOP, INNER>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, fr);
-    else if (b < (unsigned)ends.e[3]) level_tile<false, IMG_U8_DOWN2, RTOP, INNER>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, fr);
-    else if (b < (unsigned)ends.e[4]) level_tile<true, IMG_F32, RLOW, INNER>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, fr);
-    else if (b < (unsigned)ends.e[5]) level_tile<true, IMG_U8, RLOW, INNER>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, fr);
-    else level_tile<true, IMG_U8_DOWN, RLOW, INNER>(p, tile, xch, nw, counters, epoch, timeout_idx, wa, fr);
+// The job of block b, its tile there, and its input frame if the launch passes
+// it in place (frame_slot is uniform, so is the selection).
+__device__ __forceinline__ const LevelJob& job_of_block(unsigned b) {
+    const LaunchArgs& a = launch_args();
+    return *(const LevelJob*)((const FF_CONSTANT LevelJob*)a.jobs + ((const FF_CONSTANT int*)a.block_job)[b]);
+}
+__device__ __forceinline__ int job_tile(const LevelJob& p, unsigned b) {
+    return xcd_tile((int)b - p.first_block, p.tiles_x * p.tiles_y);
+}
+__device__ __forceinline__ ImgSrc frame_of(const LevelJob& p) {
+    if (p.frame_slot < 0) return ImgSrc{nullptr, 0};
+    const FrameArgs& f = launch_args().frames;
+    return ImgSrc{f.ptr[p.frame_slot], f.pitch[p.frame_slot]};
 }
 
-__global__ void k_clear_counters(unsigned* c, int n) {
+template <int RTOP, int RLOW = kRows, bool INNER = false>
+__global__ void __launch_bounds__(1024, RLOW == 4 ? 8 : 1) k_fused_frame(LaunchArgs) {
+    // row exchange between the waves of the workgroup (2 * nw * 10 * LANES floats)
+    extern __shared__ float xch[];
+    const unsigned b = blockIdx.x;
+    const LevelJob& q = job_of_block(b);
+    const int t = job_tile(q, b);
+    const ImgSrc fr = frame_of(q);
+    const int nw = launch_args().nw;
+    const GroupEnds& ends = launch_args().ends;
+    if (b < (unsigned)ends.e[0]) level_tile<false, IMG_F32, RLOW, INNER>(q, t, xch, nw, fr);
+    else if (b < (unsigned)ends.e[1]) level_tile<false, IMG_U8, RLOW, INNER>(q, t, xch, nw, fr);
+    else if (b < (unsigned)ends.e[2]) level_tile<false, IMG_U8_DOWN, RTOP, INNER>(q, t, xch, nw, fr);
+    else if (b < (unsigned)ends.e[3]) level_tile<false, IMG_U8_DOWN2, RTOP, INNER>(q, t, xch, nw, fr);
+    else if (b < (unsigned)ends.e[4]) level_tile<true, IMG_F32, RLOW, INNER>(q, t, xch, nw, fr);
+    else if (b < (unsigned)ends.e[5]) level_tile<true, IMG_U8, RLOW, INNER>(q, t, xch, nw, fr);
+    else level_tile<true, IMG_U8_DOWN, RLOW, INNER>(q, t, xch, nw, fr);
+}
+
+__global__ void __launch_bounds__(LANES) k_wait_started(const unsigned* word, unsigned target) {
+    int spins = 0;
+    while ((int)(flag_load(word) - target) < 0 && ++spins < kSpinLimit / 8) __builtin_amdgcn_s_sleep(8);
+}
+
+__global__ void k_clear_flags(unsigned* c, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) c[i] = 0u;
 }
@@ -971,6 +1074,10 @@ bool tiles_with(const LevelArgs& a, int rows) {
 }
 
 }  // namespace
+
+void launch_wait_started(const unsigned* word, unsigned target, hipStream_t s) {
+    hipLaunchKernelGGL(k_wait_started, dim3(1), dim3(LANES), 0, s, word, target);
+}
 
 bool fused_level_supported(const LevelArgs& a) {
     if (a.border < 1 || a.prop_iters < 1 || a.smooth_iters < 1) return false;
@@ -1042,18 +1149,18 @@ struct FusedFrame::Impl {
         bool inner = false;  // launched as k_fused_frame<4, 4, true>
         size_t map_offset = 0;
         unsigned long long token = 0;
-        bool waits = false;  // some job waits for another
+        int awaited = 0;  // tiles that others wait for
     };
     Table slot[2];
     int next = 0;
     unsigned long long uploads = 0;
-    // Completion counters: one region of `npairs` (done, spare) pairs per
-    // table slot (the two slots alternate when a filter's state buffers
-    // ping-pong between frames), then the timeout count.
-    DeviceArray counters;
-    int npairs = 0;
-    // per slot: launches counted since its region was last cleared, and the
-    // table they count for (0: clear before the next launch)
+    // Flags of the tiles waited for: per table slot (the two slots alternate
+    // when a filter's state buffers ping-pong between frames) nflags words;
+    // then the count of the waits that gave up.
+    DeviceArray flags;
+    int nflags = 0;
+    // per slot: launches since its flags were last cleared, and the table
+    // they were for (0: clear before the next launch)
     unsigned epoch[2] = {0, 0};
     unsigned long long counted[2] = {0, 0};
     // waves per workgroup, top-level rows per thread, other rows per thread;
@@ -1067,9 +1174,9 @@ struct FusedFrame::Impl {
     int test_spins = 0;  // > 0: the waits give up after this many polls (test hook)
 
     int table(const std::vector<LevelArgs>& jobs, int nw, int rtop, int rlow, bool inner, hipStream_t s);
-    unsigned* region(int si) const { return (unsigned*)counters.data() + (size_t)si * 2 * npairs; }
-    int timeout_word() const { return 4 * npairs; }
-    void clear_counters(int si, hipStream_t s) const;
+    unsigned* region(int si) const { return (unsigned*)flags.data() + (size_t)si * nflags; }
+    unsigned* timeout_word() const { return (unsigned*)flags.data() + (size_t)2 * nflags; }
+    void clear_flags(int si, hipStream_t s) const;
     void run(int t, hipStream_t s, const FrameRef* frames = nullptr, int nframes = 0);
     void tune(const std::vector<LevelArgs>& jobs, hipStream_t s);
 };
@@ -1140,8 +1247,8 @@ int FusedFrame::Impl::table(const std::vector<LevelArgs>& jobs, int nw, int rtop
         p.delta = a.delta;
         p.img_mode = a.img_mode;
         p.first_block = blocks;
-        p.wait_idx = -1;
-        p.signal_idx = -1;
+        p.wait_job = -1;
+        p.flags = -1;
         p.frame_slot = a.frame_slot < kMaxLaunchFrames ? a.frame_slot : -1;
         p.dt = a.dt;
         p.gamma = a.gamma;
@@ -1156,13 +1263,31 @@ int FusedFrame::Impl::table(const std::vector<LevelArgs>& jobs, int nw, int rtop
         if (!jobs[i].delta || jobs[k].delta) throw logic_error("fused frame: only delta levels wait on a top level");
         LevelJob& c = rec[pos[i]];
         LevelJob& q = rec[pos[k]];
-        c.wait_idx = pos[k];
-        c.wait_target = q.tiles_x * q.tiles_y;
-        q.signal_idx = pos[k];
+        // top levels come first, so their block indices are compact
+        q.flags = q.first_block;
+        c.wait_job = pos[k];
+        c.wait_tx = q.tiles_x;
+        c.wait_flags = q.flags;
     }
     std::vector<int> map(blocks);
     for (size_t i = 0; i < rec.size(); ++i)
         for (int b = 0; b < rec[i].tiles_x * rec[i].tiles_y; ++b) map[rec[i].first_block + b] = (int)i;
+    // the upper level's tiles that each tile row and column waits for: the
+    // results of a tile's update reach 2 K pixels further (the smoothing), and
+    // the upper flow read beyond that, finished or not, reaches no output
+    for (LevelJob& c : rec) {
+        if (c.wait_job < 0) continue;
+        const LevelJob& q = rec[c.wait_job];
+        c.wait_rows = (int)map.size();
+        auto ranges = [&](int tiles, int size, int n, int nu, int upper_size) {
+            for (int i = 0; i < tiles; ++i) {
+                const int lo = std::max(i * size - 2 * c.K, 0), hi = std::min(std::min(i * size + size, n) - 1 + 2 * c.K, n - 1);
+                map.push_back(upper_index(lo, n, nu) / upper_size | (upper_index(hi, n, nu) / upper_size) << 16);
+            }
+        };
+        ranges(c.tiles_y, c.TH, c.H, q.H, q.TH);
+        ranges(c.tiles_x, c.TW, c.W, q.W, q.TW);
+    }
 
     const size_t jobs_bytes = rec.size() * sizeof(LevelJob);
     const size_t map_offset = (jobs_bytes + 255) & ~size_t(255);
@@ -1180,22 +1305,26 @@ int FusedFrame::Impl::table(const std::vector<LevelArgs>& jobs, int nw, int rtop
     key.push_back(inner ? 1 : 0);
 
     for (int i = 0; i < 2; ++i)
-        if (slot[i].key == key) return i;
+        if (slot[i].key == key) {
+            next = i ^ 1;  // the one used less recently is replaced
+            return i;
+        }
 
-    // a table (or the counters) may be in use by launches still in flight
-    // on the stream
+    // a table (or the flags) may be in use by launches still in flight on
+    // the stream
     FF_HIP(hipStreamSynchronize(s));
-    const int need = (int)jobs.size();
-    if (npairs < need) {
-        const int n = need < 64 ? 64 : need;
+    const int need = ends[3];  // tiles of top levels
+    if (nflags < need || !flags.data()) {
+        const int n = std::max(need, 256);
         // the timed-out waits counted so far are kept
         watch->stream = s;
         watch->read();
-        std::vector<unsigned> zero(4 * (size_t)n + 2, 0u);
-        counters.assign(zero.data(), zero.size() * sizeof(unsigned));
-        npairs = n;
-        watch->retire((const unsigned*)counters.data() + timeout_word());
-        // launches recorded with the old counters must not be replayed
+        std::vector<unsigned> zero(2 * (size_t)n + 1, 0u);
+        flags.assign(zero.data(), zero.size() * sizeof(unsigned));
+        nflags = n;
+        watch->retire(timeout_word());
+        // launches recorded with the old flags must not be replayed, and the
+        // new ones count from the start
         for (Table& o : slot) o.token = ++uploads;
     }
     const int si = next;
@@ -1209,17 +1338,18 @@ int FusedFrame::Impl::table(const std::vector<LevelArgs>& jobs, int nw, int rtop
     t.rlow = rlow;
     t.inner = inner;
     t.map_offset = map_offset;
-    t.waits = false;
-    for (const LevelJob& r : rec) t.waits = t.waits || r.wait_idx >= 0;
+    t.awaited = 0;
+    for (const LevelJob& r : rec)
+        if (r.flags >= 0) t.awaited += r.tiles_x * r.tiles_y;
     for (int g = 0; g < kGroups - 1; ++g) t.ends.e[g] = ends[g];
     t.token = ++uploads;
     next ^= 1;
     return si;
 }
 
-void FusedFrame::Impl::clear_counters(int si, hipStream_t s) const {
-    const int n = 2 * npairs;
-    hipLaunchKernelGGL(k_clear_counters, dim3((n + 255) / 256), dim3(256), 0, s, region(si), n);
+void FusedFrame::Impl::clear_flags(int si, hipStream_t s) const {
+    const int n = nflags;
+    hipLaunchKernelGGL(k_clear_flags, dim3((n + 255) / 256), dim3(256), 0, s, region(si), n);
 }
 
 void FusedFrame::Impl::run(int ti, hipStream_t s, const FrameRef* frames, int nframes) {
@@ -1239,21 +1369,21 @@ void FusedFrame::Impl::run(int ti, hipStream_t s, const FrameRef* frames, int nf
     if (lds_ok8 != hipSuccess) throw_hip(lds_ok8, "hipFuncSetAttribute", __FILE__, __LINE__);
     if (lds_ok44 != hipSuccess) throw_hip(lds_ok44, "hipFuncSetAttribute", __FILE__, __LINE__);
     if (lds_ok44i != hipSuccess) throw_hip(lds_ok44i, "hipFuncSetAttribute", __FILE__, __LINE__);
-    // Sequence number of this launch for its slot's completion counters. A
-    // launch recorded into a graph clears them itself and counts as the
-    // first, so every replay is self-contained; direct launches count up
-    // from the last clear, which happens whenever the region served another
-    // table or a replay (replayed()) in between.
+    // Sequence number of this launch for its slot's flags. A launch recorded
+    // into a graph clears them itself and counts as the first, so every
+    // replay is self-contained; direct launches count up from the last
+    // clear, which happens whenever the region served another table or a
+    // replay (replayed()) in between.
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     FF_HIP(hipStreamIsCapturing(s, &cs));
     unsigned e;
     if (cs != hipStreamCaptureStatusNone) {
-        clear_counters(si, s);
+        if (t.awaited) clear_flags(si, s);
         e = 1;
         counted[si] = 0;
     } else {
-        if (counted[si] != t.token || epoch[si] == 0xffffffffu) {
-            clear_counters(si, s);
+        if (counted[si] != t.token || epoch[si] == 0x3fffffffu) {
+            if (t.awaited) clear_flags(si, s);
             epoch[si] = 0;
             counted[si] = t.token;
         }
@@ -1267,28 +1397,22 @@ void FusedFrame::Impl::run(int ti, hipStream_t s, const FrameRef* frames, int nf
         fa.pitch[k] = (int)frames[k].pitch;
     }
     watch->stream = s;
-    if (t.waits) watch->pending = true;
-    const WaitingLaunch order(s, t.waits);
+    if (t.awaited) watch->pending = true;
+    const WaitingLaunch order(s, t.awaited);
     ProfileScope ps("fused_frame", s);
     const char* base = (const char*)t.dev.data();
-    // the timeout word, relative to this slot's region
-    const int timeout_idx = timeout_word() - si * 2 * npairs;
+    const TileFlags fl{region(si), timeout_word(), order.started(), e};
+    const LaunchArgs args{(const LevelJob*)base, (const int*)(base + t.map_offset), fl, t.ends, t.nw, wa, fa};
+    const dim3 grid(t.blocks), blk(t.nw * LANES);
+    const size_t lds = lds_bytes(t.nw);
     if (t.rlow == 4 && t.inner)
-        hipLaunchKernelGGL((k_fused_frame<4, 4, true>), dim3(t.blocks), dim3(t.nw * LANES), lds_bytes(t.nw), s,
-                           (const LevelJob*)base, (const int*)(base + t.map_offset), region(si), e, timeout_idx, t.ends,
-                           t.nw, wa, fa);
+        hipLaunchKernelGGL((k_fused_frame<4, 4, true>), grid, blk, lds, s, args);
     else if (t.rlow == 4)
-        hipLaunchKernelGGL((k_fused_frame<4, 4>), dim3(t.blocks), dim3(t.nw * LANES), lds_bytes(t.nw), s,
-                           (const LevelJob*)base, (const int*)(base + t.map_offset), region(si), e, timeout_idx, t.ends,
-                           t.nw, wa, fa);
+        hipLaunchKernelGGL((k_fused_frame<4, 4>), grid, blk, lds, s, args);
     else if (t.rtop == 8)
-        hipLaunchKernelGGL(k_fused_frame<8>, dim3(t.blocks), dim3(t.nw * LANES), lds_bytes(t.nw), s,
-                           (const LevelJob*)base, (const int*)(base + t.map_offset), region(si), e, timeout_idx, t.ends,
-                           t.nw, wa, fa);
+        hipLaunchKernelGGL(k_fused_frame<8>, grid, blk, lds, s, args);
     else
-        hipLaunchKernelGGL(k_fused_frame<4>, dim3(t.blocks), dim3(t.nw * LANES), lds_bytes(t.nw), s,
-                           (const LevelJob*)base, (const int*)(base + t.map_offset), region(si), e, timeout_idx, t.ends,
-                           t.nw, wa, fa);
+        hipLaunchKernelGGL(k_fused_frame<4>, grid, blk, lds, s, args);
 }
 
 // Time the launches of every candidate tiling (waves per workgroup and, when
@@ -1398,7 +1522,7 @@ void FusedFrame::replayed() { impl_->counted[0] = impl_->counted[1] = 0; }
 
 int FusedFrame::blocks(int table) const { return impl_->slot[table & 1].blocks; }
 unsigned long long FusedFrame::token(int table) const { return impl_->slot[table & 1].token; }
-bool FusedFrame::waits(int table) const { return impl_->slot[table & 1].waits; }
+int FusedFrame::awaited(int table) const { return impl_->slot[table & 1].awaited; }
 
 void FusedFrame::setWaves(int nw) {
     bool ok = nw == 0;

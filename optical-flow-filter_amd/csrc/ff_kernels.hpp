@@ -141,6 +141,12 @@ struct LevelArgs {
     int frame_slot = -1;
 };
 
+// Upper-level texel that column (or row) x of n reads of nu: the
+// normalized-coordinate point sampling of deltaFlowUpdate_k
+// (update_k.cu:151-155), min(floor(fl(x/(n-1)) * nu), nu-1); xmap and ymap
+// hold it for every column and row (ff_stages.cpp).
+int upper_index(int x, int n, int nu);
+
 // A frame a fused launch reads in place: device u8 image, row pitch in
 // bytes (multiples of 4; pitch * rows below 2^31).
 struct FrameRef {
@@ -180,11 +186,15 @@ struct WaitCheck {
     void check(const char* who);
 };
 
+// One wave on stream s that ends once *word has reached target (compared
+// modulo 2^32; bounded by a spin limit). See WaitingLaunch.
+void launch_wait_started(const unsigned* word, unsigned target, hipStream_t s);
+
 // Returns false when the level's parameters are outside what the fused
 // kernel handles (the caller then runs the stage kernels).
 bool fused_level_supported(const LevelArgs& a);
 
-// Device tables and completion counters of fused frame launches. prepare()
+// Device tables and tile flags of fused frame launches. prepare()
 // builds the job table of a list of levels (uploading it, after waiting for
 // the work on stream s, when it matches none of the two most recent tables),
 // choosing the tile height by timing the candidates the first time it sees
@@ -207,7 +217,7 @@ public:
     // its ptr is not null).
     void launch(int table, hipStream_t s, const FrameRef* frames = nullptr, int nframes = 0);
     // A graph holding launches of this frame was replayed on the stream:
-    // the next direct launch clears the completion counters first.
+    // the next direct launch clears the tile flags first.
     void replayed();
     // Waves per workgroup (a tile's buffer is 64 columns by waves * rows
     // per thread rows): 0 = autotune (default), or 16, 15, 8, 5, 4. waves()
@@ -247,8 +257,8 @@ public:
     // whenever that memory is replaced, so recorded launches (graphs) keyed
     // by it never refer to freed memory.
     unsigned long long token(int table) const;
-    // Whether some job of the table waits for another (see WaitingLaunch).
-    bool waits(int table) const;
+    // Tiles of the table that other tiles of it wait for (see WaitingLaunch).
+    int awaited(int table) const;
 
 private:
     struct Impl;

@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <set>
 #include <sstream>
@@ -33,8 +34,7 @@ void check_launch(const char* what) {
 // ------------------------------------------------------------------ stream
 
 namespace {
-// The streams of live StreamBoxes, which WaitingLaunch may mark after the
-// fact (defined with WaitingLaunch below).
+// The streams of live StreamBoxes (defined with WaitingLaunch below).
 void owned_insert(hipStream_t s);
 void owned_erase(hipStream_t s);
 }  // namespace
@@ -42,7 +42,7 @@ void owned_erase(hipStream_t s);
 StreamBox::~StreamBox() {
     if (ev_) (void)hipEventDestroy(ev_);
     if (own_) {
-        // finish first: then no launch on it is left to order, and a new
+        // finish first: then no launch on it is left to wait for, and a new
         // stream may be given the same handle
         (void)hipStreamSynchronize(own_);
         owned_erase(own_);
@@ -439,20 +439,14 @@ void Image::swapBuffers(Image& o) {
 // ------------------------------------------------------------ WaitingLaunch
 
 namespace {
-// What marks the end of a device's last waiting launch:
-//  NONE:     nothing needs marking (no such launch, or its stream finished);
-//  PENDING:  it ran on a live library stream and is not marked yet: an event
-//            recorded on that stream when another stream launches marks it
-//            (with whatever was queued there since, which only orders more);
-//  RECORDED: `done` was recorded right after it;
-//  UNMARKED: it ran on a caller's stream, which may since have been
-//            destroyed, and was not marked.
-enum class LastMark { NONE, PENDING, RECORDED, UNMARKED };
+// Per device: the word that counts the awaited tiles as they start, what it
+// will have counted when the launches enqueued so far have started all
+// theirs (modulo 2^32), and the stream of the last of them.
 struct WaitingState {
+    unsigned* word = nullptr;
+    unsigned target = 0;
     hipStream_t last = nullptr;  // the null stream is a stream too
-    hipEvent_t done = nullptr;
-    LastMark mark = LastMark::NONE;
-    bool eager = false;  // record after every launch on a caller's stream
+    bool pending = false;        // the last launch may not have started
 };
 // Kept for the process (never destroyed), like the library stream: boxes
 // may be destroyed during the process's exit.
@@ -466,6 +460,7 @@ Waiting& waiting() {
     return *w;
 }
 thread_local int t_waiting_depth = 0;
+thread_local unsigned* t_waiting_started = nullptr;  // of the outermost guard
 
 void owned_insert(hipStream_t s) {
     Waiting& g = waiting();
@@ -477,7 +472,7 @@ void owned_erase(hipStream_t s) {
     std::lock_guard<std::mutex> lk(g.mu);
     g.owned.erase(s);
     for (WaitingState& w : g.dev)
-        if (w.last == s && w.mark != LastMark::RECORDED) w.mark = LastMark::NONE;
+        if (w.last == s) w.pending = false;
 }
 
 bool capturing(hipStream_t s) {
@@ -487,10 +482,12 @@ bool capturing(hipStream_t s) {
 }
 }  // namespace
 
-WaitingLaunch::WaitingLaunch(hipStream_t s, bool waits) : s_(s) {
-    if (!waits) return;
+WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) {
+    if (awaited <= 0) return;
     // counted (and so undone by the destructor) only once nothing can throw
     if (t_waiting_depth > 0 || capturing(s)) {
+        started_ = t_waiting_depth > 0 ? t_waiting_started : nullptr;
+        if (t_waiting_depth == 0) t_waiting_started = nullptr;
         ++t_waiting_depth;
         counted_ = true;
         return;
@@ -500,22 +497,25 @@ WaitingLaunch::WaitingLaunch(hipStream_t s, bool waits) : s_(s) {
     std::unique_lock<std::mutex> lk(g.mu);
     if ((int)g.dev.size() <= dev_) g.dev.resize(dev_ + 1);
     WaitingState& w = g.dev[dev_];
-    if (w.last != s && w.mark != LastMark::NONE) {
-        if (!w.done) FF_HIP(hipEventCreateWithFlags(&w.done, hipEventDisableTiming));
-        if (w.mark == LastMark::PENDING && !capturing(w.last)) {
-            FF_HIP(hipEventRecord(w.done, w.last));
-            FF_HIP(hipStreamWaitEvent(s, w.done, 0));
-        } else if (w.mark == LastMark::RECORDED) {
-            FF_HIP(hipStreamWaitEvent(s, w.done, 0));
-        } else {
-            // unmarked (or its stream is being captured): wait for the
-            // device, and from now on mark launches on callers' streams as
-            // they end
-            FF_HIP(hipDeviceSynchronize());
-            w.eager = true;
-        }
+    if (!w.word) {
+        unsigned* p = nullptr;
+        FF_HIP(hipMalloc((void**)&p, sizeof(unsigned)));
+        const unsigned zero = 0;
+        FF_HIP(hipMemcpy(p, &zero, sizeof(zero), hipMemcpyHostToDevice));
+        w.word = p;
     }
+    // (a stream of the caller's may have been destroyed: it is not asked)
+    if (w.pending && w.last != s && !(g.owned.count(w.last) && !capturing(w.last) && hipStreamQuery(w.last) == hipSuccess)) {
+        launch_wait_started(w.word, w.target, s);
+        check_launch("WaitingLaunch");
+    }
+    awaited_ = awaited;
+    exceptions_ = std::uncaught_exceptions();
+    w.target += (unsigned)awaited;
+    w.last = s;
+    w.pending = true;
     lk.release();  // held until the destructor
+    started_ = t_waiting_started = w.word;
     ++t_waiting_depth;
     counted_ = true;
     locked_ = true;
@@ -526,18 +526,8 @@ WaitingLaunch::~WaitingLaunch() {
     --t_waiting_depth;
     if (!locked_) return;
     Waiting& g = waiting();
-    WaitingState& w = g.dev[dev_];
-    w.last = s_;
-    if (g.owned.count(s_)) {
-        w.mark = LastMark::PENDING;
-    } else if (w.eager && w.done && hipEventRecord(w.done, s_) == hipSuccess) {
-        w.mark = LastMark::RECORDED;
-    } else if (w.eager && !w.done && hipEventCreateWithFlags(&w.done, hipEventDisableTiming) == hipSuccess &&
-               hipEventRecord(w.done, s_) == hipSuccess) {
-        w.mark = LastMark::RECORDED;
-    } else {
-        w.mark = LastMark::UNMARKED;
-    }
+    // a launch that failed counts nothing
+    if (std::uncaught_exceptions() > exceptions_) g.dev[dev_].target -= (unsigned)awaited_;
     g.mu.unlock();
 }
 

@@ -2,6 +2,7 @@
 // method (src/gpu/<file>.cu).
 #include "ff_stages.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <sstream>
 
@@ -24,19 +25,17 @@ void require_alloc(const Image& a, const char* who) {
 
 }  // namespace
 
+int upper_index(int x, int n, int nu) {
+    if (n <= 1 || nu <= 0) return 0;
+    const float u = (float)x / (float)(n - 1);
+    const float s = u * (float)nu;
+    const int i = (int)std::floor(s);
+    return std::max(0, std::min(i, nu - 1));
+}
+
 std::vector<int> upper_index_map(int n, int nu) {
     std::vector<int> m((size_t)(n > 0 ? n : 0), 0);
-    for (int x = 0; x < n; ++x) {
-        int i = 0;
-        if (n > 1 && nu > 0) {
-            const float u = (float)x / (float)(n - 1);
-            const float s = u * (float)nu;
-            i = (int)std::floor(s);
-            if (i > nu - 1) i = nu - 1;
-            if (i < 0) i = 0;
-        }
-        m[x] = i;
-    }
+    for (int x = 0; x < n; ++x) m[x] = upper_index(x, n, nu);
     return m;
 }
 

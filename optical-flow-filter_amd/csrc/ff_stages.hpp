@@ -328,9 +328,7 @@ Camera createPerspectiveCamera(float focalLength, int height, int width, float s
 // library.
 ff_image_t colorWheelRGBA();
 
-// Upper-level texel index of every output column (or row) for the
-// normalized-coordinate point sampling of deltaFlowUpdate_k
-// (update_k.cu:151-155): i = min(floor(fl(x/(n-1)) * nu), nu-1).
+// upper_index of every column (or row) x < n.
 std::vector<int> upper_index_map(int n, int nu);
 
 }  // namespace ffamd
