@@ -190,6 +190,65 @@ __device__ __forceinline__ float shl(float v) {
     else return zshl(v);
 }
 
+// Lane shifts folded into the instruction that uses the shifted value, where
+// the compiler does not fold them (a lane shift into a select; a lane shift
+// into a product with a constant). Every lane must be active. An instruction
+// that reads a register of other lanes must come two instructions after the
+// one that wrote it: the leading s_nop covers the writer before the block,
+// the order inside each block its own. (Both forms took the 2048x1088
+// two-level launch from 52.2 to 49.0 us and a 64-stream batch from 975 to
+// 930; the image model's x taps written so too gained nothing and spilled.)
+
+#define FF_PICK(k) "v_cndmask_b32_dpp %" #k ", %" #k ", %" #k ", vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define FF_PICK_HEAD(k) "v_cmp_le_f32 vcc, 0, %" #k "\n\ts_nop 1\n\t"
+// Where the speed is not >= 0 (negative or NaN), each value becomes that of
+// lane i + 1 (0 without such a lane). With the backward differences z[i] -
+// z[i-1] of an upwind pass this selects between them and the forward
+// differences.
+__device__ __forceinline__ void pick(float speed, float& a, float& b) {
+    asm(FF_PICK_HEAD(2) FF_PICK(0) FF_PICK(1) : "+v"(a), "+v"(b) : "v"(speed) : "vcc");
+}
+__device__ __forceinline__ void pick(float speed, float& a, float& b, float& c, float& d) {
+    asm(FF_PICK_HEAD(4) FF_PICK(0) FF_PICK(1) FF_PICK(2) FF_PICK(3)
+        : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+        : "v"(speed)
+        : "vcc");
+}
+__device__ __forceinline__ void pick(float speed, float& a, float& b, float& c, float& d, float& e) {
+    asm(FF_PICK_HEAD(5) FF_PICK(0) FF_PICK(1) FF_PICK(2) FF_PICK(3) FF_PICK(4)
+        : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e)
+        : "v"(speed)
+        : "vcc");
+}
+#undef FF_PICK
+#undef FF_PICK_HEAD
+
+#define FF_DPP_SHR " wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define FF_DPP_SHL " wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+// Two 5-tap sums along x, of u and of v, with weights wo, wi, wc, wi, wo:
+// taps_x<false>'s products and order, with the outer neighbours shifted
+// inside their multiply-adds (7 instructions instead of 9).
+__device__ __forceinline__ void taps_x2(float& u, float& v, float wo, float wi, float wc) {
+    float mu, pu, mv, pv, a, b;
+    asm("s_nop 1\n\t"
+        "v_mov_b32_dpp %2, %0" FF_DPP_SHR "v_mov_b32_dpp %4, %1" FF_DPP_SHR
+        "v_mov_b32_dpp %3, %0" FF_DPP_SHL "v_mov_b32_dpp %5, %1" FF_DPP_SHL
+        "v_mul_f32_dpp %6, %2, %8" FF_DPP_SHR "v_mul_f32_dpp %7, %4, %8" FF_DPP_SHR
+        "v_fmac_f32 %6, %9, %2\n\t"
+        "v_fmac_f32 %7, %9, %4\n\t"
+        "v_fmac_f32 %6, %10, %0\n\t"
+        "v_fmac_f32 %7, %10, %1\n\t"
+        "v_fmac_f32 %6, %9, %3\n\t"
+        "v_fmac_f32 %7, %9, %5\n\t"
+        "v_fmac_f32_dpp %6, %3, %8" FF_DPP_SHL "v_fmac_f32_dpp %7, %5, %8" FF_DPP_SHL
+        : "+v"(u), "+v"(v), "=&v"(mu), "=&v"(pu), "=&v"(mv), "=&v"(pv), "=&v"(a), "=&v"(b)
+        : "v"(wo), "s"(wi), "s"(wc));
+    u = a;
+    v = b;
+}
+#undef FF_DPP_SHR
+#undef FF_DPP_SHL
+
 // 5-tap correlation along x in the order of the reference loops (c = -2..2):
 // acc = 0; acc = fma(w[c], v(x+c), acc).
 template <bool CLAMP, class Wf>
@@ -376,15 +435,24 @@ __device__ __forceinline__ void prop_x(State<DELTA, R>& s, const Geo& g, const L
         const float mu = zshr(zu), pu = zshl(zu);
         const float Ud = (fabsf(pu) - fabsf(mu)) > 0.0f ? pu : mu;
         const float nd = -(p.dt * Ud);
-        const bool back = Ud >= 0.0f;
-        float ou = kSkipU ? zu : upwind(mu, zu, pu, back, nd);
-        float ov = upwind(zshr(zv), zv, zshl(zv), back, nd);
-        float os = 0.f, odu = 0.f, odv = 0.f;
+        // the upwind difference of each field: its backward difference here,
+        // or, where the flow comes from the right, the one of the next lane
+        // (26 instructions per pixel with both differences and a select, 21
+        // so)
+        float ou = zu, ov = zv, os = 0.f, odu = 0.f, odv = 0.f;
+        float bu = zu - mu, bv = zv - zshr(zv);
         if constexpr (DELTA) {
-            os = upwind(zshr(s.sa[r]), s.sa[r], zshl(s.sa[r]), back, nd);
-            odu = upwind(zshr(s.du[r]), s.du[r], zshl(s.du[r]), back, nd);
-            odv = upwind(zshr(s.dv[r]), s.dv[r], zshl(s.dv[r]), back, nd);
+            float bs = s.sa[r] - zshr(s.sa[r]), bdu = s.du[r] - zshr(s.du[r]), bdv = s.dv[r] - zshr(s.dv[r]);
+            if constexpr (kSkipU) pick(Ud, bv, bs, bdu, bdv);
+            else pick(Ud, bu, bv, bs, bdu, bdv);
+            os = fmaf(nd, bs, s.sa[r]);
+            odu = fmaf(nd, bdu, s.du[r]);
+            odv = fmaf(nd, bdv, s.dv[r]);
+        } else {
+            pick(Ud, bu, bv);
         }
+        if constexpr (!kSkipU) ou = fmaf(nd, bu, zu);
+        ov = fmaf(nd, bv, zv);
         if constexpr (BORDER) {
             const int y = g.yw + r;
             const bool in = g.xin && y >= p.border && y < p.H - p.border;
@@ -539,8 +607,12 @@ template <bool CLAMP, int R>
 __device__ __forceinline__ void smooth_x(float (&fu)[R], float (&fv)[R]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        fu[r] = taps_x<CLAMP>(fu[r], WBox{});
-        fv[r] = taps_x<CLAMP>(fv[r], WBox{});
+        if constexpr (CLAMP) {
+            fu[r] = taps_x<CLAMP>(fu[r], WBox{});
+            fv[r] = taps_x<CLAMP>(fv[r], WBox{});
+        } else {
+            taps_x2(fu[r], fv[r], kBox, kBox, kBox);
+        }
     }
 }
 
