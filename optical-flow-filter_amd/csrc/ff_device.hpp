@@ -70,6 +70,20 @@ __device__ __forceinline__ void solve2x2(float gx, float gy, float Yt, float fx,
     oy = fmaf(N01, qx, N11 * qy) * rdet;
 }
 
+// One Lax-Wendroff update of a scalar along AXIS from its neighbours m, z, p
+// with Courant number R (LaxWendroffX_k / LaxWendroffY_k,
+// propagation_k.h:49-132).
+template <int AXIS>
+__device__ __forceinline__ float lw_scalar(float m, float z, float p, float R) {
+    const float d0 = p - m;
+    double d2;
+    if constexpr (AXIS == 0) d2 = (double)((m - 2.0f * z) + p);  // float second difference
+    else d2 = ((double)m - 2.0 * (double)z) + (double)p;         // double second difference
+    const double h = 0.5 * (double)R;
+    const double t = fma(-h, (double)d0, (double)z);
+    return (float)fma(h * (double)R, d2, t);
+}
+
 __device__ __forceinline__ bool not_finite(float v) { return !__builtin_isfinite(v); }
 
 // u8 pyramid tap, imageDown{X,Y}_uint8_k (pyramid_k.cu:38-43, 72-77):

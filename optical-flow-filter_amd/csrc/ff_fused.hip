@@ -66,13 +66,14 @@
 #include "ff_device.hpp"
 #include "ff_kernels.hpp"
 #include "ff_runtime.hpp"
+#include "ff_tile.hpp"
 
 namespace ffamd {
 
 namespace {
 
-constexpr int LANES = 64;
-constexpr int OOB = (int)0x80000000;  // buffer offset beyond any image: access dropped
+using namespace tile;
+
 constexpr int kSpinLimit = 1 << 23;   // polls before a wait gives up: about 2 s at s_sleep 8
 
 // One level of one frame, as the kernel reads it. Blocks first_block ..
@@ -108,178 +109,10 @@ struct LevelJob {
     float dt, gamma, maxflow;
 };
 
-__device__ __forceinline__ int lane_id() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
-__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
 
 // A job in the constant address space: its fields are read with scalar loads
 // wherever they are used.
 #define FF_CONSTANT __attribute__((address_space(4)))
-
-// ------------------------------------------------------------ buffer access
-
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ Rsrc rsrc(const void* p, int bytes) {
-    // word 3 of the buffer descriptor for gfx9-family raw (untyped) buffers
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
-}
-__device__ __forceinline__ float ld1(Rsrc r, int off) {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-}
-__device__ __forceinline__ float2 ld2(Rsrc r, int off) {
-    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-    return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
-}
-__device__ __forceinline__ unsigned ldb(Rsrc r, int off) { return __builtin_amdgcn_raw_buffer_load_b8(r, off, 0, 0); }
-__device__ __forceinline__ unsigned ldh(Rsrc r, int off) { return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0); }
-// Cache policy sc1: stores write through this XCD's L2 and such loads do
-// not hit a stale line in its caches (device-coherent, as for agent-scope
-// atomics).
-constexpr int kCoherent = 16;
-// Every store writes through. A frame's state is written once and read by
-// the next launch only, so dirty lines kept in L2 save nothing, and they
-// cost time: 55.8 us per 2048x1088 two-level frame with write-back stores,
-// 52.8 us with write-through ones (streaming stores and loads, policy nt,
-// were slower than either). The write-through also publishes the top
-// level's unsmoothed flow to the tiles of the level below, which read it
-// within the same launch with ld2_coherent.
-__device__ __forceinline__ void st1(Rsrc r, int off, float v) {
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, kCoherent);
-}
-__device__ __forceinline__ void st2(Rsrc r, int off, float a, float b) {
-    const u32x2 v = {__float_as_uint(a), __float_as_uint(b)};
-    __builtin_amdgcn_raw_buffer_store_b64(v, r, off, 0, kCoherent);
-}
-__device__ __forceinline__ float2 ld2_coherent(Rsrc r, int off) {
-    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kCoherent);
-    return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
-}
-
-// ---------------------------------------------------------- lane shifts
-// Lane i receives lane i-1 (shr) or lane i+1 (shl). The zero-filling forms
-// give 0 to the lane without a source; the clamping forms let it keep its
-// own value (the clamp-to-edge read at an image edge).
-__device__ __forceinline__ float zshr(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float zshl(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float cshr(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x138, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float cshl(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x130, 0xf, 0xf, false));
-}
-// Lane i receives lane i-1's v; lane 0 receives `own`. (A select between a
-// shifted value and a lane's own value must not be written as a condition:
-// the compiler may then run the shift with some lanes disabled, and a lane
-// reading a disabled lane receives 0.)
-__device__ __forceinline__ unsigned shr_or(unsigned v, unsigned own) {
-    return (unsigned)__builtin_amdgcn_update_dpp((int)own, (int)v, 0x138, 0xf, 0xf, false);
-}
-template <bool CLAMP>
-__device__ __forceinline__ float shr(float v) {
-    if constexpr (CLAMP) return cshr(v);
-    else return zshr(v);
-}
-template <bool CLAMP>
-__device__ __forceinline__ float shl(float v) {
-    if constexpr (CLAMP) return cshl(v);
-    else return zshl(v);
-}
-
-// Lane shifts folded into the instruction that uses the shifted value, where
-// the compiler does not fold them (a lane shift into a select; a lane shift
-// into a product with a constant). Every lane must be active. An instruction
-// that reads a register of other lanes must come two instructions after the
-// one that wrote it: the leading s_nop covers the writer before the block,
-// the order inside each block its own. (Both forms took the 2048x1088
-// two-level launch from 52.2 to 49.0 us and a 64-stream batch from 975 to
-// 930; the image model's x taps written so too gained nothing and spilled.)
-
-#define FF_PICK(k) "v_cndmask_b32_dpp %" #k ", %" #k ", %" #k ", vcc wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-#define FF_PICK_HEAD(k) "v_cmp_le_f32 vcc, 0, %" #k "\n\ts_nop 1\n\t"
-// Where the speed is not >= 0 (negative or NaN), each value becomes that of
-// lane i + 1 (0 without such a lane). With the backward differences z[i] -
-// z[i-1] of an upwind pass this selects between them and the forward
-// differences.
-__device__ __forceinline__ void pick(float speed, float& a, float& b) {
-    asm(FF_PICK_HEAD(2) FF_PICK(0) FF_PICK(1) : "+v"(a), "+v"(b) : "v"(speed) : "vcc");
-}
-__device__ __forceinline__ void pick(float speed, float& a, float& b, float& c, float& d) {
-    asm(FF_PICK_HEAD(4) FF_PICK(0) FF_PICK(1) FF_PICK(2) FF_PICK(3)
-        : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
-        : "v"(speed)
-        : "vcc");
-}
-__device__ __forceinline__ void pick(float speed, float& a, float& b, float& c, float& d, float& e) {
-    asm(FF_PICK_HEAD(5) FF_PICK(0) FF_PICK(1) FF_PICK(2) FF_PICK(3) FF_PICK(4)
-        : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e)
-        : "v"(speed)
-        : "vcc");
-}
-#undef FF_PICK
-#undef FF_PICK_HEAD
-
-#define FF_DPP_SHR " wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-#define FF_DPP_SHL " wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-// Two 5-tap sums along x, of u and of v, with weights wo, wi, wc, wi, wo:
-// taps_x<false>'s products and order, with the outer neighbours shifted
-// inside their multiply-adds (7 instructions instead of 9).
-__device__ __forceinline__ void taps_x2(float& u, float& v, float wo, float wi, float wc) {
-    float mu, pu, mv, pv, a, b;
-    asm("s_nop 1\n\t"
-        "v_mov_b32_dpp %2, %0" FF_DPP_SHR "v_mov_b32_dpp %4, %1" FF_DPP_SHR
-        "v_mov_b32_dpp %3, %0" FF_DPP_SHL "v_mov_b32_dpp %5, %1" FF_DPP_SHL
-        "v_mul_f32_dpp %6, %2, %8" FF_DPP_SHR "v_mul_f32_dpp %7, %4, %8" FF_DPP_SHR
-        "v_fmac_f32 %6, %9, %2\n\t"
-        "v_fmac_f32 %7, %9, %4\n\t"
-        "v_fmac_f32 %6, %10, %0\n\t"
-        "v_fmac_f32 %7, %10, %1\n\t"
-        "v_fmac_f32 %6, %9, %3\n\t"
-        "v_fmac_f32 %7, %9, %5\n\t"
-        "v_fmac_f32_dpp %6, %3, %8" FF_DPP_SHL "v_fmac_f32_dpp %7, %5, %8" FF_DPP_SHL
-        : "+v"(u), "+v"(v), "=&v"(mu), "=&v"(pu), "=&v"(mv), "=&v"(pv), "=&v"(a), "=&v"(b)
-        : "v"(wo), "s"(wi), "s"(wc));
-    u = a;
-    v = b;
-}
-#undef FF_DPP_SHR
-#undef FF_DPP_SHL
-
-// 5-tap correlation along x in the order of the reference loops (c = -2..2):
-// acc = 0; acc = fma(w[c], v(x+c), acc).
-template <bool CLAMP, class Wf>
-__device__ __forceinline__ float taps_x(float v, Wf w) {
-    const float m1 = shr<CLAMP>(v), p1 = shl<CLAMP>(v);
-    float a = 0.0f;
-    a = fmaf(w(0), shr<CLAMP>(m1), a);
-    a = fmaf(w(1), m1, a);
-    a = fmaf(w(2), v, a);
-    a = fmaf(w(3), p1, a);
-    a = fmaf(w(4), shl<CLAMP>(p1), a);
-    return a;
-}
-
-struct WSmooth {
-    __device__ __forceinline__ float operator()(int i) const { return smooth_w(i); }
-};
-struct WDiff {
-    __device__ __forceinline__ float operator()(int i) const { return diff_w(i); }
-};
-struct WBox {
-    __device__ __forceinline__ float operator()(int) const { return kBox; }
-};
-
-// Map a job's tile index so that the tiles of one XCD (blocks are dealt
-// round-robin over the 8 XCDs) form a contiguous band of the image.
-__device__ __forceinline__ int xcd_tile(int b, int nt) {
-    const int q = nt / 8;
-    if (b >= 8 * q) return b;
-    return (b % 8) * q + b / 8;
-}
 
 // --------------------------------------------------- tiles waited for
 
@@ -338,15 +171,6 @@ __device__ __forceinline__ void flag_store(unsigned* f, unsigned v) {
 __device__ __forceinline__ void flag_add(unsigned* f) {
     __hip_atomic_fetch_add(f, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-// Per-thread view of the tile.
-struct Geo {
-    int lane, wave, x, yw;
-    int xl;        // column read: x, or the last column for x beyond the image
-    int xlast;     // lane of the image's last column (>= LANES - 1: not in the buffer)
-    bool xin;      // column strictly inside the propagation border
-    bool wave_in;  // every pixel of the wave strictly inside the border
-};
 
 // The tiles of the upper level that tile t waits for: first, first + 1, ..,
 // nx of them across, n in all.
@@ -414,127 +238,6 @@ __device__ __forceinline__ void signal_done(const LevelJob& p, int t, const Geo&
 
 // ------------------------------------------------------------ tile body
 
-// Registers of the level state: flow (fu, fv) and, on delta levels, the
-// scalar (old brightness) and vector (delta flow) payloads.
-template <bool DELTA, int R>
-struct State {
-    float fu[R], fv[R];
-    float sa[DELTA ? R : 1], du[DELTA ? R : 1], dv[DELTA ? R : 1];
-};
-
-// One upwind X pass (flowPropagateX_k / flowPropagatePayloadX_k,
-// propagation_k.cu:16-72, 134-232). LAST: the final iteration of a delta
-// level, whose propagated flow is read only as the Y pass's speed (the
-// delta update consumes the payloads): the u component is not advanced.
-template <bool DELTA, bool BORDER, int R, bool LAST = false>
-__device__ __forceinline__ void prop_x(State<DELTA, R>& s, const Geo& g, const LevelJob& p) {
-    constexpr bool kSkipU = DELTA && LAST;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float zu = s.fu[r], zv = s.fv[r];
-        const float mu = zshr(zu), pu = zshl(zu);
-        const float Ud = (fabsf(pu) - fabsf(mu)) > 0.0f ? pu : mu;
-        const float nd = -(p.dt * Ud);
-        // the upwind difference of each field: its backward difference here,
-        // or, where the flow comes from the right, the one of the next lane
-        // (26 instructions per pixel with both differences and a select, 21
-        // so)
-        float ou = zu, ov = zv, os = 0.f, odu = 0.f, odv = 0.f;
-        float bu = zu - mu, bv = zv - zshr(zv);
-        if constexpr (DELTA) {
-            float bs = s.sa[r] - zshr(s.sa[r]), bdu = s.du[r] - zshr(s.du[r]), bdv = s.dv[r] - zshr(s.dv[r]);
-            if constexpr (kSkipU) pick(Ud, bv, bs, bdu, bdv);
-            else pick(Ud, bu, bv, bs, bdu, bdv);
-            os = fmaf(nd, bs, s.sa[r]);
-            odu = fmaf(nd, bdu, s.du[r]);
-            odv = fmaf(nd, bdv, s.dv[r]);
-        } else {
-            pick(Ud, bu, bv);
-        }
-        if constexpr (!kSkipU) ou = fmaf(nd, bu, zu);
-        ov = fmaf(nd, bv, zv);
-        if constexpr (BORDER) {
-            const int y = g.yw + r;
-            const bool in = g.xin && y >= p.border && y < p.H - p.border;
-            if constexpr (!kSkipU) ou = in ? ou : zu;
-            ov = in ? ov : zv;
-            if constexpr (DELTA) {
-                os = in ? os : s.sa[r];
-                odu = in ? odu : s.du[r];
-                odv = in ? odv : s.dv[r];
-            }
-        }
-        s.fu[r] = ou;
-        s.fv[r] = ov;
-        if constexpr (DELTA) {
-            s.sa[r] = os;
-            s.du[r] = odu;
-            s.dv[r] = odv;
-        }
-    }
-}
-
-// Rows above (a) and below (b) a wave's strip for one Y pass.
-struct Edge5 {
-    float u, v, s, du, dv;
-};
-
-// One upwind Y pass (flowPropagateY_k / flowPropagatePayloadY_k,
-// propagation_k.cu:75-131, 235-334); rows top-down, m* keep the old values
-// of row r-1. LAST: the final pass of a delta level, whose propagated flow
-// is dead (only the payloads feed the delta update): the flow is not
-// advanced, only read for the speed Vd.
-template <bool DELTA, bool BORDER, int R, bool LAST = false>
-__device__ __forceinline__ void prop_y(State<DELTA, R>& s, const Geo& g, const LevelJob& p, const Edge5& a,
-                                       const Edge5& b) {
-    constexpr bool kSkipF = DELTA && LAST;
-    float mu = a.u, mv = a.v, ms = a.s, mdu = a.du, mdv = a.dv;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float zu = s.fu[r], zv = s.fv[r];
-        const float pu = r + 1 < R ? s.fu[r + 1] : b.u;
-        const float pv = r + 1 < R ? s.fv[r + 1] : b.v;
-        const float Vd = (fabsf(pv) - fabsf(mv)) > 0.0f ? pv : mv;
-        const float nd = -(p.dt * Vd);
-        const bool back = Vd >= 0.0f;
-        float ou = kSkipF ? zu : upwind(mu, zu, pu, back, nd);
-        float ov = kSkipF ? zv : upwind(mv, zv, pv, back, nd);
-        mu = zu;
-        mv = zv;
-        bool in = true;
-        if constexpr (BORDER) {
-            const int y = g.yw + r;
-            in = g.xin && y >= p.border && y < p.H - p.border;
-            if constexpr (!kSkipF) {
-                ou = in ? ou : zu;
-                ov = in ? ov : zv;
-            }
-        }
-        s.fu[r] = ou;
-        s.fv[r] = ov;
-        if constexpr (DELTA) {
-            const float zs = s.sa[r], zdu = s.du[r], zdv = s.dv[r];
-            const float ps = r + 1 < R ? s.sa[r + 1] : b.s;
-            const float pdu = r + 1 < R ? s.du[r + 1] : b.du;
-            const float pdv = r + 1 < R ? s.dv[r + 1] : b.dv;
-            float os = upwind(ms, zs, ps, back, nd);
-            float odu = upwind(mdu, zdu, pdu, back, nd);
-            float odv = upwind(mdv, zdv, pdv, back, nd);
-            ms = zs;
-            mdu = zdu;
-            mdv = zdv;
-            if constexpr (BORDER) {
-                os = in ? os : zs;
-                odu = in ? odu : zdu;
-                odv = in ? odv : zdv;
-            }
-            s.sa[r] = os;
-            s.du[r] = odu;
-            s.dv[r] = odv;
-        }
-    }
-}
-
 // Image model (imagePrefilter_k / imageModel_k, imagemodel_k.cu:31-133) and
 // update (flowUpdate_k, update_k.cu:15-79, or deltaFlowUpdate_k, :82-173)
 // of every row of the thread. im[j] is image row yw-2+j (clamped reads),
@@ -587,72 +290,6 @@ __device__ __forceinline__ void model_update(State<DELTA, R>& s, const float (&i
         }
         s.fu[r] = ox;
         s.fv[r] = oy;
-    }
-}
-
-// Lanes beyond the image's last column (lane xlast) take its values.
-template <int R>
-__device__ __forceinline__ void copy_last_column(float (&fu)[R], float (&fv)[R], int lane, int xlast) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float eu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fu[r]), xlast));
-        const float ev = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fv[r]), xlast));
-        fu[r] = lane > xlast ? eu : fu[r];
-        fv[r] = lane > xlast ? ev : fv[r];
-    }
-}
-
-// X pass of the box smoother (flowSmoothX_k, flowsmoothing_k.cu:21-53).
-template <bool CLAMP, int R>
-__device__ __forceinline__ void smooth_x(float (&fu)[R], float (&fv)[R]) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if constexpr (CLAMP) {
-            fu[r] = taps_x<CLAMP>(fu[r], WBox{});
-            fv[r] = taps_x<CLAMP>(fv[r], WBox{});
-        } else {
-            taps_x2(fu[r], fv[r], kBox, kBox, kBox);
-        }
-    }
-}
-
-// Y pass of the box smoother (flowSmoothY_k, flowsmoothing_k.cu:55-87) over
-// the thread's rows; a2/a1 are the rows above, b1/b2 the rows below. With
-// YCLAMP, rows after rlast (outside the image) are replaced by row rlast, the
-// clamped read; rows after rlast themselves are not needed.
-template <bool YCLAMP, int R>
-__device__ __forceinline__ void smooth_y(float (&fu)[R], float (&fv)[R], float a2u, float a2v, float a1u, float a1v,
-                                         float b1u, float b1v, float b2u, float b2v, int rlast) {
-    float m2u = a2u, m2v = a2v, m1u = a1u, m1v = a1v;  // old rows r-2, r-1
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float zu = fu[r], zv = fv[r];
-        float p1u = r + 1 < R ? fu[r + 1] : b1u, p1v = r + 1 < R ? fv[r + 1] : b1v;
-        float p2u = r + 2 < R ? fu[r + 2] : (r + 2 == R ? b1u : b2u);
-        float p2v = r + 2 < R ? fv[r + 2] : (r + 2 == R ? b1v : b2v);
-        if constexpr (YCLAMP) {
-            p2u = r + 2 <= rlast ? p2u : (r + 1 <= rlast ? p1u : zu);
-            p2v = r + 2 <= rlast ? p2v : (r + 1 <= rlast ? p1v : zv);
-            p1u = r + 1 <= rlast ? p1u : zu;
-            p1v = r + 1 <= rlast ? p1v : zv;
-        }
-        float su = 0.0f, sv = 0.0f;
-        su = fmaf(kBox, m2u, su);
-        sv = fmaf(kBox, m2v, sv);
-        su = fmaf(kBox, m1u, su);
-        sv = fmaf(kBox, m1v, sv);
-        su = fmaf(kBox, zu, su);
-        sv = fmaf(kBox, zv, sv);
-        su = fmaf(kBox, p1u, su);
-        sv = fmaf(kBox, p1v, sv);
-        su = fmaf(kBox, p2u, su);
-        sv = fmaf(kBox, p2v, sv);
-        m2u = m1u;
-        m2v = m1v;
-        m1u = zu;
-        m1v = zv;
-        fu[r] = su;
-        fv[r] = sv;
     }
 }
 
@@ -800,13 +437,6 @@ __device__ __forceinline__ void finish_image(const ImageRegs<MODE, R>& ir, float
     }
 }
 
-// Row exchange buffer of the workgroup: [2][nw][10][LANES] floats (double
-// buffered; 10 rows of each wave: its first and last rows of up to five
-// fields).
-__device__ __forceinline__ float* xrow(float* xch, int nw, int slot, int wave) {
-    return xch + ((slot * nw + wave) * 10) * LANES;
-}
-
 // INNER: a tile whose every pixel lies inside the border, away from the
 // image edges (every wave inside, no edge lanes, no clamped rows, no
 // column or row beyond the image): one straight-line body with no per-wave
@@ -901,53 +531,11 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
         constexpr bool LAST = decltype(last)::value;
         if (INNER || g.wave_in) prop_x<DELTA, false, R, LAST>(s, g, p);
         else prop_x<DELTA, true, R, LAST>(s, g, p);
-        {
-            float* my = xrow(xch, nw, slot, wave);
-            my[0 * LANES + lane] = s.fu[0];
-            my[1 * LANES + lane] = s.fv[0];
-            my[5 * LANES + lane] = s.fu[R - 1];
-            my[6 * LANES + lane] = s.fv[R - 1];
-            if constexpr (DELTA) {
-                my[2 * LANES + lane] = s.sa[0];
-                my[3 * LANES + lane] = s.du[0];
-                my[4 * LANES + lane] = s.dv[0];
-                my[7 * LANES + lane] = s.sa[R - 1];
-                my[8 * LANES + lane] = s.du[R - 1];
-                my[9 * LANES + lane] = s.dv[R - 1];
-            }
-        }
+        put_rows<DELTA, R>(s, xch, nw, slot, wave, lane);
         __syncthreads();
-        // missing neighbour rows (first/last wave): the own edge row, the
-        // clamp-to-edge read at an image edge
-        Edge5 ea{s.fu[0], s.fv[0], 0.f, 0.f, 0.f}, eb{s.fu[R - 1], s.fv[R - 1], 0.f, 0.f, 0.f};
-        if constexpr (DELTA) {
-            ea.s = s.sa[0];
-            ea.du = s.du[0];
-            ea.dv = s.dv[0];
-            eb.s = s.sa[R - 1];
-            eb.du = s.du[R - 1];
-            eb.dv = s.dv[R - 1];
-        }
-        if (wave > 0) {
-            const float* o = xrow(xch, nw, slot, wave - 1);
-            ea.u = o[5 * LANES + lane];
-            ea.v = o[6 * LANES + lane];
-            if constexpr (DELTA) {
-                ea.s = o[7 * LANES + lane];
-                ea.du = o[8 * LANES + lane];
-                ea.dv = o[9 * LANES + lane];
-            }
-        }
-        if (wave < nw - 1) {
-            const float* o = xrow(xch, nw, slot, wave + 1);
-            eb.u = o[0 * LANES + lane];
-            eb.v = o[1 * LANES + lane];
-            if constexpr (DELTA) {
-                eb.s = o[2 * LANES + lane];
-                eb.du = o[3 * LANES + lane];
-                eb.dv = o[4 * LANES + lane];
-            }
-        }
+        Edge5 ea = own_row<DELTA, R>(s, 0), eb = own_row<DELTA, R>(s, R - 1);
+        if (wave > 0) get_row<DELTA>(ea, xrow(xch, nw, slot, wave - 1) + 5 * LANES, lane);
+        if (wave < nw - 1) get_row<DELTA>(eb, xrow(xch, nw, slot, wave + 1), lane);
         slot ^= 1;
         if (INNER || g.wave_in) prop_y<DELTA, false, R, LAST>(s, g, p, ea, eb);
         else prop_y<DELTA, true, R, LAST>(s, g, p, ea, eb);
@@ -996,38 +584,10 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
         if (!INNER && xinside) copy_last_column<R>(s.fu, s.fv, g.lane, xlast);
         if (!INNER && xedge) smooth_x<true, R>(s.fu, s.fv);
         else smooth_x<false, R>(s.fu, s.fv);
-        {
-            float* my = xrow(xch, nw, slot, wave);
-            my[0 * LANES + lane] = s.fu[0];
-            my[1 * LANES + lane] = s.fv[0];
-            my[2 * LANES + lane] = s.fu[1];
-            my[3 * LANES + lane] = s.fv[1];
-            my[4 * LANES + lane] = s.fu[R - 2];
-            my[5 * LANES + lane] = s.fv[R - 2];
-            my[6 * LANES + lane] = s.fu[R - 1];
-            my[7 * LANES + lane] = s.fv[R - 1];
-        }
-        __syncthreads();
-        // rows -2, -1 (above) and R, R+1 (below)
-        float a2u = s.fu[0], a2v = s.fv[0], a1u = s.fu[0], a1v = s.fv[0];
-        float b1u = s.fu[R - 1], b1v = s.fv[R - 1], b2u = s.fu[R - 1], b2v = s.fv[R - 1];
-        if (wave > 0) {
-            const float* o = xrow(xch, nw, slot, wave - 1);
-            a2u = o[4 * LANES + lane];
-            a2v = o[5 * LANES + lane];
-            a1u = o[6 * LANES + lane];
-            a1v = o[7 * LANES + lane];
-        }
-        if (wave < nw - 1) {
-            const float* o = xrow(xch, nw, slot, wave + 1);
-            b1u = o[0 * LANES + lane];
-            b1v = o[1 * LANES + lane];
-            b2u = o[2 * LANES + lane];
-            b2v = o[3 * LANES + lane];
-        }
+        const Edge2 e = exchange_smooth_rows<R>(s.fu, s.fv, xch, nw, slot, wave, lane);
         slot ^= 1;
-        if (!INNER && yinside) smooth_y<true, R>(s.fu, s.fv, a2u, a2v, a1u, a1v, b1u, b1v, b2u, b2v, rlast);
-        else smooth_y<false, R>(s.fu, s.fv, a2u, a2v, a1u, a1v, b1u, b1v, b2u, b2v, rlast);
+        if (!INNER && yinside) smooth_y<true, R>(s.fu, s.fv, e, rlast);
+        else smooth_y<false, R>(s.fu, s.fv, e, rlast);
     }
 
     {

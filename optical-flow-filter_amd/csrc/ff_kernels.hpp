@@ -57,6 +57,38 @@ void launch_delta_update(const DevImg& a0, const DevImg& grad, const DevImg& a0o
 // One box-smoothing pass (axis 0 = x, 1 = y) on float2 images.
 void launch_smooth_pass(int axis, const DevImg& in, const DevImg& out, hipStream_t s);
 
+// Propagated fields: flow (float2) and optional payloads (scalar, float2
+// vector), with row pitches in bytes; null without payloads.
+struct PropFields {
+    float2* f = nullptr;
+    float* s = nullptr;
+    float2* v = nullptr;
+    int fp = 0, sp = 0, vp = 0;
+};
+// Iterations of one launch of the kernels below. More than four propagation
+// iterations (halo 4: 77 % of a 64 x 64 buffer is output) cost more in halo
+// than a further launch's pass over memory; a smoothing iteration's halo is 2.
+constexpr int kMaxPropIters = 4, kMaxSmoothIters = 4;
+// n <= kMaxPropIters iterations on B images one after the other in memory,
+// in one launch (ff_tiles.hip); `mid` (if its f is set) receives the fields
+// after `after` iterations. The outputs must not be the inputs.
+bool propagate_tile_supported(const PropFields& in, const PropFields& out, int H, int W, int border);
+void launch_propagate_tile(const PropFields& in, const PropFields& mid, int after, const PropFields& out, int n, int B,
+                           int H, int W, float dt, int border, hipStream_t s);
+bool smooth_tile_supported(int in_pitch, int out_pitch, int H, int W);
+void launch_smooth_tile(const void* in, int in_pitch, void* out, int out_pitch, int n, int B, int H, int W,
+                        hipStream_t s);
+// n iterations from `in` into y (propagation, smoothing) or x (Lax-Wendroff,
+// scalar images), the other buffer in between. Return false, having done
+// nothing, where the tile kernels do not apply: the caller then runs the
+// single passes. (A border of 0, where the pixels at an image edge move too;
+// an image of 2 GiB and more; an input that is one of the buffers.)
+bool launch_propagate(const PropFields& in, const PropFields& x, const PropFields& y, int n, int H, int W, float dt,
+                      int border, hipStream_t s);
+bool launch_smooth(const DevImg& in, const DevImg& x, const DevImg& y, int n, hipStream_t s);
+bool launch_lax_wendroff(const DevImg& flow, const DevImg& in, const DevImg& x, const DevImg& y, int n, float dt,
+                         hipStream_t s);
+
 // One pyramid half-resolution pass (axis 0 = x, 1 = y), u8 or float.
 void launch_down_pass(int axis, bool u8, const DevImg& in, const DevImg& out, hipStream_t s);
 

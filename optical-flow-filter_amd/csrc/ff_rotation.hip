@@ -55,17 +55,6 @@ __global__ void __launch_bounds__(BX* BY) k_rotational_flow(Camera cam, float wx
     *(float2*)((char*)flow.data + (size_t)y * flow.pitch + (size_t)x * 8) = make_float2(u, v);
 }
 
-template <int AXIS>
-__device__ __forceinline__ float lw_scalar(float m, float z, float p, float R) {
-    const float d0 = p - m;
-    double d2;
-    if constexpr (AXIS == 0) d2 = (double)((m - 2.0f * z) + p);  // float second difference
-    else d2 = ((double)m - 2.0 * (double)z) + (double)p;         // double second difference
-    const double h = 0.5 * (double)R;
-    const double t = fma(-h, (double)d0, (double)z);
-    return (float)fma(h * (double)R, d2, t);
-}
-
 __device__ __forceinline__ float lw_float(float m, float z, float p, float h, float k) {
     const float d0 = p - m;
     const float d2 = (m - 2.0f * z) + p;

@@ -18,6 +18,19 @@ void require_shape(const Image& a, const Image& b, const char* who) {
                           " vs " + b.shapeString());
 }
 
+PropFields prop_fields(const DevImg& f, const DevImg* s = nullptr, const DevImg* v = nullptr) {
+    PropFields p;
+    p.f = (float2*)f.data;
+    p.fp = (int)f.pitch;
+    if (s) {
+        p.s = (float*)s->data;
+        p.sp = (int)s->pitch;
+        p.v = (float2*)v->data;
+        p.vp = (int)v->pitch;
+    }
+    return p;
+}
+
 void require_alloc(const Image& a, const char* who) {
     if (!a.allocated() && (size_t)a.height() * a.rowBytes() > 0)
         throw logic_error(std::string(who) + ": unallocated buffer");
@@ -132,6 +145,10 @@ void FlowPropagator::run() {
         launch_scale_f2(src, -1.0f, by, s);
         src = by;
     }
+    if (launch_propagate(prop_fields(src), prop_fields(bx), prop_fields(by), iterations_, src.h, src.w, dt_, border_, s)) {
+        check_launch("FlowPropagator::compute");
+        return;
+    }
     launch_propagate_pass(0, src, bx, nullptr, nullptr, nullptr, nullptr, dt_, border_, s);
     launch_propagate_pass(1, bx, by, nullptr, nullptr, nullptr, nullptr, dt_, border_, s);
     for (int n = 0; n < iterations_ - 1; ++n) {
@@ -237,6 +254,11 @@ void FlowPropagatorPayload::run() {
     DevImg fx = flowX_.view(), fy = flowY_.view(), sx = scalarX_.view(), sy = scalarY_.view(),
            vx = vectorX_.view(), vy = vectorY_.view();
     DevImg f0 = bFlow_.view(), s0 = bScalar_.view(), v0 = bVector_.view();
+    if (launch_propagate(prop_fields(f0, &s0, &v0), prop_fields(fx, &sx, &vx), prop_fields(fy, &sy, &vy), iterations_,
+                         f0.h, f0.w, dt_, border_, s)) {
+        check_launch("FlowPropagatorPayload::compute");
+        return;
+    }
     launch_propagate_pass(0, f0, fx, &s0, &sx, &v0, &vx, dt_, border_, s);
     launch_propagate_pass(1, fx, fy, &sx, &sy, &vx, &vy, dt_, border_, s);
     for (int n = 0; n < iterations_ - 1; ++n) {
@@ -493,6 +515,10 @@ void FlowSmoother::run() {
     CrossStream x{&bound_, &bufX_, &bufY_};
     hipStream_t s = stream();
     const DevImg bx = bufX_.view(), by = bufY_.view();
+    if (launch_smooth(bound_.view(), bx, by, iterations_ > 1 ? iterations_ : 1, s)) {
+        check_launch("FlowSmoother::compute");
+        return;
+    }
     launch_smooth_pass(0, bound_.view(), bx, s);
     launch_smooth_pass(1, bx, by, s);
     for (int n = 0; n < iterations_ - 1; ++n) {
@@ -673,6 +699,11 @@ void LaxWendroffPropagator::run() {
     CrossStream x{&flow_, &image_, &bufX_, &bufY_};
     hipStream_t s = stream();
     const int c = image_.depth();
+    if (c == 1 && launch_lax_wendroff(flow_.view(), image_.view(), bufX_.view(), bufY_.view(),
+                                      iterations_ > 1 ? iterations_ : 1, dt_, s)) {
+        check_launch("LaxWendroffPropagator::compute");
+        return;
+    }
     launch_lax_wendroff_pass(1, c, flow_.view(), image_.view(), bufY_.view(), dt_, s);
     launch_lax_wendroff_pass(0, c, flow_.view(), bufY_.view(), bufX_.view(), dt_, s);
     for (int k = 0; k < iterations_ - 1; ++k) {
