@@ -521,6 +521,15 @@ FF_API ff_status ff_ad_propagate_pair(const float* flow, const float* scalar, co
 FF_API ff_status ff_ad_propagate_quad(const float* flow, const float* scalar, const float* vector, float* flow_out,
                                       float* scalar_out, float* vector_out, int B, int H, int W, float dt, int border,
                                       void* stream);
+/* 1 to 4 iterations in one launch (the same results as that many
+ * ff_ad_propagate_pair calls). With flow_mid (and scalar_mid, vector_mid
+ * when there are payloads) the fields after `after` of them (1 to iterations
+ * - 1) are written too. No output may be an input; a flow image must be
+ * smaller than 2 GiB. */
+FF_API ff_status ff_ad_propagate_steps(const float* flow, const float* scalar, const float* vector, int iterations,
+                                       int after, float* flow_mid, float* scalar_mid, float* vector_mid,
+                                       float* flow_out, float* scalar_out, float* vector_out, int B, int H, int W,
+                                       float dt, int border, void* stream);
 /* Adjoint of ff_ad_propagate_quad given the quad's input only (its three
  * inner passes are recomputed inside the launch); bitwise the adjoints of
  * the two pairs. g_*_out may be NULL (zero); accumulate as for the pass
@@ -605,6 +614,10 @@ FF_API ff_status ff_ad_smooth_pass_backward(int axis, const float* g_flow_out, c
  * output gradient g_flow_out + g_flow_out2 (g_flow_out2 may be NULL); g_flow
  * must be neither of them. */
 FF_API ff_status ff_ad_smooth_pair(const float* flow, float* flow_out, int B, int H, int W, void* stream);
+/* 1 to 4 smoothing iterations in one launch (the same results as that many
+ * ff_ad_smooth_pair calls); a flow image must be smaller than 2 GiB. */
+FF_API ff_status ff_ad_smooth_steps(const float* flow, float* flow_out, int iterations, int B, int H, int W,
+                                    void* stream);
 FF_API ff_status ff_ad_smooth_pair_backward(const float* g_flow_out, const float* g_flow_out2, float* g_flow, int B,
                                             int H, int W, int accumulate, void* stream);
 /* Photometric term of the differentiable window's loss, fused (no

@@ -1438,6 +1438,24 @@ void prop(int axis, const float* fin, const float* sin, const float* vin, float*
         else hipLaunchKernelGGL((k_ad_prop<1, false>), g, blk, 0, s, F(fin), sin, F(vin), (float2*)fout, sout, (float2*)vout, d, dt, border);
     }
 }
+namespace {
+PropFields fields(const float* f, const float* s, const float* v, int W) {
+    PropFields p;
+    p.f = (float2*)f;
+    p.s = (float*)s;
+    p.v = (float2*)v;
+    p.fp = p.vp = W * 8;
+    p.sp = W * 4;
+    return p;
+}
+}  // namespace
+bool steps_supported(int H, int W) { return (long long)H * W * 8 < 0x7fffffffLL; }
+void prop_steps(const float* fin, const float* sin, const float* vin, int n, int after, float* fmid, float* smid,
+                float* vmid, float* fout, float* sout, float* vout, int B, int H, int W, float dt, int border,
+                hipStream_t s) {
+    launch_propagate_tile(fields(fin, sin, vin, W), fields(fmid, smid, vmid, W), after, fields(fout, sout, vout, W), n,
+                          B, H, W, dt, border, s);
+}
 void prop_pair(const float* fin, const float* sin, const float* vin, float* fmid, float* smid, float* vmid,
                float* fout, float* sout, float* vout, int B, int H, int W, float dt, int border, hipStream_t s) {
     const bool pay = sin != nullptr, save = fmid != nullptr;
@@ -1572,6 +1590,9 @@ void upper_gather(const float* gup, const int* xlo, const int* xhi, const int* y
 void smooth(int axis, const float* in, float* out, int B, int H, int W, hipStream_t s) {
     if (axis == 0) hipLaunchKernelGGL((k_ad_smooth<0>), grid3(B, H, W), dim3(BX, BY), 0, s, (const float2*)in, (float2*)out, Dims{H, W});
     else hipLaunchKernelGGL((k_ad_smooth<1>), grid3(B, H, W), dim3(BX, BY), 0, s, (const float2*)in, (float2*)out, Dims{H, W});
+}
+void smooth_steps(const float* in, float* out, int n, int B, int H, int W, hipStream_t s) {
+    launch_smooth_tile(in, W * 8, out, W * 8, n, B, H, W, s);
 }
 void smooth_pair(const float* in, float* out, int B, int H, int W, hipStream_t s) {
     const dim3 g((W + 63) / 64, (H + kSmoothRows - 1) / kSmoothRows, B), blk(64, kSmoothRows + 4);

@@ -939,6 +939,34 @@ ff_status ff_ad_propagate_quad(const float* flow, const float* scalar, const flo
         check_launch("ff_ad_propagate_quad");
     });
 }
+ff_status ff_ad_propagate_steps(const float* flow, const float* scalar, const float* vector, int iterations, int after,
+                                float* flow_mid, float* scalar_mid, float* vector_mid, float* flow_out,
+                                float* scalar_out, float* vector_out, int B, int H, int W, float dt, int border,
+                                void* stream) {
+    return guard([&] {
+        dims(B, H, W);
+        if (border < 1) throw invalid_argument("border must be at least 1");
+        if (iterations < 1 || iterations > kMaxPropIters)
+            throw invalid_argument("iterations must be 1 to " + std::to_string(kMaxPropIters));
+        need(flow, "flow"), need(flow_out, "flow_out");
+        const bool pay = scalar != nullptr, save = flow_mid != nullptr;
+        if (pay != (vector != nullptr) || pay != (scalar_out != nullptr) || pay != (vector_out != nullptr))
+            throw invalid_argument("payloads: pass all of scalar, vector and their outputs, or none");
+        if (save && (pay != (scalar_mid != nullptr) || pay != (vector_mid != nullptr)))
+            throw invalid_argument("intermediates: pass those of the payloads with the flow's, or none");
+        if (save && (after < 1 || after >= iterations))
+            throw invalid_argument("the intermediates are those after 1 to iterations - 1 iterations");
+        if (!ad::steps_supported(H, W)) throw invalid_argument("the flow image must be smaller than 2 GiB");
+        for (const float* in : {flow, vector})
+            for (const float* out : {flow_out, vector_out, flow_mid, vector_mid})
+                if (in && in == out) throw invalid_argument("outputs must not be the inputs (the passes read neighbours)");
+        if (pay && (scalar_out == scalar || scalar_mid == scalar))
+            throw invalid_argument("outputs must not be the inputs (the passes read neighbours)");
+        ad::prop_steps(flow, scalar, vector, iterations, after, flow_mid, scalar_mid, vector_mid, flow_out, scalar_out,
+                       vector_out, B, H, W, dt, border, as_stream(stream));
+        check_launch("ff_ad_propagate_steps");
+    });
+}
 ff_status ff_ad_propagate_quad_backward(const float* flow, const float* scalar, const float* vector,
                                         const float* g_flow_out, const float* g_scalar_out, const float* g_vector_out,
                                         float* g_flow, float* g_scalar, float* g_vector, int B, int H, int W, float dt,
@@ -1114,6 +1142,18 @@ ff_status ff_ad_smooth_pair(const float* flow, float* flow_out, int B, int H, in
         if (flow == flow_out) throw invalid_argument("flow_out must not be flow (the passes read neighbours)");
         ad::smooth_pair(flow, flow_out, B, H, W, as_stream(stream));
         check_launch("ff_ad_smooth_pair");
+    });
+}
+ff_status ff_ad_smooth_steps(const float* flow, float* flow_out, int iterations, int B, int H, int W, void* stream) {
+    return guard([&] {
+        dims(B, H, W);
+        if (iterations < 1 || iterations > kMaxSmoothIters)
+            throw invalid_argument("iterations must be 1 to " + std::to_string(kMaxSmoothIters));
+        need(flow, "flow"), need(flow_out, "flow_out");
+        if (flow == flow_out) throw invalid_argument("flow_out must not be flow (the passes read neighbours)");
+        if (!ad::steps_supported(H, W)) throw invalid_argument("the flow image must be smaller than 2 GiB");
+        ad::smooth_steps(flow, flow_out, iterations, B, H, W, as_stream(stream));
+        check_launch("ff_ad_smooth_steps");
     });
 }
 ff_status ff_ad_smooth_pair_backward(const float* g_flow_out, const float* g_flow_out2, float* g_flow, int B, int H,

@@ -310,6 +310,12 @@ void prop(int axis, const float* fin, const float* sin, const float* vin, float*
           int H, int W, float dt, int border, hipStream_t s);
 void prop_pair(const float* fin, const float* sin, const float* vin, float* fmid, float* smid, float* vmid,
                float* fout, float* sout, float* vout, int B, int H, int W, float dt, int border, hipStream_t s);
+// n <= kMaxPropIters iterations in one launch; the fields after `after`
+// iterations too where fmid is not null. Images below 2 GiB.
+void prop_steps(const float* fin, const float* sin, const float* vin, int n, int after, float* fmid, float* smid,
+                float* vmid, float* fout, float* sout, float* vout, int B, int H, int W, float dt, int border,
+                hipStream_t s);
+bool steps_supported(int H, int W);
 void prop_quad(const float* fin, const float* sin, const float* vin, float* fout, float* sout, float* vout, int B, int H,
                int W, float dt, int border, hipStream_t s);
 void prop_quad_bwd(const float* fin, const float* sin, const float* vin, const float* gfo, const float* gso,
@@ -343,6 +349,8 @@ void upper_gather(const float* gup, const int* xlo, const int* xhi, const int* y
                   int B, int H, int W, int Hu, int Wu, int acc, hipStream_t s);
 void smooth(int axis, const float* in, float* out, int B, int H, int W, hipStream_t s);
 void smooth_pair(const float* in, float* out, int B, int H, int W, hipStream_t s);
+// n <= kMaxSmoothIters iterations in one launch. Images below 2 GiB.
+void smooth_steps(const float* in, float* out, int n, int B, int H, int W, hipStream_t s);
 void smooth_pair_bwd(const float* gout, const float* gout2, float* gin, int B, int H, int W, int acc,
                      hipStream_t s);
 void smooth_bwd(int axis, const float* gout, const float* gout2, float* gin, int B, int H, int W, int acc,

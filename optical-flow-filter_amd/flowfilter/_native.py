@@ -249,6 +249,7 @@ SIGNATURES = {
     "ff_ad_propagate_pass": [_i, _v, _v, _v, _v, _v, _v, _i, _i, _i, _f, _i, _v],
     "ff_ad_propagate_pair": [_v, _v, _v, _v, _v, _v, _v, _v, _v, _i, _i, _i, _f, _i, _v],
     "ff_ad_propagate_quad": [_v, _v, _v, _v, _v, _v, _i, _i, _i, _f, _i, _v],
+    "ff_ad_propagate_steps": [_v, _v, _v, _i, _i, _v, _v, _v, _v, _v, _v, _i, _i, _i, _f, _i, _v],
     "ff_ad_propagate_quad_backward": [_v, _v, _v, _v, _v, _v, _v, _v, _v, _i, _i, _i, _f, _i, _i, _v],
     "ff_ad_propagate_pair_backward": [_v, _v, _v, _v, _v, _v, _v, _v, _v, _v, _v, _v, _i, _i, _i, _f, _i, _i, _v],
     "ff_ad_propagate_pass_backward": [_i, _v, _v, _v, _v, _v, _v, _v, _v, _v, _i, _i, _i, _f, _i, _i, _v],
@@ -262,6 +263,7 @@ SIGNATURES = {
     "ff_ad_smooth_pass": [_i, _v, _v, _i, _i, _i, _v],
     "ff_ad_smooth_pass_backward": [_i, _v, _v, _v, _i, _i, _i, _i, _v],
     "ff_ad_smooth_pair": [_v, _v, _i, _i, _i, _v],
+    "ff_ad_smooth_steps": [_v, _v, _i, _i, _i, _i, _v],
     "ff_ad_smooth_pair_backward": [_v, _v, _v, _i, _i, _i, _i, _v],
     "ff_ad_photometric_partial_count": [_i, _i, _i, _i, _pi],
     "ff_ad_photometric": [_v, _v, _v, _i, _i, _i, _i, _v],

@@ -112,6 +112,15 @@ class FilterSpec(object):
                 lv[k] = torch.from_numpy(v).to(self.device)
 
 
+# Iterations that one launch of the tile kernels takes, and whether they
+# take an image of this size (32-bit offsets).
+_STEPS = 4
+
+
+def _tiled(h, w):
+    return h * w * 8 < 2 ** 31 - 1
+
+
 def _p(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
@@ -181,22 +190,30 @@ def _frame_forward(spec, state, image, gammas, save):
         pay = sc is not None
         it = 0
         while it < lv["N"]:
-            fo = _empty(B, h, w, 2, like=image)
-            so = _empty(B, h, w, like=image) if pay else None
-            vo = _empty(B, h, w, 2, like=image) if pay else None
-            # two iterations per launch, then one if N is odd; only their
-            # input is kept: the adjoints recompute the passes inside
-            n = 2 if it + 2 <= lv["N"] else 1
-            if n == 2:
-                N.call("ff_ad_propagate_quad", _p(f), _p(sc), _p(vc), _p(fo), _p(so), _p(vo), B, h, w,
+            fields = lambda: (_empty(B, h, w, 2, like=image), _empty(B, h, w, like=image) if pay else None,
+                              _empty(B, h, w, 2, like=image) if pay else None)
+            # up to four iterations per launch; what is kept is the input of
+            # every two (and of a last single one): the adjoints recompute
+            # the passes inside
+            n = min(_STEPS if _tiled(h, w) else 2, lv["N"] - it)
+            kept = [(min(2, n), f, sc, vc)]
+            out = fields()
+            if _tiled(h, w):
+                mid = fields() if save and n > 2 else (None, None, None)
+                N.call("ff_ad_propagate_steps", _p(f), _p(sc), _p(vc), n, 2, _p(mid[0]), _p(mid[1]), _p(mid[2]),
+                       _p(out[0]), _p(out[1]), _p(out[2]), B, h, w, ctypes.c_float(lv["dt"]), spec.border, s)
+                if n > 2:
+                    kept.append((n - 2,) + mid)
+            elif n == 2:
+                N.call("ff_ad_propagate_quad", _p(f), _p(sc), _p(vc), _p(out[0]), _p(out[1]), _p(out[2]), B, h, w,
                        ctypes.c_float(lv["dt"]), spec.border, s)
             else:
-                N.call("ff_ad_propagate_pair", _p(f), _p(sc), _p(vc), None, None, None, _p(fo), _p(so), _p(vo),
-                       B, h, w, ctypes.c_float(lv["dt"]), spec.border, s)
+                N.call("ff_ad_propagate_pair", _p(f), _p(sc), _p(vc), None, None, None, _p(out[0]), _p(out[1]),
+                       _p(out[2]), B, h, w, ctypes.c_float(lv["dt"]), spec.border, s)
             if save:
-                passes.append((n, f, sc, vc))
+                passes.extend(kept)
             it += n
-            f, sc, vc = fo, so, vo
+            f, sc, vc = out
         prop[l] = (f, sc, vc)
         if save:
             saved["passes"][l] = passes
@@ -233,10 +250,14 @@ def _frame_forward(spec, state, image, gammas, save):
 
 
 def _smooth(f, K, B, h, w, s):
-    for _ in range(K):  # an X and a Y pass per launch
+    while K > 0:  # up to four iterations (an X and a Y pass each) per launch
+        n = min(_STEPS if _tiled(h, w) else 1, K)
         o = torch.empty_like(f)
-        N.call("ff_ad_smooth_pair", _p(f), _p(o), B, h, w, s)
-        f = o
+        if _tiled(h, w):
+            N.call("ff_ad_smooth_steps", _p(f), _p(o), n, B, h, w, s)
+        else:
+            N.call("ff_ad_smooth_pair", _p(f), _p(o), B, h, w, s)
+        f, K = o, K - n
     return f
 
 

@@ -79,3 +79,45 @@ def test_own_output_as_input(ffo, n):
     m.configure()
     m.compute()  # the buffers are new ones: the input is the old output
     assert _same(m.getSmoothedFlow().download(np.float32), ffo.smooth(want, n))
+
+
+@pytest.mark.parametrize("B,h,w", [(1, 33, 65), (3, 57, 113), (2, 130, 200)])
+@pytest.mark.parametrize("n,after", [(1, 0), (2, 1), (3, 2), (4, 2)])
+@pytest.mark.parametrize("pay", [False, True])
+def test_ad_steps_match_single_passes(B, h, w, n, after, pay):
+    """ff_ad_propagate_steps (with the fields in between) and
+    ff_ad_smooth_steps on a batch are bitwise the single passes."""
+    import ctypes
+
+    import torch
+    from flowfilter import _native as N
+    print("ad steps", (B, h, w), n, after, pay, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(h * n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda") * 0.7
+    new = lambda: [torch.empty(B, h, w, 2, device="cuda")] + ([torch.empty(B, h, w, device="cuda"),
+                                                             torch.empty(B, h, w, 2, device="cuda")] if pay else [])
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    arg = lambda fs: [p(t) for t in fs] + [None] * (3 - len(fs))
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    dt = ctypes.c_float(1.0 / n)
+    fields = [rnd(B, h, w, 2)] + ([rnd(B, h, w), rnd(B, h, w, 2)] if pay else [])
+    ref, kept = fields, None
+    for k in range(n):
+        for axis in (0, 1):
+            out = new()
+            N.call("ff_ad_propagate_pass", axis, *arg(ref), *arg(out), B, h, w, dt, 3, s)
+            ref = out
+        if k + 1 == after:
+            kept = ref
+    mid, out = (new() if after else []), new()
+    N.call("ff_ad_propagate_steps", *arg(fields), n, after, *arg(mid), *arg(out), B, h, w, dt, 3, s)
+    assert all(torch.equal(a, b) for a, b in zip(ref, out))
+    if after:
+        assert all(torch.equal(a, b) for a, b in zip(kept, mid))
+    sm, got = fields[0], torch.empty_like(fields[0])
+    for _ in range(n):
+        o = torch.empty_like(sm)
+        N.call("ff_ad_smooth_pair", p(sm), p(o), B, h, w, s)
+        sm = o
+    N.call("ff_ad_smooth_steps", p(fields[0]), p(got), n, B, h, w, s)
+    assert torch.equal(sm, got)
