@@ -618,6 +618,11 @@ FF_API ff_status ff_ad_smooth_pair(const float* flow, float* flow_out, int B, in
  * ff_ad_smooth_pair calls); a flow image must be smaller than 2 GiB. */
 FF_API ff_status ff_ad_smooth_steps(const float* flow, float* flow_out, int iterations, int B, int H, int W,
                                     void* stream);
+/* Adjoint of ff_ad_smooth_steps for the output gradient g_flow_out +
+ * g_flow_out2 (g_flow_out2 may be NULL); the same results as that many
+ * ff_ad_smooth_pair_backward calls. g_flow must be neither of them. */
+FF_API ff_status ff_ad_smooth_steps_backward(const float* g_flow_out, const float* g_flow_out2, float* g_flow,
+                                             int iterations, int B, int H, int W, int accumulate, void* stream);
 FF_API ff_status ff_ad_smooth_pair_backward(const float* g_flow_out, const float* g_flow_out2, float* g_flow, int B,
                                             int H, int W, int accumulate, void* stream);
 /* Photometric term of the differentiable window's loss, fused (no

@@ -112,26 +112,9 @@ __global__ void __launch_bounds__(BX* BY) k_ad_image_model(const float* I, float
     g[at(b, y, x, d)] = make_float2(dx, dy);
 }
 
-// a0 = Sx(sy), gx = Dx(sy), gy = Dy(sx) with sy = Sy(I), sx = Sx(I): the
-// adjoint first forms g_sy = Sx^T g_a0 + Dx^T g_gx and g_sx = Dy^T g_gy.
-__global__ void __launch_bounds__(BX* BY)
-    k_ad_image_model_bwd1(const float* ga0, const float2* gg, float* gsy, float* gsx, Dims d) {
-    const int x = blockIdx.x * BX + threadIdx.x, y = blockIdx.y * BY + wave_y(), b = blockIdx.z;
-    if (x >= d.W || y >= d.H) return;
-    const float s1 = corr5_adjoint(x, d.W, WS{}, [&](int i) { return ga0[at(b, y, i, d)]; });
-    const float s2 = corr5_adjoint(x, d.W, WD{}, [&](int i) { return gg[at(b, y, i, d)].x; });
-    gsy[at(b, y, x, d)] = s1 + s2;
-    gsx[at(b, y, x, d)] = corr5_adjoint(y, d.H, WD{}, [&](int i) { return gg[at(b, i, x, d)].y; });
-}
-
-// g_I = Sy^T g_sy + Sx^T g_sx.
-__global__ void __launch_bounds__(BX* BY)
-    k_ad_image_model_bwd2(const float* gsy, const float* gsx, float* gI, Dims d, int acc) {
-    const int x = blockIdx.x * BX + threadIdx.x, y = blockIdx.y * BY + wave_y(), b = blockIdx.z;
-    if (x >= d.W || y >= d.H) return;
-    const float a = corr5_adjoint(y, d.H, WS{}, [&](int i) { return gsy[at(b, i, x, d)]; });
-    const float c = corr5_adjoint(x, d.W, WS{}, [&](int i) { return gsx[at(b, y, i, d)]; });
-    put(gI, at(b, y, x, d), a + c, acc);
+__global__ void __launch_bounds__(256) k_ad_put(const float* v, float* out, size_t n, int acc) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) put(out, i, v[i], acc);
 }
 
 // ----------------------------------------------------------- float pyramid
@@ -1407,11 +1390,18 @@ void image_model(const float* I, float* a0, float* g, int B, int H, int W, hipSt
 }
 void image_model_bwd(const float* ga0, const float* gg, float* gI, float* work, int B, int H, int W, int acc,
                      hipStream_t s) {
-    const size_t n = (size_t)B * H * W;
-    hipLaunchKernelGGL(k_ad_image_model_bwd1, grid3(B, H, W), dim3(BX, BY), 0, s, ga0, (const float2*)gg, work,
-                       work + n, Dims{H, W});
-    hipLaunchKernelGGL(k_ad_image_model_bwd2, grid3(B, H, W), dim3(BX, BY), 0, s, work, work + n, gI, Dims{H, W},
-                       acc);
+    // a result that replaces an input goes through the work buffer, since the
+    // adjoint reads neighbours
+    const bool inplace = gI == ga0 || gI == gg;
+    launch_image_model_adjoint(ga0, gg, inplace ? work : gI, B, H, W, inplace ? 0 : acc, s);
+    if (inplace) {
+        const size_t n = (size_t)B * H * W;
+        hipLaunchKernelGGL(k_ad_put, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, work, gI, n, acc);
+    }
+}
+void smooth_steps_bwd(const float* gout, const float* gout2, float* gin, int n, int B, int H, int W, int acc,
+                      hipStream_t s) {
+    launch_smooth_adjoint(gout, gout2, gin, n, B, H, W, acc, s);
 }
 void down(const float* I, float* O, float* work, int B, int H, int W, hipStream_t s) {
     const Dims d0{H, W}, d1{H, W / 2}, d2{H / 2, W / 2};

@@ -1156,6 +1156,20 @@ ff_status ff_ad_smooth_steps(const float* flow, float* flow_out, int iterations,
         check_launch("ff_ad_smooth_steps");
     });
 }
+ff_status ff_ad_smooth_steps_backward(const float* g_flow_out, const float* g_flow_out2, float* g_flow, int iterations,
+                                      int B, int H, int W, int accumulate, void* stream) {
+    return guard([&] {
+        dims(B, H, W);
+        if (iterations < 1 || iterations > kMaxSmoothIters)
+            throw invalid_argument("iterations must be 1 to " + std::to_string(kMaxSmoothIters));
+        need(g_flow_out, "g_flow_out"), need(g_flow, "g_flow");
+        if (g_flow == g_flow_out || g_flow == g_flow_out2)
+            throw invalid_argument("g_flow must not be an output gradient (the adjoint reads neighbours)");
+        ad::smooth_steps_bwd(g_flow_out, g_flow_out2, g_flow, iterations, B, H, W, accumulate != 0 ? 1 : 0,
+                             as_stream(stream));
+        check_launch("ff_ad_smooth_steps_backward");
+    });
+}
 ff_status ff_ad_smooth_pair_backward(const float* g_flow_out, const float* g_flow_out2, float* g_flow, int B, int H,
                                      int W, int accumulate, void* stream) {
     return guard([&] {

@@ -78,6 +78,13 @@ void launch_propagate_tile(const PropFields& in, const PropFields& mid, int afte
 bool smooth_tile_supported(int in_pitch, int out_pitch, int H, int W);
 void launch_smooth_tile(const void* in, int in_pitch, void* out, int out_pitch, int n, int B, int H, int W,
                         hipStream_t s);
+// Adjoints (ff_tiles.hip) of the image model, and of n <= kMaxSmoothIters
+// smoothing iterations for the output gradient gout + gout2 (may be null), on
+// B images of any size; with acc the result is added.
+void launch_image_model_adjoint(const float* ga0, const float* gg, float* gI, int B, int H, int W, int acc,
+                                hipStream_t s);
+void launch_smooth_adjoint(const float* gout, const float* gout2, float* gin, int n, int B, int H, int W, int acc,
+                           hipStream_t s);
 // n iterations from `in` into y (propagation, smoothing) or x (Lax-Wendroff,
 // scalar images), the other buffer in between. Return false, having done
 // nothing, where the tile kernels do not apply: the caller then runs the
@@ -304,6 +311,9 @@ namespace ad {
 void image_model(const float* I, float* a0, float* g, int B, int H, int W, hipStream_t s);
 void image_model_bwd(const float* ga0, const float* gg, float* gI, float* work, int B, int H, int W, int acc,
                      hipStream_t s);
+// Adjoint of smooth_steps (gout2 may be null).
+void smooth_steps_bwd(const float* gout, const float* gout2, float* gin, int n, int B, int H, int W, int acc,
+                      hipStream_t s);
 void down(const float* I, float* O, float* work, int B, int H, int W, hipStream_t s);
 void down_bwd(const float* gO, float* gI, float* work, int B, int H, int W, int acc, hipStream_t s);
 void prop(int axis, const float* fin, const float* sin, const float* vin, float* fout, float* sout, float* vout, int B,

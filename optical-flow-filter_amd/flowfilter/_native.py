@@ -264,6 +264,7 @@ SIGNATURES = {
     "ff_ad_smooth_pass_backward": [_i, _v, _v, _v, _i, _i, _i, _i, _v],
     "ff_ad_smooth_pair": [_v, _v, _i, _i, _i, _v],
     "ff_ad_smooth_steps": [_v, _v, _i, _i, _i, _i, _v],
+    "ff_ad_smooth_steps_backward": [_v, _v, _v, _i, _i, _i, _i, _i, _v],
     "ff_ad_smooth_pair_backward": [_v, _v, _v, _i, _i, _i, _i, _v],
     "ff_ad_photometric_partial_count": [_i, _i, _i, _i, _pi],
     "ff_ad_photometric": [_v, _v, _v, _i, _i, _i, _i, _v],

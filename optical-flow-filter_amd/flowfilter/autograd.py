@@ -275,10 +275,12 @@ def _smooth_bwd(parts, K, B, h, w, s, out=None):
         out.add_(total)
         return out
     g, g2 = parts[0], (parts[1] if len(parts) > 1 else None)
-    for i in range(K):  # the Y pass's and then the X pass's adjoint per launch
-        last = i == K - 1
-        o = out if (last and out is not None) else torch.empty_like(g)
-        N.call("ff_ad_smooth_pair_backward", _p(g), _p(g2), _p(o), B, h, w, 1 if (last and out is not None) else 0, s)
+    while K > 0:  # up to four iterations' adjoints per launch
+        n = min(_STEPS, K)
+        K -= n
+        last = K == 0 and out is not None
+        o = out if last else torch.empty_like(g)
+        N.call("ff_ad_smooth_steps_backward", _p(g), _p(g2), _p(o), n, B, h, w, 1 if last else 0, s)
         g, g2 = o, None
     return g
 

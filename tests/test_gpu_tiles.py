@@ -121,3 +121,49 @@ def test_ad_steps_match_single_passes(B, h, w, n, after, pay):
         sm = o
     N.call("ff_ad_smooth_steps", p(fields[0]), p(got), n, B, h, w, s)
     assert torch.equal(sm, got)
+
+
+@pytest.mark.parametrize("B,h,w", [(2, 1, 1), (1, 2, 4), (3, 5, 3), (1, 31, 63), (2, 33, 65), (1, 61, 60), (3, 130, 122)])
+@pytest.mark.parametrize("n", [1, 2, 3])
+@pytest.mark.parametrize("second,acc", [(False, 0), (True, 1)])
+def test_ad_tile_adjoints(B, h, w, n, second, acc):
+    """The smoothing iterations' adjoint is bitwise that many single
+    iterations'; the image model's adjoint is the transpose of the image model:
+    <g, M x> = <M^T g, x> in float64 sums of float32 results, to 1e-5 of the
+    terms' magnitude (a few float32 roundings each)."""
+    import ctypes
+
+    import torch
+    from flowfilter import _native as N
+    print("ad adjoints", (B, h, w), n, second, acc, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(h * 7 + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    a, b = rnd(B, h, w, 2), rnd(B, h, w, 2) if second else None
+    base = rnd(B, h, w, 2)
+    ref, two = a, b
+    for k in range(n):
+        last = k == n - 1
+        o = base.clone() if last and acc else torch.empty_like(a)
+        N.call("ff_ad_smooth_pair_backward", p(ref), p(two), p(o), B, h, w, acc if last else 0, s)
+        ref, two = o, None
+    got = base.clone() if acc else torch.empty_like(a)
+    N.call("ff_ad_smooth_steps_backward", p(a), p(b), p(got), n, B, h, w, acc, s)
+    assert torch.equal(ref, got)
+    img, ga, gg = rnd(B, h, w), rnd(B, h, w), rnd(B, h, w, 2)
+    a0, gr, work = torch.empty_like(img), torch.empty_like(gg), torch.empty(B, 2 * h, w, device="cuda")
+    N.call("ff_ad_image_model", p(img), p(a0), p(gr), B, h, w, s)
+    out = base[..., 0].contiguous() if acc else torch.empty_like(img)
+    start = out.double().clone() if acc else 0.0
+    N.call("ff_ad_image_model_backward", p(ga), p(gg), p(out), p(work), B, h, w, acc, s)
+    left = (ga.double() * a0.double()).sum() + (gg.double() * gr.double()).sum()
+    terms = (out.double() - start) * img.double()
+    scale = terms.abs().sum() + (ga.double() * a0.double()).abs().sum() + (gg.double() * gr.double()).abs().sum()
+    assert abs(float(left - terms.sum())) <= 1e-5 * float(scale)
+    # in place, through the work buffer
+    inplace = ga.clone()
+    N.call("ff_ad_image_model_backward", p(inplace), p(gg), p(inplace), p(work), B, h, w, 0, s)
+    plain = torch.empty_like(img)
+    N.call("ff_ad_image_model_backward", p(ga), p(gg), p(plain), p(work), B, h, w, 0, s)
+    assert torch.equal(inplace, plain)
