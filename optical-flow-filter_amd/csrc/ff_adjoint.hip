@@ -25,6 +25,7 @@
 #include "ff_device.hpp"
 #include "ff_kernels.hpp"
 #include "ff_runtime.hpp"
+#include "ff_tile.hpp"
 
 namespace ffamd {
 
@@ -74,12 +75,6 @@ __device__ __forceinline__ float corr5_adjoint(int j, int n, Wf w, Dy dy) {
     return acc;
 }
 
-struct WS {
-    __device__ __forceinline__ float operator()(int i) const { return smooth_w(i); }
-};
-struct WD {
-    __device__ __forceinline__ float operator()(int i) const { return diff_w(i); }
-};
 struct WB {
     __device__ __forceinline__ float operator()(int) const { return kBox; }
 };
@@ -281,17 +276,9 @@ __global__ void __launch_bounds__(64 * (kPairRows + 2))
     }
 }
 
-// What an output of a pass contributes to its three inputs (see out_terms).
-struct OutTerms {
-    float cm, cz, cp;  // coefficients of the inputs at o-1, o, o+1
-    float gud;         // adjoint of the speed
-    unsigned flags;    // bit 0: o inside the border; bit 1: speed taken from o+1
-};
-
 // Rows of pixels (Px5) in LDS as planes (flow, scalar, vector), 20 bytes
 // per pixel with consecutive lanes at consecutive addresses (an array of
-// Px5 takes 24 bytes, its padded size, and strides the banks). A row can
-// hold a pixel or an output's OutTerms instead.
+// Px5 takes 24 bytes, its padded size, and strides the banks).
 template <int S>
 struct LdsRows {
     float2 f[S][64];
@@ -312,21 +299,6 @@ struct LdsRows {
         r.s = PAY ? s[i][tx] : 0.f;
         r.v = PAY ? v[i][tx] : make_float2(0.f, 0.f);
         return r;
-    }
-    __device__ __forceinline__ void put_terms(int i, int tx, const OutTerms& t) {
-        f[i][tx] = make_float2(t.cm, t.cz);
-        s[i][tx] = t.cp;
-        v[i][tx] = make_float2(t.gud, __uint_as_float(t.flags));
-    }
-    __device__ __forceinline__ OutTerms get_terms(int i, int tx) const {
-        const float2 a = f[i][tx], c = v[i][tx];
-        OutTerms t;
-        t.cm = a.x;
-        t.cz = a.y;
-        t.cp = s[i][tx];
-        t.gud = c.x;
-        t.flags = __float_as_uint(c.y);
-        return t;
     }
 };
 
@@ -485,94 +457,6 @@ __device__ __forceinline__ Px5 upwind_adjoint_px(const Px5 (&X)[5], const Px5 (&
     return r;
 }
 
-// upwind_adjoint_px in two halves, for kernels that hold every output of a
-// pass: out_terms computes, once per output o, what o contributes to its
-// three inputs (the coefficients of the inputs at o-1, o, o+1 and the
-// adjoint of its speed, routed to the neighbour the speed came from), and
-// gather_px sums the terms of outputs j-1, j, j+1 for input j. Both use
-// upwind_adjoint_px's expressions in its order, so together they give its
-// results bit for bit, while each output's terms are computed once instead
-// of once per input that reads them (OutTerms above).
-template <int C, bool PAY>
-__device__ __forceinline__ OutTerms out_terms(const Px5& xm, const Px5& x0, const Px5& xp, const Px5& g, bool interior,
-                                              float dt) {
-    OutTerms t;
-    t.cm = t.cz = t.cp = t.gud = 0.f;
-    t.flags = 0u;
-    if (!interior) return t;
-    const float um = C == 0 ? xm.f.x : xm.f.y, up = C == 0 ? xp.f.x : xp.f.y;
-    const bool selp = (fabsf(up) - fabsf(um)) > 0.0f;
-    const float Ud = selp ? up : um;
-    const float nd = -(dt * Ud);
-    const bool back = Ud >= 0.0f;
-    t.cz = 1.0f + (back ? nd : -nd);
-    t.cm = back ? -nd : 0.f;
-    t.cp = back ? 0.f : nd;
-    auto D = [&](float m, float z, float p) { return back ? (z - m) : (p - z); };
-    float gUd = g.f.x * D(xm.f.x, x0.f.x, xp.f.x) + g.f.y * D(xm.f.y, x0.f.y, xp.f.y);
-    if constexpr (PAY)
-        gUd += g.s * D(xm.s, x0.s, xp.s) + g.v.x * D(xm.v.x, x0.v.x, xp.v.x) + g.v.y * D(xm.v.y, x0.v.y, xp.v.y);
-    gUd *= -dt;
-    t.gud = gUd;
-    t.flags = 1u | (selp ? 2u : 0u);
-    return t;
-}
-
-// Input j from outputs j-1, j, j+1 (T, G; valid: the output is inside the
-// line).
-template <int C, bool PAY>
-__device__ __forceinline__ Px5 gather_px(const OutTerms (&T)[3], const Px5 (&G)[3], const bool (&valid)[3]) {
-    float2 gf = make_float2(0.f, 0.f), gv = make_float2(0.f, 0.f);
-    float gs = 0.f;
-#pragma unroll
-    for (int oi = 0; oi < 3; ++oi) {
-        if (!valid[oi]) continue;
-        const Px5& g = G[oi];
-        if (!(T[oi].flags & 1u)) {
-            if (oi == 1) {  // out = z
-                gf.x += g.f.x;
-                gf.y += g.f.y;
-                if (PAY) {
-                    gs += g.s;
-                    gv.x += g.v.x;
-                    gv.y += g.v.y;
-                }
-            }
-            continue;
-        }
-        const float c = (oi == 1) ? T[oi].cz : ((oi == 2) ? T[oi].cm : T[oi].cp);
-        gf.x = fmaf(c, g.f.x, gf.x);
-        gf.y = fmaf(c, g.f.y, gf.y);
-        if constexpr (PAY) {
-            gs = fmaf(c, g.s, gs);
-            gv.x = fmaf(c, g.v.x, gv.x);
-            gv.y = fmaf(c, g.v.y, gv.y);
-        }
-        const bool selp = (T[oi].flags & 2u) != 0u;
-        const bool from = selp ? (oi == 0) : (oi == 2);
-        if (from) {
-            if (C == 0) gf.x += T[oi].gud;
-            else gf.y += T[oi].gud;
-        }
-    }
-    Px5 r;
-    r.f = gf;
-    r.s = gs;
-    r.v = gv;
-    return r;
-}
-
-template <bool PREV>
-__device__ __forceinline__ OutTerms lane_shift_terms(const OutTerms& t) {
-    OutTerms r;
-    r.cm = lane_shift<PREV>(t.cm);
-    r.cz = lane_shift<PREV>(t.cz);
-    r.cp = lane_shift<PREV>(t.cp);
-    r.gud = lane_shift<PREV>(t.gud);
-    r.flags = (unsigned)__builtin_amdgcn_update_dpp(0, (int)t.flags, PREV ? 0x138 : 0x130, 0xf, 0xf, true);
-    return r;
-}
-
 template <bool PAY>
 __device__ __forceinline__ Px5 load_grad_px(const float2* f, const float* s, const float2* v, size_t i) {
     Px5 r;
@@ -726,188 +610,330 @@ __global__ void __launch_bounds__(64 * kPairBwdRows)
 }
 
 
-// Adjoint of k_ad_prop_quad (two iterations), recomputing the forward
-// passes inside the launch. A workgroup of 64 x NW threads covers 64
-// columns, lane tx being column x0-3+tx, and S = NW x RPW staged rows, wave
-// w holding staged rows i = w + NW k, image rows y0-4+i (reads clamped into
-// the image); R = S - 8 output rows. Forward: the first X pass on the S rows
-// (row neighbours from the adjacent lanes, the edge lanes load theirs) into
-// LDS, the first Y pass on rows 1..S-2, the second X pass on those rows
-// (adjacent lanes; valid on lanes 1..62) into LDS. Adjoints, each as
-// per-output terms (out_terms) and a gather (gather_px), which give the
-// single passes' adjoints bit for bit:
-//   second Y pass: terms of rows 2..S-3 (lanes 1..62; the output gradients
-//     read from memory) into LDS in place of the second X pass, gathered at
-//     rows 3..S-4;
-//   second X pass: terms at every lane (its inputs and neighbours from the
-//     adjacent lanes), gathered from the adjacent lanes at lanes 2..61;
-//     the result, the first Y pass's output gradient, into LDS;
-//   first Y pass: terms of rows 3..S-4 into LDS in place of the first X
-//     pass, gathered at rows 4..S-5;
-//   first X pass: as the second, written for lanes 3..60 (columns
-//     x0 .. x0+57, rows y0 .. y0+R-1).
-constexpr int kQuadBwdCols = 58;
-// Workgroup shape of the launches: 16 waves of 2 rows, 32 staged rows for
-// 24 output rows, two 40 KB sets of LDS planes; two workgroups per CU, so
-// the kernel is held to 64 VGPRs (8 waves per SIMD). With 16 waves of one
-// row (16 staged rows for 8 output rows, the gradients staged in LDS too,
-// each input recomputing the terms of the three outputs that read it) the
-// 3840x2160 launch took 249 us; with 8 waves of 4 rows (99 VGPRs, 4 waves
-// per SIMD) 253 us.
-constexpr int kQuadBwdWaves = 16, kQuadBwdRowsPerWave = 2;
-template <int NW, int RPW>
-struct QuadBwdShape {
-    static constexpr int stage = NW * RPW, rows = stage - 8;
+// The passes and their adjoints on pixels inside the border: upwind_px, and
+// upwind_adjoint_px in two halves for kernels that hold every output of a
+// pass. inner_terms gives, once per output, what it contributes to its three
+// inputs (instead of once per input that reads it), and inner_gather_x/_y sum
+// the terms of the outputs j-1, j, j+1 for input j. The expressions and their
+// order are upwind_adjoint_px's, so the results are bitwise its.
+
+// One upwind X pass; lanes 0 and 63 lack a neighbour.
+template <bool PAY>
+__device__ __forceinline__ Px5 inner_pass_x(const Px5& z, float dt) {
+    const float mu = lane_shift<true>(z.f.x), pu = lane_shift<false>(z.f.x);
+    const float Ud = (fabsf(pu) - fabsf(mu)) > 0.0f ? pu : mu;
+    const float nd = -(dt * Ud);
+    float du = z.f.x - mu, dv = z.f.y - lane_shift<true>(z.f.y), ds = 0.f, dx = 0.f, dy = 0.f;
+    Px5 o;
+    if constexpr (PAY) {
+        ds = z.s - lane_shift<true>(z.s);
+        dx = z.v.x - lane_shift<true>(z.v.x);
+        dy = z.v.y - lane_shift<true>(z.v.y);
+        tile::pick(Ud, du, dv, ds, dx, dy);
+        o.s = fmaf(nd, ds, z.s);
+        o.v = make_float2(fmaf(nd, dx, z.v.x), fmaf(nd, dy, z.v.y));
+    } else {
+        tile::pick(Ud, du, dv);
+    }
+    o.f = make_float2(fmaf(nd, du, z.f.x), fmaf(nd, dv, z.f.y));
+    return o;
+}
+
+// What an output contributes to its inputs at o-1, o, o+1: cm, cz, cp times
+// its gradient, and to the speed component gm and gp (one of them 0).
+struct InnerTerms {
+    float cm, cz, cp, gm, gp;
 };
-template <bool PAY, int NW, int RPW>
-__global__ void __launch_bounds__(64 * NW, NW / 2)
+// D: the upwind difference of each field at the output (as fields of a Px5).
+template <bool PAY>
+__device__ __forceinline__ InnerTerms inner_terms(float um, float up, const Px5& D, const Px5& g, float dt) {
+    InnerTerms t;
+    const bool selp = (fabsf(up) - fabsf(um)) > 0.0f;
+    const float Ud = selp ? up : um;
+    const float nd = -(dt * Ud);
+    const bool back = Ud >= 0.0f;
+    t.cz = 1.0f + (back ? nd : -nd);
+    t.cm = back ? -nd : 0.f;
+    t.cp = back ? 0.f : nd;
+    float gUd = g.f.x * D.f.x + g.f.y * D.f.y;
+    if constexpr (PAY) gUd += g.s * D.s + g.v.x * D.v.x + g.v.y * D.v.y;
+    gUd *= -dt;
+    t.gp = selp ? gUd : 0.f;
+    t.gm = selp ? 0.f : gUd;
+    return t;
+}
+// Terms of a Y pass's output from the rows around it.
+template <bool PAY>
+__device__ __forceinline__ InnerTerms inner_terms_y(const Px5& m, const Px5& z, const Px5& p, const Px5& g, float dt) {
+    const bool selp = (fabsf(p.f.y) - fabsf(m.f.y)) > 0.0f;
+    const bool back = (selp ? p.f.y : m.f.y) >= 0.0f;
+    auto d = [&](float a, float b, float c) { return back ? (b - a) : (c - b); };
+    Px5 D;
+    D.f = make_float2(d(m.f.x, z.f.x, p.f.x), d(m.f.y, z.f.y, p.f.y));
+    if constexpr (PAY) {
+        D.s = d(m.s, z.s, p.s);
+        D.v = make_float2(d(m.v.x, z.v.x, p.v.x), d(m.v.y, z.v.y, p.v.y));
+    }
+    return inner_terms<PAY>(m.f.y, p.f.y, D, g, dt);
+}
+// Terms of an X pass's output at this lane's column.
+template <bool PAY>
+__device__ __forceinline__ InnerTerms inner_terms_x(const Px5& z, const Px5& g, float dt) {
+    const float mu = lane_shift<true>(z.f.x), pu = lane_shift<false>(z.f.x);
+    const float Ud = (fabsf(pu) - fabsf(mu)) > 0.0f ? pu : mu;
+    Px5 D;
+    D.f = make_float2(z.f.x - mu, z.f.y - lane_shift<true>(z.f.y));
+    if constexpr (PAY) {
+        D.s = z.s - lane_shift<true>(z.s);
+        D.v = make_float2(z.v.x - lane_shift<true>(z.v.x), z.v.y - lane_shift<true>(z.v.y));
+        tile::pick(Ud, D.f.x, D.f.y, D.s, D.v.x, D.v.y);
+    } else {
+        tile::pick(Ud, D.f.x, D.f.y);
+    }
+    return inner_terms<PAY>(mu, pu, D, g, dt);
+}
+// Input j of a Y pass from the terms and gradients of outputs j-1, j, j+1.
+template <bool PAY>
+__device__ __forceinline__ Px5 inner_gather_y(float cp, float gp, const Px5& g0, float cz, const Px5& g1, float cm,
+                                              float gm, const Px5& g2) {
+    auto sum = [&](float a, float b, float c) { return fmaf(cm, c, fmaf(cz, b, cp * a)); };
+    Px5 r;
+    r.f.x = sum(g0.f.x, g1.f.x, g2.f.x);
+    r.f.y = fmaf(cm, g2.f.y, fmaf(cz, g1.f.y, cp * g0.f.y + gp)) + gm;
+    r.s = 0.f;
+    r.v = make_float2(0.f, 0.f);
+    if constexpr (PAY) {
+        r.s = sum(g0.s, g1.s, g2.s);
+        r.v = make_float2(sum(g0.v.x, g1.v.x, g2.v.x), sum(g0.v.y, g1.v.y, g2.v.y));
+    }
+    return r;
+}
+// Input at this lane's column of an X pass from the terms and gradients of the
+// lanes around it (n: this lane's gradient as its neighbours see it), the lane
+// shifts folded into the multiply-adds as in tile::taps_x2.
+#define FF_SHR " wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define FF_SHL " wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+template <bool PAY>
+__device__ __forceinline__ Px5 inner_gather_x(const InnerTerms& t, const Px5& g, const Px5& n) {
+    const float cp = lane_shift<true>(t.cp), cm = lane_shift<false>(t.cm);
+    Px5 r;
+    r.s = 0.f;
+    r.v = make_float2(0.f, 0.f);
+    asm("s_nop 1\n\t"
+        "v_mul_f32_dpp %0, %9, %4" FF_SHR "v_mul_f32_dpp %1, %10, %4" FF_SHR
+        "v_add_f32_dpp %0, %7, %0" FF_SHR
+        "v_fmac_f32 %0, %5, %2\n\t"
+        "v_fmac_f32 %1, %5, %3\n\t"
+        "v_fmac_f32_dpp %0, %9, %6" FF_SHL "v_fmac_f32_dpp %1, %10, %6" FF_SHL
+        "v_add_f32_dpp %0, %8, %0" FF_SHL
+        : "=&v"(r.f.x), "=&v"(r.f.y)
+        : "v"(g.f.x), "v"(g.f.y), "v"(cp), "v"(t.cz), "v"(cm), "v"(t.gp), "v"(t.gm), "v"(n.f.x), "v"(n.f.y));
+    if constexpr (PAY) {
+        asm("s_nop 1\n\t"
+            "v_mul_f32_dpp %0, %9, %6" FF_SHR "v_mul_f32_dpp %1, %10, %6" FF_SHR "v_mul_f32_dpp %2, %11, %6" FF_SHR
+            "v_fmac_f32 %0, %7, %3\n\t"
+            "v_fmac_f32 %1, %7, %4\n\t"
+            "v_fmac_f32 %2, %7, %5\n\t"
+            "v_fmac_f32_dpp %0, %9, %8" FF_SHL "v_fmac_f32_dpp %1, %10, %8" FF_SHL "v_fmac_f32_dpp %2, %11, %8" FF_SHL
+            : "=&v"(r.s), "=&v"(r.v.x), "=&v"(r.v.y)
+            : "v"(g.s), "v"(g.v.x), "v"(g.v.y), "v"(cp), "v"(t.cz), "v"(cm), "v"(n.s), "v"(n.v.x), "v"(n.v.y));
+    }
+    return r;
+}
+#undef FF_SHR
+#undef FF_SHL
+
+// Adjoint of k_ad_prop_quad (two iterations), recomputing the forward passes
+// inside the launch. A workgroup of 64 x 8 threads covers 64 columns, lane tx
+// being column x0-4+tx, and 32 staged rows, four consecutive ones a thread, of
+// which it writes the inner 56 columns and 24 rows. Every pass works on the
+// thread's own rows and the row above and below them, which the neighbouring
+// waves leave in LDS; a lane's row neighbours come from the adjacent lanes.
+// The steps, with the pixels they are valid on shrinking by one per pass:
+//   first X pass (its edge rows to LDS), first Y pass, second X pass (to LDS);
+//   second Y pass: terms of each output, its edge rows' to LDS with their
+//     gradients, then the gather; second X pass: terms and gather;
+//   first Y pass and first X pass alike.
+// With EDGE, pixels outside the border keep their value (coefficient 1 of
+// themselves, and nothing to their neighbours), and so have no use for what
+// lies around them; pixels outside the image are such pixels. Bitwise the
+// single passes' adjoints.
+//
+// What bounds it: latency, between the reads and behind the four barriers, at
+// 16 waves per CU. 8 waves of four rows held to 128 VGPRs, two workgroups per
+// CU; 113 are used, and what would take more is done again instead: the first X
+// pass is computed twice, and the output gradients are read only when the
+// second Y pass needs them. 3840x2160 with payloads: 140 us, 3.6 TB/s of the
+// 498 MB it has to move (fields and their gradients read, gradients written,
+// five floats a pixel each).
+// Of other forms there: 16 waves of two interleaved rows with whole planes of
+// pixels in LDS and nine barriers 212-225 us (205 us without the border's cases
+// in interior workgroups, though that took out a third of the instructions);
+// the gradients read at the start (14 values spilled) 186 us; the first X pass
+// kept (34 spilled) 216 us; one workgroup of 16 waves per CU, 7/8 instead of
+// 3/4 of the staged rows written, 165 us; five rows per wave 147 us; tiles of
+// an XCD side by side 148 us.
+constexpr int kQuadBwdCols = 56, kQuadBwdWaves = 8, kQuadBwdR = 4;
+constexpr int kQuadBwdRows = kQuadBwdWaves * kQuadBwdR - 8;
+
+// Edge rows in LDS, a value a lane: of each wave, n values of its first row
+// and then n of its last.
+template <bool PAY>
+__device__ __forceinline__ void put_row(float* o, int tx, const Px5& p) {
+    o[0 * 64 + tx] = p.f.x;
+    o[1 * 64 + tx] = p.f.y;
+    if constexpr (PAY) {
+        o[2 * 64 + tx] = p.s;
+        o[3 * 64 + tx] = p.v.x;
+        o[4 * 64 + tx] = p.v.y;
+    }
+}
+template <bool PAY>
+__device__ __forceinline__ Px5 get_row(const float* o, int tx) {
+    Px5 p;
+    p.f = make_float2(o[0 * 64 + tx], o[1 * 64 + tx]);
+    p.s = PAY ? o[2 * 64 + tx] : 0.f;
+    p.v = PAY ? make_float2(o[3 * 64 + tx], o[4 * 64 + tx]) : make_float2(0.f, 0.f);
+    return p;
+}
+
+template <bool PAY, bool EDGE>
+__device__ __forceinline__ void quad_bwd_tile(float (*A)[10][64], float (*B)[14][64], float (*C)[14][64],
+                                              const float2* fin, const float* sin, const float2* vin,
+                                              const float2* gfo, const float* gso, const float2* gvo, float2* gfi,
+                                              float* gsi, float2* gvi, const Dims& d, float dt, int border, int acc,
+                                              int x, int y0, int tx, int w, int b) {
+    constexpr int R = kQuadBwdR, NW = kQuadBwdWaves;
+    const int yw = y0 - 4 + w * R;
+    const int xc = EDGE ? clampi(x, 0, d.W - 1) : x;
+    // inside the border
+    auto in = [&](int r) {
+        return !EDGE || (x >= border && x < d.W - border && yw + r >= border && yw + r < d.H - border);
+    };
+    auto index = [&](int r) { return at(b, EDGE ? clampi(yw + r, 0, d.H - 1) : yw + r, xc, d); };
+    auto keep = [&](int r, const Px5& o, const Px5& z) { return !EDGE || in(r) ? o : z; };
+    // a gradient as its neighbours see it
+    auto shown = [&](int r, Px5 g) {
+        if (EDGE && !in(r)) {
+            g.f = g.v = make_float2(0.f, 0.f);
+            g.s = 0.f;
+        }
+        return g;
+    };
+    auto terms = [&](int r, InnerTerms t) {
+        if (EDGE && !in(r)) {
+            t.cm = t.cp = t.gm = t.gp = 0.f;
+            t.cz = 1.f;
+        }
+        return t;
+    };
+    const int wa = w > 0 ? w - 1 : 0, wb = w < NW - 1 ? w + 1 : NW - 1;  // waves above and below
+
+    // ---- forward
+    Px5 F[R], Y1[R], X2[R], G[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) F[r] = load_px<PAY>(fin, sin, vin, index(r));
+    // (computed again for the first Y pass's terms: cheaper than the registers)
+    auto first_x = [&](Px5 (&X1)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) X1[r] = keep(r, inner_pass_x<PAY>(F[r], dt), F[r]);
+    };
+    {
+        Px5 X1[R];
+        first_x(X1);
+        put_row<PAY>(A[w][0], tx, X1[0]);
+        put_row<PAY>(A[w][5], tx, X1[R - 1]);
+        __syncthreads();
+        const Px5 up = get_row<PAY>(A[wa][5], tx), down = get_row<PAY>(A[wb][0], tx);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            Y1[r] = upwind_px<1, PAY>(r > 0 ? X1[r > 0 ? r - 1 : 0] : up, X1[r], r + 1 < R ? X1[r + 1 < R ? r + 1 : 0] : down,
+                                      dt, in(r));
+            X2[r] = keep(r, inner_pass_x<PAY>(Y1[r], dt), Y1[r]);
+        }
+    }
+    put_row<PAY>(B[w][0], tx, X2[0]);
+    put_row<PAY>(B[w][5], tx, X2[R - 1]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) G[r] = load_grad_px<PAY>(gfo, gso, gvo, index(r));
+    __syncthreads();
+
+    InnerTerms t[R];
+    // Gradient at each row of a Y pass's input: its output's terms `t` and
+    // gradients g, and the edge rows of both in E.
+    auto export_terms = [&](float (*E)[14][64], const Px5 (&g)[R]) {
+        put_row<PAY>(E[w][0], tx, shown(0, g[0]));
+        E[w][5][tx] = t[0].cm;
+        E[w][6][tx] = t[0].gm;
+        put_row<PAY>(E[w][7], tx, shown(R - 1, g[R - 1]));
+        E[w][12][tx] = t[R - 1].cp;
+        E[w][13][tx] = t[R - 1].gp;
+    };
+    auto gather = [&](float (*E)[14][64], const Px5 (&g)[R], int r) {
+        const Px5 g0 = r > 0 ? shown(r - 1, g[r > 0 ? r - 1 : 0]) : get_row<PAY>(E[wa][7], tx);
+        const Px5 g2 = r + 1 < R ? shown(r + 1, g[r + 1 < R ? r + 1 : 0]) : get_row<PAY>(E[wb][0], tx);
+        const float cp = r > 0 ? t[r > 0 ? r - 1 : 0].cp : E[wa][12][tx], gp = r > 0 ? t[r > 0 ? r - 1 : 0].gp : E[wa][13][tx];
+        const float cm = r + 1 < R ? t[r + 1 < R ? r + 1 : 0].cm : E[wb][5][tx],
+                    gm = r + 1 < R ? t[r + 1 < R ? r + 1 : 0].gm : E[wb][6][tx];
+        return inner_gather_y<PAY>(cp, gp, g0, t[r].cz, g[r], cm, gm, g2);
+    };
+    // ---- second Y pass: terms
+    {
+        const Px5 up = get_row<PAY>(B[wa][5], tx), down = get_row<PAY>(B[wb][0], tx);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            t[r] = terms(r, inner_terms_y<PAY>(r > 0 ? X2[r > 0 ? r - 1 : 0] : up, X2[r],
+                                               r + 1 < R ? X2[r + 1 < R ? r + 1 : 0] : down, G[r], dt));
+    }
+    export_terms(C, G);
+    __syncthreads();
+    // ---- its gather, and the second X pass
+    Px5 gy[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const Px5 g = gather(C, G, r);
+        gy[r] = inner_gather_x<PAY>(terms(r, inner_terms_x<PAY>(Y1[r], g, dt)), g, shown(r, g));
+    }
+    // ---- first Y pass: terms (the first X pass's edge rows are still in A;
+    // every wave is past its reads of B)
+    {
+        Px5 X1[R];
+        first_x(X1);
+        const Px5 up = get_row<PAY>(A[wa][5], tx), down = get_row<PAY>(A[wb][0], tx);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            t[r] = terms(r, inner_terms_y<PAY>(r > 0 ? X1[r > 0 ? r - 1 : 0] : up, X1[r],
+                                               r + 1 < R ? X1[r + 1 < R ? r + 1 : 0] : down, gy[r], dt));
+    }
+    export_terms(B, gy);
+    __syncthreads();
+    // ---- its gather, and the first X pass
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const Px5 g = gather(B, gy, r);
+        const Px5 o = inner_gather_x<PAY>(terms(r, inner_terms_x<PAY>(F[r], g, dt)), g, shown(r, g));
+        if (w >= 1 && w <= NW - 2 && tx >= 4 && tx < kQuadBwdCols + 4 && (!EDGE || (x < d.W && yw + r < d.H)))
+            put_px<PAY>(gfi, gsi, gvi, at(b, yw + r, x, d), o, acc);
+    }
+}
+
+template <bool PAY>
+__global__ void __launch_bounds__(64 * kQuadBwdWaves, 4)
     k_ad_prop_quad_bwd(const float2* fin, const float* sin, const float2* vin, const float2* gfo, const float* gso,
                        const float2* gvo, float2* gfi, float* gsi, float2* gvi, Dims d, float dt, int border,
                        int acc) {
-    constexpr int S = QuadBwdShape<NW, RPW>::stage, R = QuadBwdShape<NW, RPW>::rows;
-    __shared__ LdsRows<S> LA;  // first X pass; later the first Y pass's terms
-    __shared__ LdsRows<S> LB;  // second X pass; later the second Y pass's terms, then the first Y pass's output gradient
+    // 76 KB: two workgroups to a CU
+    __shared__ float A[kQuadBwdWaves][10][64], B[kQuadBwdWaves][14][64], C[kQuadBwdWaves][14][64];
     const int tx = threadIdx.x, w = wave_y(), b = blockIdx.z;
-    const int x = (int)blockIdx.x * kQuadBwdCols - 3 + tx;  // column of this lane
-    const int y0 = (int)blockIdx.y * R;
-    const int xc = clampi(x, 0, d.W - 1);
-    const bool xin = x >= border && x < d.W - border;
-    auto srow = [&](int r) { return clampi(r, 0, d.H - 1) - (y0 - 4); };  // staged row of image row clamp(r)
-    Px5 zero;
-    zero.f = make_float2(0.f, 0.f);
-    zero.s = 0.f;
-    zero.v = make_float2(0.f, 0.f);
-    const bool xvalid[3] = {x - 1 >= 0 && x - 1 < d.W, x >= 0 && x < d.W, x + 1 >= 0 && x + 1 < d.W};
-    // this wave's staged rows i = w + NW k, image rows y0-4+i
-    Px5 F[RPW], Y1[RPW], gy1[RPW];
-    int yr[RPW], yc[RPW];
-    bool in[RPW], pix[RPW];
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = w + NW * k;
-        yr[k] = y0 - 4 + i;
-        yc[k] = clampi(yr[k], 0, d.H - 1);
-        in[k] = xin && yc[k] >= border && yc[k] < d.H - border;
-        pix[k] = x >= 0 && x < d.W && yr[k] >= 0 && yr[k] < d.H;
-    }
-    auto yinterior = [&](int o) { return xin && o >= border && o < d.H - border; };
-
-    // ---- forward
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = w + NW * k;
-        F[k] = load_px<PAY>(fin, sin, vin, at(b, yc[k], xc, d));
-        Px5 m = lane_shift_px<true, PAY>(F[k]), p = lane_shift_px<false, PAY>(F[k]);
-        if (tx == 0) m = load_px<PAY>(fin, sin, vin, at(b, yc[k], clampi(x - 1, 0, d.W - 1), d));
-        if (tx == 63) p = load_px<PAY>(fin, sin, vin, at(b, yc[k], clampi(x + 1, 0, d.W - 1), d));
-        LA.template put<PAY>(i, tx, upwind_px<0, PAY>(m, F[k], p, dt, in[k]));
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = w + NW * k;
-        const bool mid = i >= 1 && i <= S - 2;  // rows of the first Y and second X pass
-        Y1[k] = zero;
-        if (mid)
-            Y1[k] = upwind_px<1, PAY>(LA.template get<PAY>(srow(yc[k] - 1), tx), LA.template get<PAY>(srow(yc[k]), tx),
-                                      LA.template get<PAY>(srow(yc[k] + 1), tx), dt, in[k]);
-        const Px5 m = lane_shift_px<true, PAY>(Y1[k]), p = lane_shift_px<false, PAY>(Y1[k]);
-        if (mid) LB.template put<PAY>(i, tx, upwind_px<0, PAY>(m, Y1[k], p, dt, in[k]));
-    }
-    __syncthreads();
-
-    // ---- second Y pass: terms of output rows 2 .. S-3 (inside the image)
-    OutTerms t[RPW];
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = w + NW * k;
-        t[k] = out_terms<1, PAY>(zero, zero, zero, zero, false, dt);
-        if (i >= 2 && i <= S - 3 && pix[k] && tx >= 1 && tx <= 62) {
-            const Px5 g = load_grad_px<PAY>(gfo, gso, gvo, at(b, yr[k], xc, d));
-            t[k] = out_terms<1, PAY>(LB.template get<PAY>(srow(yr[k] - 1), tx), LB.template get<PAY>(srow(yr[k]), tx),
-                                     LB.template get<PAY>(srow(yr[k] + 1), tx), g, yinterior(yr[k]), dt);
-        }
-    }
-    __syncthreads();  // every read of LB (second X pass) is done
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) LB.put_terms(w + NW * k, tx, t[k]);
-    __syncthreads();
-
-    // ---- gathers of the second pair (rows 3 .. S-4)
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = w + NW * k;
-        const bool rows2 = i >= 3 && i <= S - 4;
-        Px5 g_x2 = zero;
-        if (rows2 && pix[k] && tx >= 1 && tx <= 62) {
-            OutTerms T[3];
-            Px5 G[3];
-            bool valid[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const int o = yr[k] - 1 + q;  // output row, staged row i-1+q
-                valid[q] = o >= 0 && o < d.H;
-                T[q] = LB.get_terms(i - 1 + q, tx);
-                G[q] = load_grad_px<PAY>(gfo, gso, gvo, at(b, clampi(o, 0, d.H - 1), xc, d));
-            }
-            g_x2 = gather_px<1, PAY>(T, G, valid);
-        }
-        // second X pass: terms at this lane's column, gathered from the
-        // adjacent lanes
-        const bool yin = yr[k] >= border && yr[k] < d.H - border;
-        const Px5 m1 = lane_shift_px<true, PAY>(Y1[k]), p1 = lane_shift_px<false, PAY>(Y1[k]);
-        const OutTerms to = out_terms<0, PAY>(m1, Y1[k], p1, g_x2, yin && x >= border && x < d.W - border, dt);
-        const OutTerms T3[3] = {lane_shift_terms<true>(to), to, lane_shift_terms<false>(to)};
-        const Px5 G3[3] = {lane_shift_px<true, PAY>(g_x2), g_x2, lane_shift_px<false, PAY>(g_x2)};
-        gy1[k] = zero;
-        if (rows2 && pix[k] && tx >= 2 && tx <= 61) gy1[k] = gather_px<0, PAY>(T3, G3, xvalid);
-    }
-    __syncthreads();  // every read of LB (the second Y pass's terms) is done
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) LB.template put<PAY>(w + NW * k, tx, gy1[k]);
-    __syncthreads();
-
-    // ---- first Y pass: terms of output rows 3 .. S-4
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = w + NW * k;
-        t[k] = out_terms<1, PAY>(zero, zero, zero, zero, false, dt);
-        if (i >= 3 && i <= S - 4 && pix[k] && tx >= 2 && tx <= 61)
-            t[k] = out_terms<1, PAY>(LA.template get<PAY>(srow(yr[k] - 1), tx), LA.template get<PAY>(srow(yr[k]), tx),
-                                     LA.template get<PAY>(srow(yr[k] + 1), tx), LB.template get<PAY>(i, tx), yinterior(yr[k]), dt);
-    }
-    __syncthreads();  // every read of LA (first X pass) is done
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) LA.put_terms(w + NW * k, tx, t[k]);
-    __syncthreads();
-
-    // ---- gathers of the first pair (rows 4 .. S-5), written for lanes 3..60
-#pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = w + NW * k;
-        const bool rows1 = i >= 4 && i <= S - 5;
-        Px5 g_x1 = zero;
-        if (rows1 && pix[k] && tx >= 2 && tx <= 61) {
-            OutTerms T[3];
-            Px5 G[3];
-            bool valid[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const int o = yr[k] - 1 + q;
-                valid[q] = o >= 0 && o < d.H;
-                T[q] = LA.get_terms(i - 1 + q, tx);
-                G[q] = LB.template get<PAY>(i - 1 + q, tx);
-            }
-            g_x1 = gather_px<1, PAY>(T, G, valid);
-        }
-        const bool yin = yr[k] >= border && yr[k] < d.H - border;
-        const Px5 m1 = lane_shift_px<true, PAY>(F[k]), p1 = lane_shift_px<false, PAY>(F[k]);
-        const OutTerms to = out_terms<0, PAY>(m1, F[k], p1, g_x1, yin && x >= border && x < d.W - border, dt);
-        const OutTerms T3[3] = {lane_shift_terms<true>(to), to, lane_shift_terms<false>(to)};
-        const Px5 G3[3] = {lane_shift_px<true, PAY>(g_x1), g_x1, lane_shift_px<false, PAY>(g_x1)};
-        if (rows1 && pix[k] && tx >= 3 && tx < kQuadBwdCols + 3)
-            put_px<PAY>(gfi, gsi, gvi, at(b, yr[k], x, d), gather_px<0, PAY>(T3, G3, xvalid), acc);
-    }
+    const int x = (int)blockIdx.x * kQuadBwdCols - 4 + tx;
+    const int y0 = (int)blockIdx.y * kQuadBwdRows;
+    // whether every pixel read, the row neighbours of the edge lanes included,
+    // lies inside the border
+    const int xa = (int)blockIdx.x * kQuadBwdCols - 5, ya = y0 - 5;
+    if (xa >= border && xa + 65 < d.W - border && ya >= border && ya + kQuadBwdRows + 9 < d.H - border)
+        quad_bwd_tile<PAY, false>(A, B, C, fin, sin, vin, gfo, gso, gvo, gfi, gsi, gvi, d, dt, border, acc, x, y0, tx, w, b);
+    else
+        quad_bwd_tile<PAY, true>(A, B, C, fin, sin, vin, gfo, gso, gvo, gfi, gsi, gvi, d, dt, border, acc, x, y0, tx, w, b);
 }
 
 // ----------------------------------------------------------------- update
@@ -1477,18 +1503,16 @@ void prop_quad(const float* fin, const float* sin, const float* vin, float* fout
 void prop_quad_bwd(const float* fin, const float* sin, const float* vin, const float* gfo, const float* gso,
                    const float* gvo, float* gfi, float* gsi, float* gvi, int B, int H, int W, float dt, int border,
                    int acc, hipStream_t s) {
-    constexpr int NW = kQuadBwdWaves, RPW = kQuadBwdRowsPerWave;
-    constexpr int rows = QuadBwdShape<NW, RPW>::rows;
-    const dim3 g((W + kQuadBwdCols - 1) / kQuadBwdCols, (H + rows - 1) / rows, B), blk(64, NW);
+    const dim3 g((W + kQuadBwdCols - 1) / kQuadBwdCols, (H + kQuadBwdRows - 1) / kQuadBwdRows, B), blk(64, kQuadBwdWaves);
     const Dims d{H, W};
     auto F = [](const float* p) { return (const float2*)p; };
     auto O = [](float* p) { return (float2*)p; };
     if (sin)
-        hipLaunchKernelGGL((k_ad_prop_quad_bwd<true, NW, RPW>), g, blk, 0, s, F(fin), sin, F(vin), F(gfo), gso,
-                           F(gvo), O(gfi), gsi, O(gvi), d, dt, border, acc);
+        hipLaunchKernelGGL((k_ad_prop_quad_bwd<true>), g, blk, 0, s, F(fin), sin, F(vin), F(gfo), gso, F(gvo), O(gfi),
+                           gsi, O(gvi), d, dt, border, acc);
     else
-        hipLaunchKernelGGL((k_ad_prop_quad_bwd<false, NW, RPW>), g, blk, 0, s, F(fin), sin, F(vin), F(gfo), gso,
-                           F(gvo), O(gfi), gsi, O(gvi), d, dt, border, acc);
+        hipLaunchKernelGGL((k_ad_prop_quad_bwd<false>), g, blk, 0, s, F(fin), sin, F(vin), F(gfo), gso, F(gvo), O(gfi),
+                           gsi, O(gvi), d, dt, border, acc);
 }
 void prop_pair_bwd(const float* fin, const float* sin, const float* vin, const float* fmid, const float* smid,
                    const float* vmid, const float* gfo, const float* gso, const float* gvo, float* gfi, float* gsi,

@@ -167,3 +167,43 @@ def test_ad_tile_adjoints(B, h, w, n, second, acc):
     plain = torch.empty_like(img)
     N.call("ff_ad_image_model_backward", p(ga), p(gg), p(plain), p(work), B, h, w, 0, s)
     assert torch.equal(inplace, plain)
+
+
+@pytest.mark.parametrize("B,h,w,border", [(1, 80, 180, 1), (2, 57, 122, 1), (1, 81, 181, 3), (1, 49, 113, 20),
+                                          (1, 120, 240, 2)])
+@pytest.mark.parametrize("pay", [False, True])
+@pytest.mark.parametrize("special", [False, True])
+def test_ad_two_iterations_adjoint(B, h, w, border, pay, special):
+    """The adjoint of two propagation iterations in one launch, at sizes with
+    workgroups wholly inside the border (and one pixel short of that), is
+    bitwise the adjoints of the two iterations, infinite and NaN flows and
+    gradients included."""
+    import ctypes
+
+    import torch
+    from flowfilter import _native as N
+    print("ad two iterations", (B, h, w), border, pay, special, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(h * 5 + w)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    dt = ctypes.c_float(0.25)
+    new = lambda: [rnd(B, h, w, 2), rnd(B, h, w) if pay else None, rnd(B, h, w, 2) if pay else None]
+    f, go, mid, gmid, ref = new(), new(), new(), new(), new()
+    if special:
+        for k, t in enumerate((f[0], go[0])):
+            for i, v in enumerate((float("inf"), float("nan"), -float("inf"))):
+                t[0, (7 + 17 * i + 31 * k) % h, (5 + 41 * i + 23 * k) % w, i % 2] = v
+                t[-1, 0, (60 * i + k) % w, 0] = v
+    got = [t.clone() if t is not None else None for t in ref]
+    acc = 5  # (added to the flow's and the vector's, the scalar's written)
+    N.call("ff_ad_propagate_pair", *map(p, f), None, None, None, *map(p, mid), B, h, w, dt, border, s)
+    N.call("ff_ad_propagate_pair_backward", *map(p, mid), None, None, None, *map(p, go), *map(p, gmid), B, h, w, dt,
+           border, 0, s)
+    N.call("ff_ad_propagate_pair_backward", *map(p, f), None, None, None, *map(p, gmid), *map(p, ref), B, h, w, dt,
+           border, acc, s)
+    N.call("ff_ad_propagate_quad_backward", *map(p, f), *map(p, go), *map(p, got), B, h, w, dt, border, acc, s)
+    for a, b in zip(ref, got):
+        if a is not None:
+            assert torch.equal(torch.isnan(a), torch.isnan(b))
+            assert torch.equal(torch.nan_to_num(a, nan=0.0), torch.nan_to_num(b, nan=0.0))
