@@ -530,6 +530,35 @@ FF_API ff_status ff_ad_propagate_steps(const float* flow, const float* scalar, c
                                        int after, float* flow_mid, float* scalar_mid, float* vector_mid,
                                        float* flow_out, float* scalar_out, float* vector_out, int B, int H, int W,
                                        float dt, int border, void* stream);
+/* One level of one frame in one launch: propagation (iterations), image
+ * model, update and smoothing (smooth_iterations), the same results as the
+ * functions for each. With iterations = 0, flow (top level) or bright and
+ * dflow (delta level; flow is not read) are propagated already. Images of a
+ * batch one after the other. */
+typedef struct ff_ad_level {
+    const float* image;
+    const float *flow, *bright;      /* the old smoothed flow and brightness */
+    const float *dflow, *upper;      /* delta level (top level: NULL): the old delta flow, the flow above */
+    const int *xmap, *ymap;          /* delta level: the column and row read above */
+    float *flow_out, *bright_out;    /* the new smoothed flow and brightness */
+    float* dflow_out;                /* delta level: the new delta flow */
+    float* flow_upd;                 /* top level: the unsmoothed new flow, or NULL */
+    /* what the adjoints read, or all NULL */
+    float* grad;                     /* the image model's gradient */
+    float* prop_flow;                /* top level: the propagated flow (NULL if iterations is 0) */
+    float *prop_scalar, *prop_vector;                /* delta level: the propagated payloads (likewise) */
+    float *mid_flow, *mid_scalar, *mid_vector;       /* fields (top level: the flow alone) after 2, 4, .. iterations
+                                                        short of all, a batch each; NULL if iterations <= 2 */
+} ff_ad_level;
+/* Whether ff_ad_level_forward takes a level of this size and iterations (its
+ * flow image below 2 GiB; twice max(iterations, 2) + 2 smooth_iterations
+ * below 64). */
+FF_API ff_status ff_ad_level_supported(int H, int W, int iterations, int smooth_iterations, int* supported);
+/* No output may be an input. gamma, maxflow: as for ff_ad_update (top level)
+ * and ff_ad_delta_update; border >= 1. */
+FF_API ff_status ff_ad_level_forward(const ff_ad_level* level, int iterations, int smooth_iterations, int B, int H,
+                                     int W, int Hu, int Wu, float dt, int border, float gamma, float maxflow,
+                                     void* stream);
 /* Adjoint of ff_ad_propagate_quad given the quad's input only (its three
  * inner passes are recomputed inside the launch); bitwise the adjoints of
  * the two pairs. g_*_out may be NULL (zero); accumulate as for the pass

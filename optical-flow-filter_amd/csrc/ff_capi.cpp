@@ -967,6 +967,50 @@ ff_status ff_ad_propagate_steps(const float* flow, const float* scalar, const fl
         check_launch("ff_ad_propagate_steps");
     });
 }
+ff_status ff_ad_level_supported(int H, int W, int iterations, int smooth_iterations, int* supported) {
+    return guard([&] {
+        need(supported, "supported");
+        *supported = level_tile_supported(H, W, iterations, smooth_iterations) ? 1 : 0;
+    });
+}
+ff_status ff_ad_level_forward(const ff_ad_level* level, int iterations, int smooth_iterations, int B, int H, int W,
+                              int Hu, int Wu, float dt, int border, float gamma, float maxflow, void* stream) {
+    return guard([&] {
+        need(level, "level");
+        const ff_ad_level& l = *level;
+        dims(B, H, W);
+        if (border < 1) throw invalid_argument("border must be at least 1");
+        if (!level_tile_supported(H, W, iterations, smooth_iterations))
+            throw invalid_argument("iterations or image size not supported in one launch");
+        const bool delta = l.dflow != nullptr, save = l.grad != nullptr;
+        for (const void* p : {l.image, l.flow, l.bright, (const float*)l.flow_out, (const float*)l.bright_out})
+            need(p, "argument");
+        if (delta) {
+            dims(B, Hu, Wu);
+            for (const void* p : {(const void*)l.upper, (const void*)l.xmap, (const void*)l.ymap,
+                                  (const void*)l.dflow_out})
+                need(p, "argument of a delta level");
+        } else if (l.upper || l.dflow_out) {
+            throw invalid_argument("a delta level needs dflow");
+        }
+        if (save) {
+            if (iterations > 0 && (delta ? (!l.prop_scalar || !l.prop_vector) : !l.prop_flow))
+                throw invalid_argument("pass the propagated fields with the gradient");
+            if (iterations > 2 && (!l.mid_flow || (delta && (!l.mid_scalar || !l.mid_vector))))
+                throw invalid_argument("pass the middle fields with the gradient");
+        }
+        for (const float* in : {l.image, l.flow, l.bright, l.dflow, l.upper})
+            for (const float* out : {l.flow_out, l.bright_out, l.dflow_out, l.flow_upd, l.grad, l.prop_flow,
+                                     l.prop_scalar, l.prop_vector, l.mid_flow, l.mid_scalar, l.mid_vector})
+                if (in && in == out) throw invalid_argument("outputs must not be the inputs (the passes read neighbours)");
+        const LevelFields f{l.image,      l.flow,        l.bright,      l.dflow,    l.upper,      l.xmap,
+                            l.ymap,       l.flow_out,    l.bright_out,  l.dflow_out, l.flow_upd,  l.grad,
+                            l.prop_flow,  l.prop_scalar, l.prop_vector, l.mid_flow, l.mid_scalar, l.mid_vector};
+        launch_level_tile(f, B, H, W, Hu, Wu, iterations, smooth_iterations, border, dt, gamma, maxflow,
+                          as_stream(stream));
+        check_launch("ff_ad_level_forward");
+    });
+}
 ff_status ff_ad_propagate_quad_backward(const float* flow, const float* scalar, const float* vector,
                                         const float* g_flow_out, const float* g_scalar_out, const float* g_vector_out,
                                         float* g_flow, float* g_scalar, float* g_vector, int B, int H, int W, float dt,

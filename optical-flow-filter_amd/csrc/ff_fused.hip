@@ -238,61 +238,6 @@ __device__ __forceinline__ void signal_done(const LevelJob& p, int t, const Geo&
 
 // ------------------------------------------------------------ tile body
 
-// Image model (imagePrefilter_k / imageModel_k, imagemodel_k.cu:31-133) and
-// update (flowUpdate_k, update_k.cu:15-79, or deltaFlowUpdate_k, :82-173)
-// of every row of the thread. im[j] is image row yw-2+j (clamped reads),
-// aold[r] the old brightness (top level) and up[r] the upper-level flow
-// (delta level) of row r. Writes the new brightness (and delta flow) of the
-// tile's output pixels; leaves the updated flow in s.fu/s.fv.
-template <bool DELTA, bool CLAMP, int R>
-__device__ __forceinline__ void model_update(State<DELTA, R>& s, const float (&im)[R + 4], const float (&aold)[R],
-                                             const float2 (&up)[R], const LevelJob& p, const Rsrc& ra0,
-                                             const Rsrc& rdf, const Rsrc& rfu, const int (&offa)[R],
-                                             const int (&offf)[R]) {
-    float sx[R + 4];
-#pragma unroll
-    for (int j = 0; j < R + 4; ++j) sx[j] = taps_x<CLAMP>(im[j], WSmooth{});
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        float sy = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 5; ++k) sy = fmaf(smooth_w(k), im[r + k], sy);
-        const float a0 = taps_x<CLAMP>(sy, WSmooth{});
-        const float gx = taps_x<CLAMP>(sy, WDiff{});
-        float gy = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 5; ++k) gy = fmaf(diff_w(k), sx[r + k], gy);
-        float ox, oy;
-        if constexpr (DELTA) {
-            const float Yt = s.sa[r] - a0;
-            solve2x2(gx, gy, Yt, s.du[r], s.dv[r], p.gamma, ox, oy);
-            ox = not_finite(ox) ? 0.0f : ox;
-            oy = not_finite(oy) ? 0.0f : oy;
-            const float half = 0.5f * p.maxflow;
-            ox = fmaxf(-half, fminf(ox, half));
-            oy = fmaxf(-half, fminf(oy, half));
-            float fx = ox + 2.0f * up[r].x, fy = oy + 2.0f * up[r].y;
-            fx = fmaxf(-p.maxflow, fminf(fx, p.maxflow));
-            fy = fmaxf(-p.maxflow, fminf(fy, p.maxflow));
-            st1(ra0, offa[r], a0);
-            st2(rdf, offf[r], ox, oy);
-            ox = fx;
-            oy = fy;
-        } else {
-            const float Yt = aold[r] - a0;
-            solve2x2(gx, gy, Yt, s.fu[r], s.fv[r], p.gamma, ox, oy);
-            ox = fmaxf(-p.maxflow, fminf(ox, p.maxflow));
-            oy = fmaxf(-p.maxflow, fminf(oy, p.maxflow));
-            ox = not_finite(ox) ? 0.0f : ox;
-            oy = not_finite(oy) ? 0.0f : oy;
-            st1(ra0, offa[r], a0);
-            if (p.flow_upd) st2(rfu, offf[r], ox, oy);
-        }
-        s.fu[r] = ox;
-        s.fv[r] = oy;
-    }
-}
-
 // Image rows yw-2 .. yw+R+1 (clamped to the level) at the thread's column.
 // load_image issues the loads; finish_image turns them into normalized
 // values once they are needed, so the latency of the F32 and U8 loads
@@ -574,8 +519,9 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
     }
     float im[R + 4];
     finish_image<MODE, R>(ir, im);
-    if (!INNER && xedge) model_update<DELTA, true, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf);
-    else model_update<DELTA, false, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf);
+    const auto none = [](int, float, float) {};
+    if (!INNER && xedge) model_update<DELTA, true, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf, none);
+    else model_update<DELTA, false, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf, none);
 
     }
     // ------------------------------------------------------------ smoothing

@@ -304,6 +304,24 @@ private:
     Impl* impl_;
 };
 
+// A level of the differentiable form (launch_level_tile): contiguous images of
+// a batch, float2 where named a flow, a gradient or a vector. Read: image, the
+// old flow and brightness, and on a delta level (dflow not null) the old delta
+// flow, the upper level's flow and the index maps into it. Written: the new
+// smoothed flow, brightness and delta flow, and on a top level the unsmoothed
+// flow unless null. For the adjoints, with grad not null: the image gradient,
+// the propagated flow (top) or payloads (delta), and the fields after 2, 4, ..
+// iterations, each a batch, unless n <= 2.
+struct LevelFields {
+    const float *image, *flow, *bright, *dflow, *upper;
+    const int *xmap, *ymap;
+    float *flow_out, *bright_out, *dflow_out, *flow_upd;
+    float *grad, *prop_flow, *prop_scalar, *prop_vector, *mid_flow, *mid_scalar, *mid_vector;
+};
+bool level_tile_supported(int H, int W, int n, int K);
+void launch_level_tile(const LevelFields& f, int B, int H, int W, int Hu, int Wu, int n, int K, int border, float dt,
+                       float gamma, float maxflow, hipStream_t s);
+
 // ------------------------------------------------- differentiable form
 // Batched forward stages on float images and their adjoints
 // (ff_adjoint.hip). B contiguous images of H x W; vector fields are float2.

@@ -318,6 +318,63 @@ __device__ __forceinline__ void prop_y(State<DELTA, R>& s, const Geo& g, const P
     }
 }
 
+// Image model (imagePrefilter_k / imageModel_k, imagemodel_k.cu:31-133) and
+// update (flowUpdate_k, update_k.cu:15-79, or deltaFlowUpdate_k, :82-173)
+// of every row of the thread. im[j] is image row yw-2+j (clamped reads),
+// aold[r] the old brightness (top level) and up[r] the upper-level flow
+// (delta level) of row r. Writes the new brightness (and delta flow) of the
+// tile's output pixels; leaves the updated flow in s.fu/s.fv. p: gamma, maxflow
+// and flow_upd. gradient(r, gx, gy) is called for each row.
+template <bool DELTA, bool CLAMP, int R, class P, class G>
+__device__ __forceinline__ void model_update(State<DELTA, R>& s, const float (&im)[R + 4], const float (&aold)[R],
+                                             const float2 (&up)[R], const P& p, const Rsrc& ra0,
+                                             const Rsrc& rdf, const Rsrc& rfu, const int (&offa)[R],
+                                             const int (&offf)[R], G&& gradient) {
+    float sx[R + 4];
+#pragma unroll
+    for (int j = 0; j < R + 4; ++j) sx[j] = taps_x<CLAMP>(im[j], WSmooth{});
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        float sy = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) sy = fmaf(smooth_w(k), im[r + k], sy);
+        const float a0 = taps_x<CLAMP>(sy, WSmooth{});
+        const float gx = taps_x<CLAMP>(sy, WDiff{});
+        float gy = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) gy = fmaf(diff_w(k), sx[r + k], gy);
+        gradient(r, gx, gy);
+        float ox, oy;
+        if constexpr (DELTA) {
+            const float Yt = s.sa[r] - a0;
+            solve2x2(gx, gy, Yt, s.du[r], s.dv[r], p.gamma, ox, oy);
+            ox = not_finite(ox) ? 0.0f : ox;
+            oy = not_finite(oy) ? 0.0f : oy;
+            const float half = 0.5f * p.maxflow;
+            ox = fmaxf(-half, fminf(ox, half));
+            oy = fmaxf(-half, fminf(oy, half));
+            float fx = ox + 2.0f * up[r].x, fy = oy + 2.0f * up[r].y;
+            fx = fmaxf(-p.maxflow, fminf(fx, p.maxflow));
+            fy = fmaxf(-p.maxflow, fminf(fy, p.maxflow));
+            st1(ra0, offa[r], a0);
+            st2(rdf, offf[r], ox, oy);
+            ox = fx;
+            oy = fy;
+        } else {
+            const float Yt = aold[r] - a0;
+            solve2x2(gx, gy, Yt, s.fu[r], s.fv[r], p.gamma, ox, oy);
+            ox = fmaxf(-p.maxflow, fminf(ox, p.maxflow));
+            oy = fmaxf(-p.maxflow, fminf(oy, p.maxflow));
+            ox = not_finite(ox) ? 0.0f : ox;
+            oy = not_finite(oy) ? 0.0f : oy;
+            st1(ra0, offa[r], a0);
+            if (p.flow_upd) st2(rfu, offf[r], ox, oy);
+        }
+        s.fu[r] = ox;
+        s.fv[r] = oy;
+    }
+}
+
 // Lanes beyond the image's last column (lane xlast) take its values.
 template <int R>
 __device__ __forceinline__ void copy_last_column(float (&fu)[R], float (&fv)[R], int lane, int xlast) {

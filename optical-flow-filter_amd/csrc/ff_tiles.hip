@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "ff_device.hpp"
 #include "ff_kernels.hpp"
@@ -180,6 +181,159 @@ __global__ void __launch_bounds__(1024, 8) k_propagate_tile(PropFields in, PropF
         store(middle ? mid : out);
         if (!middle) break;
     }
+}
+
+// --------------------------------------------------------- a whole level
+
+// What the passes, the update and the outputs of a level read (as the fused
+// frame kernel's job).
+struct LevelParams {
+    float dt;
+    int border, H;
+    float gamma, maxflow;
+    float2* flow_upd;
+};
+
+// One level of one frame of the differentiable form, images of a batch: n
+// propagation iterations of the old flow (on a delta level with the old
+// brightness and delta flow as payloads; without PROP none, what is read being
+// propagated already), the image model, the update and K smoothing iterations,
+// as the fused frame kernel's tiles. SAVE: what the adjoints read is written as
+// well: the fields after every two iterations but the last (f.mid_*, images of a
+// batch one after the other, then the next two iterations'), the propagated
+// fields and the image gradient. Halo: max(n, 2) + 2 K, an error's way in from
+// the buffer's edge.
+//
+// What bounds it: without PROP, HBM and the latency of its four phases (3840x2160
+// delta level, K = 1: 95 us for 316 MB, with the gradient 117 us for 382 MB; the
+// launches it replaces, image model, update and smoothing, took 149 us). With
+// PROP, the VALU: n = 4 193 us, n = 8 338 us, the halo being 6 and 10 of 64
+// columns. 16 x 512x512, n = 4: 101 us (161 in four launches).
+template <bool DELTA, bool SAVE, bool PROP>
+__global__ void __launch_bounds__(1024, 8) k_level_tile(LevelFields f, Tiling tl, int Hu, int Wu, int n, int K,
+                                                        LevelParams lp) {
+    constexpr int R = kTileRows;
+    extern __shared__ float xch[];
+    const int nw = (int)blockDim.x / LANES, b = (int)blockIdx.y, B = (int)gridDim.y;
+    const TilePos p = tile_pos(tl, nw, lp.border);
+    const Geo& g = p.g;
+    const int pa = tl.W * 4, pf = tl.W * 8;  // row pitches in bytes
+    State<DELTA, R> s;
+    {
+        const Rsrc rf = image_rsrc(f.flow, pf, tl.H, b), rs = image_rsrc(f.bright, pa, tl.H, b),
+                   rv = image_rsrc(f.dflow, pf, tl.H, b);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int y = min(g.yw + r, tl.H - 1);
+            if constexpr (PROP || !DELTA) {
+                const float2 v = ld2(rf, y * pf + g.xl * 8);
+                s.fu[r] = v.x;
+                s.fv[r] = v.y;
+            }
+            if constexpr (DELTA) {
+                s.sa[r] = ld1(rs, y * pa + g.xl * 4);
+                const float2 d = ld2(rv, y * pf + g.xl * 8);
+                s.du[r] = d.x;
+                s.dv[r] = d.y;
+            }
+        }
+    }
+    // this lane's column, from the lane's number anew, so that nothing of the
+    // addresses is held through the iterations
+    auto column = [&] {
+        int x;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+        return x + p.x0;
+    };
+    // (null pointers are skipped)
+    auto store = [&](float* of, float* os, float* ov, int image) {
+        const int x = column();
+        const bool ox = x >= p.ox0 && x < p.ox1;
+        const Rsrc rf = image_rsrc(of, pf, tl.H, image), rs = image_rsrc(os, pa, tl.H, image),
+                   rv = image_rsrc(ov, pf, tl.H, image);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int y = g.yw + r;
+            const bool ok = ox && p.out_row(r);
+            if (of) st2(rf, ok ? y * pf + x * 8 : OOB, s.fu[r], s.fv[r]);
+            if constexpr (DELTA) {
+                st1(rs, ok ? y * pa + x * 4 : OOB, s.sa[r]);
+                st2(rv, ok ? y * pf + x * 8 : OOB, s.du[r], s.dv[r]);
+            }
+        }
+    };
+    const bool inner = p.x0 >= lp.border && p.x0 + LANES - 1 < tl.W - lp.border && p.y0 >= lp.border &&
+                       p.y0 + nw * R - 1 < tl.H - lp.border;
+    int slot = 0;
+    // (a loop of its own for each form of the passes, as in k_propagate_tile)
+    auto iterate = [&](auto interior, int count) {
+        constexpr bool INNER = decltype(interior)::value;
+        for (int it = 0; it < count; ++it) {
+            prop_x<DELTA, !INNER, R>(s, g, lp);
+            put_rows<DELTA, R>(s, xch, nw, slot, g.wave, g.lane);
+            __syncthreads();
+            Edge5 ea = own_row<DELTA, R>(s, 0), eb = own_row<DELTA, R>(s, R - 1);
+            if (g.wave > 0) get_row<DELTA>(ea, xrow(xch, nw, slot, g.wave - 1) + 5 * LANES, g.lane);
+            if (g.wave < nw - 1) get_row<DELTA>(eb, xrow(xch, nw, slot, g.wave + 1), g.lane);
+            slot ^= 1;
+            prop_y<DELTA, !INNER, R>(s, g, lp, ea, eb);
+        }
+    };
+    for (int done = 0; PROP && done < n;) {
+        const int count = SAVE ? min(2, n - done) : n;
+        if (inner) iterate(std::true_type{}, count);
+        else iterate(std::false_type{}, count);
+        done += count;
+        if constexpr (SAVE) {
+            if (done < n) store(f.mid_flow, f.mid_scalar, f.mid_vector, (done / 2 - 1) * B + b);
+            else store(DELTA ? nullptr : f.prop_flow, f.prop_scalar, f.prop_vector, b);
+        }
+    }
+    // image model and update
+    {
+        const int x = column(), xl = min(x, tl.W - 1);
+        const bool ox = x >= p.ox0 && x < p.ox1;
+        float im[R + 4];
+        const Rsrc ri = image_rsrc(f.image, pa, tl.H, b);
+#pragma unroll
+        for (int j = 0; j < R + 4; ++j) im[j] = ld1(ri, clampi(g.yw - 2 + j, 0, tl.H - 1) * pa + xl * 4);
+        float aold[R];
+        float2 up[R];
+        int offa[R], offf[R];
+        const Rsrc ra = image_rsrc(f.bright, pa, tl.H, b), ru = image_rsrc(f.upper, Wu * 8, Hu, b);
+        const int xm = DELTA ? f.xmap[xl] * 8 : 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int y = g.yw + r, yl = min(y, tl.H - 1);
+            const bool out = ox && p.out_row(r);
+            offa[r] = out ? y * pa + x * 4 : OOB;
+            offf[r] = out ? y * pf + x * 8 : OOB;
+            aold[r] = DELTA ? 0.f : ld1(ra, yl * pa + xl * 4);
+            up[r] = DELTA ? ld2(ru, f.ymap[yl] * Wu * 8 + xm) : make_float2(0.f, 0.f);
+        }
+        const Rsrc rao = image_rsrc(f.bright_out, pa, tl.H, b), rdf = image_rsrc(f.dflow_out, pf, tl.H, b),
+                   rfu = image_rsrc(f.flow_upd, pf, tl.H, b), rg = image_rsrc(f.grad, pf, tl.H, b);
+        auto gradient = [&](int r, float gx, float gy) {
+            if constexpr (SAVE) st2(rg, offf[r], gx, gy);
+        };
+        if (p.xedge) model_update<DELTA, true, R>(s, im, aold, up, lp, rao, rdf, rfu, offa, offf, gradient);
+        else model_update<DELTA, false, R>(s, im, aold, up, lp, rao, rdf, rfu, offa, offf, gradient);
+    }
+    for (int it = 0; it < K; ++it) {
+        if (p.xinside) copy_last_column<R>(s.fu, s.fv, g.lane, g.xlast);
+        if (p.xedge) smooth_x<true, R>(s.fu, s.fv);
+        else smooth_x<false, R>(s.fu, s.fv);
+        const Edge2 e = exchange_smooth_rows<R>(s.fu, s.fv, xch, nw, slot, g.wave, g.lane);
+        slot ^= 1;
+        if (p.yinside) smooth_y<true, R>(s.fu, s.fv, e, p.rlast);
+        else smooth_y<false, R>(s.fu, s.fv, e, p.rlast);
+    }
+    const int x = column();
+    const bool ox = x >= p.ox0 && x < p.ox1;
+    const Rsrc ro = image_rsrc(f.flow_out, pf, tl.H, b);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        st2(ro, ox && p.out_row(r) ? (g.yw + r) * pf + x * 8 : OOB, s.fu[r], s.fv[r]);
 }
 
 // -------------------------------------------------------------- smoothing
@@ -487,6 +641,53 @@ void launch_propagate_tile(const PropFields& in, const PropFields& mid, int afte
     else
         hipLaunchKernelGGL(k_propagate_tile<false>, grid, blk, exchange_bytes(nw), s, in, mid, out, tl, n, after, dt,
                            border);
+}
+
+// A level's halo, and waves per workgroup: 16, or 8 where the taller tiles
+// would leave CUs without one and the halo is at most half of the shorter
+// buffer.
+namespace {
+int level_halo(int n, int K) { return std::max(n, 2) + 2 * K; }
+int level_waves(int B, int H, int W, int halo) {
+    return 4 * halo <= 8 * kTileRows ? waves_for(B, H, W, halo) : 16;
+}
+}  // namespace
+
+bool level_tile_supported(int H, int W, int n, int K) {
+    return H > 0 && W > 0 && n >= 0 && K >= 0 && fits((long long)W * 8, H) && n < LANES && K < LANES &&
+           2 * level_halo(n, K) < 16 * kTileRows;
+}
+
+void launch_level_tile(const LevelFields& f, int B, int H, int W, int Hu, int Wu, int n, int K, int border, float dt,
+                       float gamma, float maxflow, hipStream_t s) {
+    if (!level_tile_supported(H, W, n, K)) throw logic_error("level: iterations or size of one launch out of range");
+    static const bool once = [] {
+        allow_lds(k_level_tile<true, true, true>);
+        allow_lds(k_level_tile<true, false, true>);
+        allow_lds(k_level_tile<false, true, true>);
+        allow_lds(k_level_tile<false, false, true>);
+        allow_lds(k_level_tile<true, true, false>);
+        allow_lds(k_level_tile<true, false, false>);
+        allow_lds(k_level_tile<false, true, false>);
+        allow_lds(k_level_tile<false, false, false>);
+        return true;
+    }();
+    (void)once;
+    const int halo = level_halo(n, K), nw = level_waves(B, H, W, halo);
+    const Tiling tl = tiling(H, W, halo, nw * kTileRows);
+    const dim3 grid(tl.tiles_x * tl.tiles_y, B), blk(nw * LANES);
+    const LevelParams lp{dt, border, H, gamma, maxflow, (float2*)f.flow_upd};
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, blk, exchange_bytes(nw), s, f, tl, Hu, Wu, n, K, lp);
+    };
+    auto form = [&](auto delta, auto save) {
+        if (n) launch(k_level_tile<decltype(delta)::value, decltype(save)::value, true>);
+        else launch(k_level_tile<decltype(delta)::value, decltype(save)::value, false>);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (f.dflow) f.grad ? form(yes, yes) : form(yes, no);
+    else f.grad ? form(no, yes) : form(no, no);
 }
 
 bool smooth_tile_supported(int in_pitch, int out_pitch, int H, int W) {

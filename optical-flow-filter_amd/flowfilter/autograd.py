@@ -100,6 +100,10 @@ class FilterSpec(object):
                                     dt=float(np.float32(1.0) / np.float32(n)), K=int(smooth[l])))
             if l < self.L - 1:
                 ml = np.float32(ml / np.float32(2.0))
+        # whether every level of a frame runs in one launch (image size and
+        # iterations)
+        self.tiled = all(N.get_int("ff_ad_level_supported", lv["H"], lv["W"], lv["N"], lv["K"])
+                         for lv in self.levels)
         self.device = torch.device(device)
         for l in range(self.L - 1):
             h, w = self.sizes[l]
@@ -147,6 +151,133 @@ def _effective_gammas(gamma):
 
 # ------------------------------------------------------------ one frame
 
+def _propagate(fields, iterations, dt, border, B, h, w, save, s):
+    """`iterations` propagation iterations of the flow and its payloads (or
+    None, None). Returns the propagated fields, and with `save` what the
+    adjoints start from: for every two iterations (and a last single one)
+    their number and input."""
+    passes = []
+    f, sc, vc = fields
+    pay = sc is not None
+    new = lambda: (_empty(B, h, w, 2, like=f), _empty(B, h, w, like=f) if pay else None,
+                   _empty(B, h, w, 2, like=f) if pay else None)
+    it = 0
+    while it < iterations:
+        # up to four iterations per launch; the adjoints recompute the passes
+        # inside each two
+        n = min(_STEPS if _tiled(h, w) else 2, iterations - it)
+        kept = [(min(2, n), f, sc, vc)]
+        out = new()
+        if _tiled(h, w):
+            mid = new() if save and n > 2 else (None, None, None)
+            N.call("ff_ad_propagate_steps", _p(f), _p(sc), _p(vc), n, 2, _p(mid[0]), _p(mid[1]), _p(mid[2]),
+                   _p(out[0]), _p(out[1]), _p(out[2]), B, h, w, ctypes.c_float(dt), border, s)
+            if n > 2:
+                kept.append((n - 2,) + mid)
+        elif n == 2:
+            N.call("ff_ad_propagate_quad", _p(f), _p(sc), _p(vc), _p(out[0]), _p(out[1]), _p(out[2]), B, h, w,
+                   ctypes.c_float(dt), border, s)
+        else:
+            N.call("ff_ad_propagate_pair", _p(f), _p(sc), _p(vc), None, None, None, _p(out[0]), _p(out[1]),
+                   _p(out[2]), B, h, w, ctypes.c_float(dt), border, s)
+        if save:
+            passes.extend(kept)
+        it += n
+        f, sc, vc = out
+    return (f, sc, vc), passes
+
+
+def _last_iterations(pixels, n, save):
+    """Propagation iterations of a level that run in the launch of its image
+    model, update and smoothing; those before run in launches of their own.
+
+    Iterations widen the halo of the tiles (2 + 2 K without any), which the
+    smoothing's passes then cover too, but save a pass over the fields. Of 8
+    at 3840x2160, one smoothing iteration: all in the launch 338 us, 4 of them
+    116 + 193, none 2 x 116 + 95, 2 of them 361; of 4 at 16 x 512x512: all 101,
+    none 70 + 47. With what the adjoints read written as well, none is best
+    (2 x 140 + 117 us, and 4 of 8 in the launch 140 + 340), except on images so
+    small that a launch costs more than its work."""
+    if pixels < 1 << 18:
+        return n
+    if save:
+        return 0
+    return n if n <= 6 else 4
+
+
+class _Level(ctypes.Structure):  # ff_ad_level
+    _fields_ = [(n, ctypes.c_void_p) for n in
+                ("image", "flow", "bright", "dflow", "upper", "xmap", "ymap", "flow_out", "bright_out", "dflow_out",
+                 "flow_upd", "grad", "prop_flow", "prop_scalar", "prop_vector", "mid_flow", "mid_scalar",
+                 "mid_vector")]
+
+
+def _level_forward(spec, l, image, state, upper, gamma, save, want_upd, s):
+    """One level of a frame after the first: the propagation's first
+    iterations in launches of their own, the rest of them and all that follows
+    in one. Returns the new state, the unsmoothed flow (top level, want_upd),
+    and with `save` the image gradient, the propagated fields and the
+    propagation's inputs as _frame_forward keeps them."""
+    B, h, w = image.shape
+    lv = spec.levels[l]
+    delta = l < spec.L - 1
+    new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=image.device)
+    vec, sca = (lambda: new(B, h, w, 2)), (lambda: new(B, h, w))
+    ptrs = lambda ts: [t.data_ptr() if t is not None else None for t in ts]
+    n = _last_iterations(B * h * w, lv["N"], save)
+    fields = (state["f"], state["a0"] if delta else None, state["d"] if delta else None)
+    passes = []
+    if n < lv["N"]:
+        fields, passes = _propagate(fields, lv["N"] - n, lv["dt"], spec.border, B, h, w, save, s)
+    st = dict(f=vec(), a0=sca())
+    a = _Level(image.data_ptr(), *ptrs((fields[0], fields[1] if delta else state["a0"], fields[2])))
+    a.flow_out, a.bright_out = st["f"].data_ptr(), st["a0"].data_ptr()
+    hu = wu = 0
+    upd = grad = None
+    if delta:
+        hu, wu = spec.sizes[l + 1]
+        st["d"] = vec()
+        a.dflow_out = st["d"].data_ptr()
+        a.upper, a.xmap, a.ymap = upper.data_ptr(), lv["xmap"].data_ptr(), lv["ymap"].data_ptr()
+    elif want_upd:
+        upd = vec()
+        a.flow_upd = upd.data_ptr()
+    if save:
+        grad = vec()
+        a.grad = grad.data_ptr()
+        if n:
+            mids = (n + 1) // 2 - 1
+            mid = (new(mids, B, h, w, 2), new(mids, B, h, w) if delta else None,
+                   new(mids, B, h, w, 2) if delta else None)
+            if mids:
+                a.mid_flow, a.mid_scalar, a.mid_vector = ptrs(mid)
+            passes.append((min(2, n),) + fields)
+            for k in range(mids):
+                passes.append((min(2, n - 2 * (k + 1)),) + tuple(t[k] if t is not None else None for t in mid))
+            fields = (None, sca(), vec()) if delta else (vec(), None, None)
+            a.prop_flow, a.prop_scalar, a.prop_vector = ptrs(fields)
+    N.call("ff_ad_level_forward", ctypes.byref(a), n, lv["K"], B, h, w, hu, wu, lv["dt"], spec.border, gamma,
+           lv["maxflow"], s)
+    return st, upd, grad, fields, passes
+
+
+def _frame_levels(spec, state, imgs, gammas, save):
+    """_frame_forward after the pyramid, for a frame after the first whose
+    levels each run in one launch."""
+    top = spec.L - 1
+    s = _stream()
+    out = [None] * spec.L
+    out[top] = _level_forward(spec, top, imgs[top], state[top], None, gammas[top], save, top > 0, s)
+    uppers = [None] * spec.L
+    for l in range(top):  # (the order of reads: as below)
+        uppers[l] = out[top][1] if l == top - 1 else state[l + 1]["f"]
+        out[l] = _level_forward(spec, l, imgs[l], state[l], uppers[l], gammas[l], save, False, s)
+    new_state, _, g, prop, passes = (list(x) for x in zip(*out))
+    saved = dict(first=False, a0=[st["a0"] for st in new_state], g=g, passes=passes, prop=prop, upper=uppers,
+                 state=state) if save else None
+    return new_state, new_state[0]["f"], saved
+
+
 def _frame_forward(spec, state, image, gammas, save):
     """One frame for all levels. state: per level dict(f, a0[, d]) or None
     for the first frame. Returns (new_state, output_flow, saved)."""
@@ -160,6 +291,8 @@ def _frame_forward(spec, state, image, gammas, save):
         work = _empty(B, h, w // 2, like=image)
         N.call("ff_ad_down", _p(imgs[-1]), _p(out), _p(work), B, h, w, s)
         imgs.append(out)
+    if state is not None and spec.tiled:
+        return _frame_levels(spec, state, imgs, gammas, save)
     a0, g = [], []
     for l in range(L):
         h, w = spec.sizes[l]
@@ -186,35 +319,7 @@ def _frame_forward(spec, state, image, gammas, save):
         f = state[l]["f"]
         sc = state[l]["a0"] if l < top else None
         vc = state[l]["d"] if l < top else None
-        passes = []
-        pay = sc is not None
-        it = 0
-        while it < lv["N"]:
-            fields = lambda: (_empty(B, h, w, 2, like=image), _empty(B, h, w, like=image) if pay else None,
-                              _empty(B, h, w, 2, like=image) if pay else None)
-            # up to four iterations per launch; what is kept is the input of
-            # every two (and of a last single one): the adjoints recompute
-            # the passes inside
-            n = min(_STEPS if _tiled(h, w) else 2, lv["N"] - it)
-            kept = [(min(2, n), f, sc, vc)]
-            out = fields()
-            if _tiled(h, w):
-                mid = fields() if save and n > 2 else (None, None, None)
-                N.call("ff_ad_propagate_steps", _p(f), _p(sc), _p(vc), n, 2, _p(mid[0]), _p(mid[1]), _p(mid[2]),
-                       _p(out[0]), _p(out[1]), _p(out[2]), B, h, w, ctypes.c_float(lv["dt"]), spec.border, s)
-                if n > 2:
-                    kept.append((n - 2,) + mid)
-            elif n == 2:
-                N.call("ff_ad_propagate_quad", _p(f), _p(sc), _p(vc), _p(out[0]), _p(out[1]), _p(out[2]), B, h, w,
-                       ctypes.c_float(lv["dt"]), spec.border, s)
-            else:
-                N.call("ff_ad_propagate_pair", _p(f), _p(sc), _p(vc), None, None, None, _p(out[0]), _p(out[1]),
-                       _p(out[2]), B, h, w, ctypes.c_float(lv["dt"]), spec.border, s)
-            if save:
-                passes.extend(kept)
-            it += n
-            f, sc, vc = out
-        prop[l] = (f, sc, vc)
+        prop[l], passes = _propagate((f, sc, vc), lv["N"], lv["dt"], spec.border, B, h, w, save, s)
         if save:
             saved["passes"][l] = passes
             saved["prop"][l] = prop[l]
@@ -244,8 +349,6 @@ def _frame_forward(spec, state, image, gammas, save):
         new_state[l] = dict(f=_smooth(fl, lv["K"], B, h, w, s), a0=a0[l], d=dn)
         if save:
             saved["upper"][l] = upper
-    if save:
-        saved["upd"] = upd
     return new_state, new_state[0]["f"], saved
 
 

@@ -207,3 +207,96 @@ def test_ad_two_iterations_adjoint(B, h, w, border, pay, special):
         if a is not None:
             assert torch.equal(torch.isnan(a), torch.isnan(b))
             assert torch.equal(torch.nan_to_num(a, nan=0.0), torch.nan_to_num(b, nan=0.0))
+
+
+@pytest.mark.parametrize("B,h,w", [(1, 2, 3), (2, 31, 63), (1, 33, 65), (3, 64, 57), (2, 130, 200), (1, 420, 700)])
+@pytest.mark.parametrize("n,K", [(0, 1), (1, 0), (2, 1), (3, 2), (4, 1), (7, 1), (9, 3)])
+@pytest.mark.parametrize("delta", [False, True])
+def test_ad_level_matches_stages(B, h, w, n, K, delta):
+    """A level in one launch is bitwise its stages' own launches: the new state,
+    the unsmoothed flow, and what is kept for the adjoints; an infinite and a
+    NaN brightness included."""
+    import ctypes
+
+    import torch
+    from flowfilter import _native as N
+    from flowfilter.autograd import FilterSpec, _Level, _propagate
+    print("ad level", (B, h, w), n, K, delta, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(h + 3 * w + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    f32 = ctypes.c_float
+    dt, border, gamma, maxflow = 1.0 / max(n, 1), 1 + n % 3, 3e-4, 2.5
+    hu, wu = max(h // 2, 1), max(w // 2, 1)
+    image, flow, bright = rnd(B, h, w).abs(), rnd(B, h, w, 2), rnd(B, h, w).abs()
+    bright[0, h // 2, w // 3], bright[-1, h // 3, w // 2] = float("inf"), float("nan")
+    dflow, upper = (rnd(B, h, w, 2), rnd(B, hu, wu, 2)) if delta else (None, None)
+    maps = FilterSpec(max(h, 2), max(w, 2), 2).levels[0]
+    # the stages
+    a0, gr = torch.empty_like(image), torch.empty_like(flow)
+    N.call("ff_ad_image_model", p(image), p(a0), p(gr), B, h, w, s)
+    fields = (flow, bright if delta else None, dflow)
+    prop, passes = _propagate(fields, n, dt, border, B, h, w, True, s)
+    upd, dn = torch.empty_like(flow), torch.empty_like(flow)
+    if delta:
+        N.call("ff_ad_delta_update", p(a0), p(gr), p(prop[1]), p(prop[2]), p(upper), p(maps["xmap"]), p(maps["ymap"]),
+               p(dn), p(upd), B, h, w, hu, wu, f32(gamma), f32(maxflow), s)
+    else:
+        N.call("ff_ad_update", p(a0), p(gr), p(bright), p(prop[0]), p(upd), B, h, w, f32(gamma), f32(maxflow), s)
+    sm = upd
+    for _ in range(K):
+        o = torch.empty_like(sm)
+        N.call("ff_ad_smooth_pair", p(sm), p(o), B, h, w, s)
+        sm = o
+    same = lambda a, b: torch.equal(torch.nan_to_num(a, 7e7), torch.nan_to_num(b, 7e7))
+    for save in (False, True):
+        new = lambda *shape: torch.full(shape, -5.0, device="cuda")
+        mids = max((n + 1) // 2 - 1, 0)
+        got = dict(flow_out=new(B, h, w, 2), bright_out=new(B, h, w))
+        ref = dict(flow_out=sm, bright_out=a0)
+        if delta:
+            got["dflow_out"], ref["dflow_out"] = new(B, h, w, 2), dn
+        else:
+            got["flow_upd"], ref["flow_upd"] = new(B, h, w, 2), upd
+        if save:
+            got["grad"], ref["grad"] = new(B, h, w, 2), gr
+            names = ("flow", "scalar", "vector") if delta else ("flow",)
+            for k, name in enumerate(names):
+                if n and (not delta or k):
+                    got["prop_" + name], ref["prop_" + name] = torch.full_like(prop[k], -5.0), prop[k]
+                if mids:
+                    ref["mid_" + name] = torch.stack([q[1 + k] for q in passes[1:]])
+                    got["mid_" + name] = torch.full_like(ref["mid_" + name], -5.0)
+        a = _Level(image=image.data_ptr(), flow=flow.data_ptr(), bright=bright.data_ptr())
+        if delta:
+            a.dflow, a.upper = dflow.data_ptr(), upper.data_ptr()
+            a.xmap, a.ymap = maps["xmap"].data_ptr(), maps["ymap"].data_ptr()
+        for name, t in got.items():
+            setattr(a, name, t.data_ptr())
+        N.call("ff_ad_level_forward", ctypes.byref(a), n, K, B, h, w, hu, wu, f32(dt), border, f32(gamma),
+               f32(maxflow), s)
+        for name in got:
+            assert same(ref[name], got[name]), (save, name)
+
+
+def test_ad_level_refusals():
+    """Sizes and iterations that no tile has room for, and outputs that are
+    inputs, are errors, not launches."""
+    import ctypes
+
+    import torch
+    from flowfilter import _native as N
+    from flowfilter.autograd import _Level
+    ok = lambda *a: N.get_int("ff_ad_level_supported", *a)
+    assert ok(64, 64, 8, 2) and ok(64, 64, 0, 0) and ok(64, 64, 29, 1) and ok(64, 64, 2, 14)
+    assert not ok(64, 64, 30, 1) and not ok(64, 64, 2, 15) and not ok(20000, 20000, 4, 1) and not ok(64, 64, -1, 1)
+    assert not ok(64, 64, 1, 2 ** 30) and not ok(0, 64, 1, 1)
+    t = torch.zeros(1, 8, 8, 2, device="cuda")
+    a = _Level(*[t.data_ptr()] * 3)
+    a.flow_out, a.bright_out = t.data_ptr(), t.data_ptr()
+    call = lambda n: N.call("ff_ad_level_forward", ctypes.byref(a), n, 1, 1, 8, 8, 0, 0, ctypes.c_float(1), 1,
+                            ctypes.c_float(1), ctypes.c_float(1), None)
+    for n in (1, 30):
+        with pytest.raises(Exception):
+            call(n)
