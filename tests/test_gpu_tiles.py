@@ -300,3 +300,43 @@ def test_ad_level_refusals():
     for n in (1, 30):
         with pytest.raises(Exception):
             call(n)
+
+
+@pytest.mark.parametrize("B,T,h,w", [(1, 2, 1, 1), (2, 3, 3, 2), (1, 4, 5, 63), (2, 2, 16, 64), (1, 3, 17, 65), (1, 2, 90, 200)])
+@pytest.mark.parametrize("kind", ["zero", "smooth", "rough"])
+def test_photometric_adjoint(B, T, h, w, kind):
+    """The photometric term's gradients against the float64 composition's (on
+    the CPU): fields whose shares of a sampled pixel all meet, mostly meet, or
+    rarely do. A frame pixel's gradient is a sum over the pixels that sample it,
+    each share a float32 product within 4e-7 of itself times the terms'
+    magnitude (coordinates of up to 200 px carry 1e-5 px of float32 rounding,
+    and the differences up to 1): 2e-5 of the largest gradient of its kind, and
+    for the flow 1e-3 more where a coordinate is that close to a pixel's edge,
+    which only the random fields' 1 in 1e4 pixels are; none of the flows here
+    samples a pixel's edge exactly but `zero`, whose coordinates are integers
+    (left out for the flow: the derivative there is one-sided)."""
+    import torch
+    from flowfilter.autograd import photometric_error
+    print("photometric adjoint", (B, T, h, w), kind, flush=True)
+    g = torch.Generator().manual_seed(h * 100 + w)
+    frames = torch.rand(B, T, h, w, generator=g)
+    y, x = torch.meshgrid(torch.arange(h), torch.arange(w), indexing="ij")
+    if kind == "zero":
+        flows = torch.zeros(B, T, h, w, 2)
+    elif kind == "smooth":
+        flows = torch.stack([0.3 + 0.5 * torch.sin(x / 40.0), -0.4 + 0.5 * torch.cos(y / 30.0)], -1).expand(
+            B, T, h, w, 2).contiguous()
+    else:
+        flows = torch.randn(B, T, h, w, 2, generator=g) * 3.0
+    out = []
+    for dev, dt in (("cpu", torch.float64), ("cuda", torch.float32)):
+        fr = frames.to(dev, dt).requires_grad_()
+        fl = flows.to(dev, dt).requires_grad_()
+        photometric_error(fr, fl).backward()
+        out.append((fr.grad.cpu().double(), fl.grad.cpu().double()))
+    (a, b), (c, d) = out
+    assert float((a - c).abs().max()) <= 2e-5 * max(float(a.abs().max()), 1.0 / (B * T * h * w))
+    if kind != "zero":
+        near = (flows.double() - flows.double().round()).abs().amin(-1, keepdim=True) < 1e-4
+        bad = ((b - d).abs() > 1e-3 * float(b.abs().max()) + 1e-12) & ~near
+        assert not bool(bad.any())
