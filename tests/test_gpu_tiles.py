@@ -340,3 +340,41 @@ def test_photometric_adjoint(B, T, h, w, kind):
         near = (flows.double() - flows.double().round()).abs().amin(-1, keepdim=True) < 1e-4
         bad = ((b - d).abs() > 1e-3 * float(b.abs().max()) + 1e-12) & ~near
         assert not bool(bad.any())
+
+
+@pytest.mark.parametrize("B,h,w", [(1, 2, 2), (2, 3, 5), (1, 9, 130), (3, 16, 63), (2, 67, 129)])
+@pytest.mark.parametrize("inplace", [False, True])
+def test_float_pyramid_step(ffo, B, h, w, inplace):
+    """The reduction is bitwise the oracle's, and its adjoint, added to what is
+    there, its transpose: <g, D x> = <D^T g, x> in float64 sums to 1e-6 of the
+    terms' magnitude (weights that are powers of two; a rounding per sum). Also
+    with the result in the input's place, and the adjoint's in its input's."""
+    import ctypes
+
+    import torch
+    from flowfilter import _native as N
+    print("pyramid step", (B, h, w), inplace, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(h * w)
+    rnd = lambda *s: torch.rand(*s, generator=g, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    img, work = rnd(B, h, w), torch.empty(B, h, w // 2, device="cuda")
+    hh, hw = h // 2, w // 2
+    n = B * hh * hw
+    buf = img.clone()
+    half = buf.view(-1)[:n] if inplace else torch.empty(n, device="cuda")
+    N.call("ff_ad_down", p(buf), p(half), p(work), B, h, w, s)
+    half = half.view(B, hh, hw).clone()
+    for b in range(B):
+        assert np.array_equal(half[b].cpu().numpy(), ffo.pyramid(img[b].cpu().numpy(), 2)[1])
+    gh, base = rnd(B, hh, hw) - 0.5, rnd(B, h, w)
+    out = base.clone()
+    src = gh.contiguous()
+    if inplace:
+        out.view(-1)[:n] = gh.view(-1)
+        base = out.clone()
+        src = out.view(-1)[:n]
+    N.call("ff_ad_down_backward", p(src), p(out), p(work), B, h, w, 1, s)
+    left = (gh.double() * half.double()).sum()
+    right = ((out.double() - base.double()) * img.double()).sum()
+    assert abs(float(left - right)) <= 1e-6 * float((gh.abs().double() * half.double()).sum() + base.sum().double())
