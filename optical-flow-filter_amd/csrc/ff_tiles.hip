@@ -205,9 +205,9 @@ struct LevelParams {
 // the buffer's edge.
 //
 // What bounds it: without PROP, HBM and the latency of its four phases (3840x2160
-// delta level, K = 1: 95 us for 316 MB, with the gradient 117 us for 382 MB; the
+// delta level, K = 2: 95 us for 316 MB, with the gradient 117 us for 382 MB; the
 // launches it replaces, image model, update and smoothing, took 149 us). With
-// PROP, the VALU: n = 4 193 us, n = 8 338 us, the halo being 6 and 10 of 64
+// PROP, the VALU: n = 4 193 us, n = 8 338 us, the halo being 8 and 12 of 64
 // columns. 16 x 512x512, n = 4: 101 us (161 in four launches).
 template <bool DELTA, bool SAVE, bool PROP>
 __global__ void __launch_bounds__(1024, 8) k_level_tile(LevelFields f, Tiling tl, int Hu, int Wu, int n, int K,

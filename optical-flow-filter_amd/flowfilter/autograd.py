@@ -100,10 +100,6 @@ class FilterSpec(object):
                                     dt=float(np.float32(1.0) / np.float32(n)), K=int(smooth[l])))
             if l < self.L - 1:
                 ml = np.float32(ml / np.float32(2.0))
-        # whether every level of a frame runs in one launch (image size and
-        # iterations)
-        self.tiled = all(N.get_int("ff_ad_level_supported", lv["H"], lv["W"], lv["N"], lv["K"])
-                         for lv in self.levels)
         self.device = torch.device(device)
         for l in range(self.L - 1):
             h, w = self.sizes[l]
@@ -114,6 +110,12 @@ class FilterSpec(object):
             lv = self.levels[l]
             for k, v in (("xmap", xm), ("ymap", ym), ("xlo", xlo), ("xhi", xhi), ("ylo", ylo), ("yhi", yhi)):
                 lv[k] = torch.from_numpy(v).to(self.device)
+
+    @property
+    def tiled(self):
+        """Whether each level of a frame can run in one launch: image size and
+        iterations (also of a spec that was copied, loaded or changed)."""
+        return all(N.get_int("ff_ad_level_supported", lv["H"], lv["W"], lv["N"], lv["K"]) for lv in self.levels)
 
 
 # Iterations that one launch of the tile kernels takes, and whether they
@@ -193,7 +195,7 @@ def _last_iterations(pixels, n, save):
 
     Iterations widen the halo of the tiles (2 + 2 K without any), which the
     smoothing's passes then cover too, but save a pass over the fields. Of 8
-    at 3840x2160, one smoothing iteration: all in the launch 338 us, 4 of them
+    at 3840x2160, two smoothing iterations: all in the launch 338 us, 4 of them
     116 + 193, none 2 x 116 + 95, 2 of them 361; of 4 at 16 x 512x512: all 101,
     none 70 + 47. With what the adjoints read written as well, none is best
     (2 x 140 + 117 us, and 4 of 8 in the launch 140 + 340), except on images so
