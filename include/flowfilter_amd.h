@@ -405,6 +405,11 @@ FF_API ff_status ff_filter_get_wait_timeouts(ff_stage* s, unsigned long long* ou
  * counts a timeout (every kernel still ends; the flow of those frames is
  * not valid); 0 restores the normal waits. For tests of the error path. */
 FF_API ff_status ff_filter_set_wait_test(ff_stage* s, int spins);
+/* Test hook (no reference counterpart): fused launches of different streams
+ * are ordered by a count of the tiles that have started. After waiting for the
+ * device: how many its launches should have started, and have (the same,
+ * modulo 2^32). */
+FF_API ff_status ff_wait_order_state(unsigned* expected, unsigned* started);
 
 /* Tile height of the fused frame kernel, in waves per workgroup (no
  * reference counterpart): 0 (the default) times the candidates 16, 15, 8, 5

@@ -682,6 +682,13 @@ ff_status ff_filter_get_wait_timeouts(ff_stage* s, unsigned long long* out) {
     });
 }
 
+ff_status ff_wait_order_state(unsigned* expected, unsigned* started) {
+    return guard([&] {
+        out_ptr(expected, "expected"), out_ptr(started, "started");
+        wait_order_state(expected, started);
+    });
+}
+
 ff_status ff_filter_set_wait_test(ff_stage* s, int spins) {
     return guard_on(s, [&] {
         if (!s || !s->obj) throw null_handle("ff_stage");

@@ -571,7 +571,7 @@ namespace {
 // was launched.
 template <class F>
 bool run_maybe_graphed(bool graphs_on, GraphCache& cache, const std::vector<LevelArgs>& args,
-                       unsigned long long token, hipStream_t s, F work) {
+                       unsigned long long token, hipStream_t s, const WaitingLaunch& order, F work) {
     if (!graphs_on || profiling_active()) {
         work();
         return false;
@@ -594,6 +594,7 @@ bool run_maybe_graphed(bool graphs_on, GraphCache& cache, const std::vector<Leve
         cache.insert(args, token, exec);
     }
     FF_HIP(hipGraphLaunch(exec, s));
+    order.launched();
     return true;
 }
 }  // namespace
@@ -608,7 +609,7 @@ void PyramidalFlowFilter::computeFused(const std::vector<LevelArgs>& args, const
     const WaitingLaunch order(s, frame_.awaited(table));
     // a frame in place is a launch argument, which a replayed graph would
     // not update: such frames are launched directly
-    if (run_maybe_graphed(graphs_on_ && levels_ > 3 && !frame, graphs_, args, frame_.token(table), s,
+    if (run_maybe_graphed(graphs_on_ && levels_ > 3 && !frame, graphs_, args, frame_.token(table), s, order,
                           [&] { enqueueFused(table, s, frame ? &fr : nullptr); }))
         frame_.replayed();
     commitFused();
@@ -847,7 +848,7 @@ void BatchedFlowFilter::compute() {
         // the step is replayed as a HIP graph when graphs are on (the
         // default) and no frame is read in place (a launch argument, which
         // a replay would not update)
-        if (run_maybe_graphed(graphs_on_ && frames.empty(), graphs_, all, frame_.token(table), s, [&] {
+        if (run_maybe_graphed(graphs_on_ && frames.empty(), graphs_, all, frame_.token(table), s, order, [&] {
                 for (PyramidalFlowFilter* f : fused) f->enqueuePreFused();
                 frame_.launch(table, s, frames.data(), (int)frames.size());
                 check_launch("BatchedFlowFilter::compute (fused frame)");

@@ -981,16 +981,15 @@ void FusedFrame::Impl::run(int ti, hipStream_t s, const FrameRef* frames, int nf
     const char* base = (const char*)t.dev.data();
     const TileFlags fl{region(si), timeout_word(), order.started(), e};
     const LaunchArgs args{(const LevelJob*)base, (const int*)(base + t.map_offset), fl, t.ends, t.nw, wa, fa};
-    const dim3 grid(t.blocks), blk(t.nw * LANES);
-    const size_t lds = lds_bytes(t.nw);
-    if (t.rlow == 4 && t.inner)
-        hipLaunchKernelGGL((k_fused_frame<4, 4, true>), grid, blk, lds, s, args);
-    else if (t.rlow == 4)
-        hipLaunchKernelGGL((k_fused_frame<4, 4>), grid, blk, lds, s, args);
-    else if (t.rtop == 8)
-        hipLaunchKernelGGL(k_fused_frame<8>, grid, blk, lds, s, args);
-    else
-        hipLaunchKernelGGL(k_fused_frame<4>, grid, blk, lds, s, args);
+    const void* kernel = t.rlow == 4 ? (t.inner ? (const void*)k_fused_frame<4, 4, true> : (const void*)k_fused_frame<4, 4>)
+                                     : (t.rtop == 8 ? (const void*)k_fused_frame<8> : (const void*)k_fused_frame<4>);
+    void* argv[] = {(void*)&args};
+    const hipError_t err = hipLaunchKernel(kernel, dim3(t.blocks), dim3(t.nw * LANES), argv, lds_bytes(t.nw), s);
+    if (err != hipSuccess) {
+        (void)hipGetLastError();  // reported here
+        throw_hip(err, "the fused frame's launch", __FILE__, __LINE__);
+    }
+    if (cs == hipStreamCaptureStatusNone) order.launched();
 }
 
 // Time the launches of every candidate tiling (waves per workgroup and, when

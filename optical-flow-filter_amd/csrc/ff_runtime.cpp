@@ -2,6 +2,7 @@
 #include "ff_runtime.hpp"
 
 #include "ff_kernels.hpp"
+#include "ff_launch_order.hpp"
 
 #include <sched.h>
 #include <unistd.h>
@@ -9,7 +10,6 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstring>
-#include <exception>
 #include <mutex>
 #include <set>
 #include <sstream>
@@ -439,14 +439,11 @@ void Image::swapBuffers(Image& o) {
 // ------------------------------------------------------------ WaitingLaunch
 
 namespace {
-// Per device: the word that counts the awaited tiles as they start, what it
-// will have counted when the launches enqueued so far have started all
-// theirs (modulo 2^32), and the stream of the last of them.
+// Per device: the order of the launches, and the word that counts their
+// awaited tiles as they start.
 struct WaitingState {
+    LaunchOrder order;
     unsigned* word = nullptr;
-    unsigned target = 0;
-    hipStream_t last = nullptr;  // the null stream is a stream too
-    bool pending = false;        // the last launch may not have started
 };
 // Kept for the process (never destroyed), like the library stream: boxes
 // may be destroyed during the process's exit.
@@ -459,8 +456,7 @@ Waiting& waiting() {
     static Waiting* w = new Waiting;
     return *w;
 }
-thread_local int t_waiting_depth = 0;
-thread_local unsigned* t_waiting_started = nullptr;  // of the outermost guard
+thread_local const WaitingLaunch* t_outermost = nullptr;  // of the guards alive on this thread
 
 void owned_insert(hipStream_t s) {
     Waiting& g = waiting();
@@ -471,8 +467,7 @@ void owned_erase(hipStream_t s) {
     Waiting& g = waiting();
     std::lock_guard<std::mutex> lk(g.mu);
     g.owned.erase(s);
-    for (WaitingState& w : g.dev)
-        if (w.last == s) w.pending = false;
+    for (WaitingState& w : g.dev) w.order.finished(s);
 }
 
 bool capturing(hipStream_t s) {
@@ -482,14 +477,11 @@ bool capturing(hipStream_t s) {
 }
 }  // namespace
 
-WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) {
+WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) : s_(s), awaited_(awaited) {
     if (awaited <= 0) return;
-    // counted (and so undone by the destructor) only once nothing can throw
-    if (t_waiting_depth > 0 || capturing(s)) {
-        started_ = t_waiting_depth > 0 ? t_waiting_started : nullptr;
-        if (t_waiting_depth == 0) t_waiting_started = nullptr;
-        ++t_waiting_depth;
-        counted_ = true;
+    if (t_outermost || capturing(s)) {
+        if (!t_outermost) t_outermost = this;
+        outer_ = t_outermost;
         return;
     }
     FF_HIP(hipGetDevice(&dev_));
@@ -504,31 +496,38 @@ WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) {
         FF_HIP(hipMemcpy(p, &zero, sizeof(zero), hipMemcpyHostToDevice));
         w.word = p;
     }
+    const auto last = (hipStream_t)w.order.last;
     // (a stream of the caller's may have been destroyed: it is not asked)
-    if (w.pending && w.last != s && !(g.owned.count(w.last) && !capturing(w.last) && hipStreamQuery(w.last) == hipSuccess)) {
-        launch_wait_started(w.word, w.target, s);
+    if (w.order.follows(s) && !(g.owned.count(last) && !capturing(last) && hipStreamQuery(last) == hipSuccess)) {
+        launch_wait_started(w.word, w.order.target, s);
         check_launch("WaitingLaunch");
     }
-    awaited_ = awaited;
-    exceptions_ = std::uncaught_exceptions();
-    w.target += (unsigned)awaited;
-    w.last = s;
-    w.pending = true;
     lk.release();  // held until the destructor
-    started_ = t_waiting_started = w.word;
-    ++t_waiting_depth;
-    counted_ = true;
+    word_ = w.word;
     locked_ = true;
+    t_outermost = outer_ = this;
+}
+
+void WaitingLaunch::launched() const {
+    if (outer_ && outer_->locked_) waiting().dev[outer_->dev_].order.launched(outer_->s_, awaited_);
 }
 
 WaitingLaunch::~WaitingLaunch() {
-    if (!counted_) return;
-    --t_waiting_depth;
-    if (!locked_) return;
+    if (outer_ == this) t_outermost = nullptr;
+    if (locked_) waiting().mu.unlock();
+}
+
+bool wait_order_state(unsigned* expected, unsigned* started) {
+    int dev = 0;
+    FF_HIP(hipGetDevice(&dev));
+    FF_HIP(hipDeviceSynchronize());
     Waiting& g = waiting();
-    // a launch that failed counts nothing
-    if (std::uncaught_exceptions() > exceptions_) g.dev[dev_].target -= (unsigned)awaited_;
-    g.mu.unlock();
+    std::lock_guard<std::mutex> lk(g.mu);
+    *expected = *started = 0;
+    if ((int)g.dev.size() <= dev || !g.dev[dev].word) return false;
+    *expected = g.dev[dev].order.target;
+    FF_HIP(hipMemcpy(started, g.dev[dev].word, sizeof(unsigned), hipMemcpyDeviceToHost));
+    return true;
 }
 
 // ------------------------------------------------------------- InputFrames

@@ -219,9 +219,10 @@ private:
 // took 81 us per 2048x1088 two-level frame, for a launch of 55 us.)
 //
 // Constructed under a process-wide lock that is held until destruction, so
-// that launches are numbered in the order in which they are enqueued. Nested
-// guards on one thread count once; a launch into a caller's own stream
-// capture is neither counted nor ordered, since its replays are not seen.
+// that launches are numbered in the order in which they are enqueued, and
+// counted when they have been (launched()). A guard inside another on the same
+// thread belongs to it; a launch into a caller's own stream capture is neither
+// counted nor ordered, since its replays are not seen.
 class WaitingLaunch {
 public:
     WaitingLaunch(hipStream_t s, int awaited);
@@ -229,13 +230,24 @@ public:
     WaitingLaunch(const WaitingLaunch&) = delete;
     WaitingLaunch& operator=(const WaitingLaunch&) = delete;
     // Where the launch's awaited tiles count themselves (null: nowhere).
-    unsigned* started() const { return started_; }
+    unsigned* started() const { return outer_ ? outer_->word_ : nullptr; }
+    // The launch was enqueued, by its own status (an earlier call's error says
+    // nothing about it): once for every kernel or graph launch, not for one
+    // that is being captured.
+    void launched() const;
 
 private:
-    bool counted_ = false, locked_ = false;
-    int dev_ = 0, awaited_ = 0, exceptions_ = 0;
-    unsigned* started_ = nullptr;
+    hipStream_t s_ = nullptr;
+    int awaited_ = 0, dev_ = 0;
+    const WaitingLaunch* outer_ = nullptr;  // this one, or the one it is nested in
+    unsigned* word_ = nullptr;
+    bool locked_ = false;
 };
+
+// Test hook: the awaited tiles that the current device's launches should have
+// started, and that have, after waiting for the device. Returns false (zeros)
+// before the first such launch.
+bool wait_order_state(unsigned* expected, unsigned* started);
 
 // Host frames for a filter's own input image, double buffered: load()
 // copies a host frame into a pinned host buffer (on a few threads), then
