@@ -611,7 +611,7 @@ void PyramidalFlowFilter::computeFused(const std::vector<LevelArgs>& args, const
     // not update: such frames are launched directly
     if (run_maybe_graphed(graphs_on_ && levels_ > 3 && !frame, graphs_, args, frame_.token(table), s, order,
                           [&] { enqueueFused(table, s, frame ? &fr : nullptr); }))
-        frame_.replayed();
+        frame_.replayed(table, s);
     commitFused();
 }
 
@@ -853,7 +853,7 @@ void BatchedFlowFilter::compute() {
                 frame_.launch(table, s, frames.data(), (int)frames.size());
                 check_launch("BatchedFlowFilter::compute (fused frame)");
             }))
-            frame_.replayed();
+            frame_.replayed(table, s);
         for (PyramidalFlowFilter* f : fused) {
             f->commitFused();
             f->waitBatch_.follow(frame_.watch());

@@ -1095,7 +1095,12 @@ void FusedFrame::launch(int table, hipStream_t s, const FrameRef* frames, int nf
     impl_->run(table, s, frames, nframes);
 }
 
-void FusedFrame::replayed() { impl_->counted[0] = impl_->counted[1] = 0; }
+void FusedFrame::replayed(int table, hipStream_t s) {
+    impl_->counted[0] = impl_->counted[1] = 0;
+    if (!impl_->slot[table & 1].awaited) return;
+    impl_->watch->stream = s;
+    impl_->watch->pending = true;
+}
 
 int FusedFrame::blocks(int table) const { return impl_->slot[table & 1].blocks; }
 unsigned long long FusedFrame::token(int table) const { return impl_->slot[table & 1].token; }

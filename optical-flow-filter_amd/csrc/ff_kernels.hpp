@@ -255,9 +255,10 @@ public:
     // frame_slot is k read frames[k] in place instead of their img (when
     // its ptr is not null).
     void launch(int table, hipStream_t s, const FrameRef* frames = nullptr, int nframes = 0);
-    // A graph holding launches of this frame was replayed on the stream:
-    // the next direct launch clears the tile flags first.
-    void replayed();
+    // A graph holding a launch of the table was replayed on s: the next direct
+    // launch clears the tile flags first, and the next check reads the count
+    // of the waits that gave up.
+    void replayed(int table, hipStream_t s);
     // Waves per workgroup (a tile's buffer is 64 columns by waves * rows
     // per thread rows): 0 = autotune (default), or 16, 15, 8, 5, 4. waves()
     // reports the fixed or tuned value (0 before tuning).

@@ -94,3 +94,28 @@ def test_an_earlier_error_does_not_upset_the_count(ffo):
             assert f.waitTimeouts() == 0
         after = _order_state()
         assert after[0] == after[1]
+
+
+@pytest.mark.gpu
+def test_timeouts_of_replayed_frames_are_reported():
+    """Frames of four levels are replayed from a graph: a wait in a replay that
+    gives up (forced by the test hook) is an error of the next check, also
+    after an earlier check has read the count."""
+    from flowfilter import errors
+    h, w = 1088, 2048
+    f = _pyr(h, w, 4)
+    assert f.graphs
+    frames = _frames(h, w, 2, 4)
+    step = lambda t: (f.loadImage(frames[t % 2]), f.compute())
+    for t in range(4):
+        step(t)
+    f.elapsedTime()
+    f.setWaitTest(4)
+    for t in range(8):  # records the graphs, then replays them
+        print("replayed frame", t, flush=True)
+        step(t)
+        with pytest.raises(errors.FilterError, match="spin limit"):
+            f.elapsedTime()
+    f.setWaitTest(0)
+    step(0)
+    f.elapsedTime()
