@@ -408,8 +408,9 @@ FF_API ff_status ff_filter_set_wait_test(ff_stage* s, int spins);
 /* Test hook (no reference counterpart): fused launches of different streams
  * are ordered by a count of the tiles that have started. After waiting for the
  * device: how many its launches should have started, and have (the same,
- * modulo 2^32). */
-FF_API ff_status ff_wait_order_state(unsigned* expected, unsigned* started);
+ * modulo 2^32), and how many times a launch found that a wait for another
+ * stream's launch had given up. */
+FF_API ff_status ff_wait_order_state(unsigned* expected, unsigned* started, unsigned* gave_up);
 
 /* Tile height of the fused frame kernel, in waves per workgroup (no
  * reference counterpart): 0 (the default) times the candidates 16, 15, 8, 5

@@ -682,10 +682,13 @@ ff_status ff_filter_get_wait_timeouts(ff_stage* s, unsigned long long* out) {
     });
 }
 
-ff_status ff_wait_order_state(unsigned* expected, unsigned* started) {
+ff_status ff_wait_order_state(unsigned* expected, unsigned* started, unsigned* gave_up) {
     return guard([&] {
-        out_ptr(expected, "expected"), out_ptr(started, "started");
-        wait_order_state(expected, started);
+        out_ptr(expected, "expected"), out_ptr(started, "started"), out_ptr(gave_up, "gave_up");
+        const WaitOrderState st = wait_order_state();
+        *expected = st.expected;
+        *started = st.started;
+        *gave_up = st.gave_up;
     });
 }
 

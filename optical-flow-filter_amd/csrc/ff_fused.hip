@@ -602,9 +602,20 @@ __global__ void __launch_bounds__(1024, RLOW == 4 ? 8 : 1) k_fused_frame(LaunchA
     else level_tile<true, IMG_U8_DOWN, RLOW, INNER>(q, t, xch, nw, fr);
 }
 
-__global__ void __launch_bounds__(LANES) k_wait_started(const unsigned* word, unsigned target) {
+// (The stream behind it goes on either way, so that its work ends; the count
+// makes the filter's next check an error.)
+__global__ void __launch_bounds__(LANES) k_wait_started(const unsigned* word, unsigned target, int spin_limit,
+                                                        unsigned* timeouts, unsigned* gave_up) {
     int spins = 0;
-    while ((int)(flag_load(word) - target) < 0 && ++spins < kSpinLimit / 8) __builtin_amdgcn_s_sleep(8);
+    while ((int)(flag_load(word) - target) < 0) {
+        __builtin_amdgcn_s_sleep(8);
+        if (++spins <= spin_limit) continue;
+        if (lane_id() == 0) {
+            flag_add(timeouts);
+            __hip_atomic_store(gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        break;
+    }
 }
 
 __global__ void k_clear_flags(unsigned* c, int n) {
@@ -653,8 +664,9 @@ bool tiles_with(const LevelArgs& a, int rows) {
 
 }  // namespace
 
-void launch_wait_started(const unsigned* word, unsigned target, hipStream_t s) {
-    hipLaunchKernelGGL(k_wait_started, dim3(1), dim3(LANES), 0, s, word, target);
+void launch_wait_started(const unsigned* word, unsigned target, int spin_limit, unsigned* timeouts, unsigned* gave_up,
+                         hipStream_t s) {
+    hipLaunchKernelGGL(k_wait_started, dim3(1), dim3(LANES), 0, s, word, target, spin_limit, timeouts, gave_up);
 }
 
 bool fused_level_supported(const LevelArgs& a) {
@@ -754,6 +766,14 @@ struct FusedFrame::Impl {
     int table(const std::vector<LevelArgs>& jobs, int nw, int rtop, int rlow, bool inner, hipStream_t s);
     unsigned* region(int si) const { return (unsigned*)flags.data() + (size_t)si * nflags; }
     unsigned* timeout_word() const { return (unsigned*)flags.data() + (size_t)2 * nflags; }
+    // the waits of the test hook wait for what no launch writes
+    WaitArgs wait_args() const {
+        return test_spins > 0 ? WaitArgs{test_spins, 0x40000000u} : WaitArgs{kSpinLimit, 0u};
+    }
+    AwaitedTiles awaited(const Table& t) const {
+        const WaitArgs wa = wait_args();
+        return AwaitedTiles{t.awaited, timeout_word(), wa.spin_limit, wa.bias};
+    }
     void clear_flags(int si, hipStream_t s) const;
     void run(int t, hipStream_t s, const FrameRef* frames = nullptr, int nframes = 0);
     void tune(const std::vector<LevelArgs>& jobs, hipStream_t s);
@@ -967,7 +987,7 @@ void FusedFrame::Impl::run(int ti, hipStream_t s, const FrameRef* frames, int nf
         }
         e = ++epoch[si];
     }
-    const WaitArgs wa{test_spins > 0 ? test_spins : kSpinLimit, test_spins > 0 ? 0x40000000u : 0u};
+    const WaitArgs wa = wait_args();
     FrameArgs fa;
     std::memset(&fa, 0, sizeof(fa));
     for (int k = 0; k < nframes; ++k) {
@@ -976,7 +996,7 @@ void FusedFrame::Impl::run(int ti, hipStream_t s, const FrameRef* frames, int nf
     }
     watch->stream = s;
     if (t.awaited) watch->pending = true;
-    const WaitingLaunch order(s, t.awaited);
+    const WaitingLaunch order(s, awaited(t));
     ProfileScope ps("fused_frame", s);
     const char* base = (const char*)t.dev.data();
     const TileFlags fl{region(si), timeout_word(), order.started(), e};
@@ -1104,7 +1124,7 @@ void FusedFrame::replayed(int table, hipStream_t s) {
 
 int FusedFrame::blocks(int table) const { return impl_->slot[table & 1].blocks; }
 unsigned long long FusedFrame::token(int table) const { return impl_->slot[table & 1].token; }
-int FusedFrame::awaited(int table) const { return impl_->slot[table & 1].awaited; }
+AwaitedTiles FusedFrame::awaited(int table) const { return impl_->awaited(impl_->slot[table & 1]); }
 
 void FusedFrame::setWaves(int nw) {
     bool ok = nw == 0;
@@ -1196,8 +1216,9 @@ void WaitCheck::check(const char* who) {
         const unsigned long long d = n - seen;
         seen = n;
         throw runtime_error(std::string(who) + ": " + std::to_string(d) +
-                            " wait(s) of the fused frame kernel for the level above gave up after the spin limit "
-                            "since the last check; the flow of those frames is not valid");
+                            " wait(s) of the fused frame kernel (for the level above, or for a launch on another "
+                            "stream) gave up after the spin limit since the last check; the flow of those frames is "
+                            "not valid");
     }
 }
 

@@ -225,9 +225,13 @@ struct WaitCheck {
     void check(const char* who);
 };
 
+struct AwaitedTiles;  // ff_runtime.hpp
+
 // One wave on stream s that ends once *word has reached target (compared
-// modulo 2^32; bounded by a spin limit). See WaitingLaunch.
-void launch_wait_started(const unsigned* word, unsigned target, hipStream_t s);
+// modulo 2^32). After spin_limit polls it gives up, adds 1 to *timeouts and sets
+// *gave_up (pinned host memory). See WaitingLaunch.
+void launch_wait_started(const unsigned* word, unsigned target, int spin_limit, unsigned* timeouts, unsigned* gave_up,
+                         hipStream_t s);
 
 // Returns false when the level's parameters are outside what the fused
 // kernel handles (the caller then runs the stage kernels).
@@ -297,8 +301,8 @@ public:
     // whenever that memory is replaced, so recorded launches (graphs) keyed
     // by it never refer to freed memory.
     unsigned long long token(int table) const;
-    // Tiles of the table that other tiles of it wait for (see WaitingLaunch).
-    int awaited(int table) const;
+    // Tiles of the table that other tiles of it wait for.
+    AwaitedTiles awaited(int table) const;
 
 private:
     struct Impl;

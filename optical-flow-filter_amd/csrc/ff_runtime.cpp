@@ -439,11 +439,20 @@ void Image::swapBuffers(Image& o) {
 // ------------------------------------------------------------ WaitingLaunch
 
 namespace {
-// Per device: the order of the launches, and the word that counts their
-// awaited tiles as they start.
+// Per device: the order of the launches, the word that counts their awaited
+// tiles as they start, the mark of the last launch, and whether a poll gave up
+// (pinned, written by the device).
 struct WaitingState {
     LaunchOrder order;
     unsigned* word = nullptr;
+    hipEvent_t mark = nullptr;
+    volatile unsigned* gave_up = nullptr;
+    unsigned times = 0;  // that it had
+    unsigned read() const {
+        unsigned n = 0;
+        FF_HIP(hipMemcpy(&n, word, sizeof(n), hipMemcpyDeviceToHost));
+        return n;
+    }
 };
 // Kept for the process (never destroyed), like the library stream: boxes
 // may be destroyed during the process's exit.
@@ -477,8 +486,8 @@ bool capturing(hipStream_t s) {
 }
 }  // namespace
 
-WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) : s_(s), awaited_(awaited) {
-    if (awaited <= 0) return;
+WaitingLaunch::WaitingLaunch(hipStream_t s, const AwaitedTiles& awaited) : s_(s), awaited_(awaited.count) {
+    if (awaited.count <= 0) return;
     if (t_outermost || capturing(s)) {
         if (!t_outermost) t_outermost = this;
         outer_ = t_outermost;
@@ -489,6 +498,16 @@ WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) : s_(s), awaited_(await
     std::unique_lock<std::mutex> lk(g.mu);
     if ((int)g.dev.size() <= dev_) g.dev.resize(dev_ + 1);
     WaitingState& w = g.dev[dev_];
+    // (it orders launches and no data, so it needs no flush to the system's
+    // scope: 58.6 us per 2048x1088 two-level frame of three filters taking
+    // turns, 59.5 us with one)
+    if (!w.mark) FF_HIP(hipEventCreateWithFlags(&w.mark, hipEventDisableTiming | hipEventDisableSystemFence));
+    if (!w.gave_up) {
+        unsigned* p = nullptr;
+        FF_HIP(hipHostMalloc((void**)&p, sizeof(unsigned), hipHostMallocDefault));
+        *p = 0;
+        w.gave_up = p;
+    }
     if (!w.word) {
         unsigned* p = nullptr;
         FF_HIP(hipMalloc((void**)&p, sizeof(unsigned)));
@@ -496,12 +515,38 @@ WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) : s_(s), awaited_(await
         FF_HIP(hipMemcpy(p, &zero, sizeof(zero), hipMemcpyHostToDevice));
         w.word = p;
     }
-    const auto last = (hipStream_t)w.order.last;
-    // (a stream of the caller's may have been destroyed: it is not asked)
-    if (w.order.follows(s) && !(g.owned.count(last) && !capturing(last) && hipStreamQuery(last) == hipSuccess)) {
-        launch_wait_started(w.word, w.order.target, s);
-        check_launch("WaitingLaunch");
+    if (*w.gave_up) {
+        // the launch behind that poll may be beside the one it waited for
+        FF_HIP(hipDeviceSynchronize());
+        *w.gave_up = 0;
+        ++w.times;
+        w.order.restart(w.read());
     }
+    // (a stream of the caller's may have been destroyed: it is not asked, nor
+    // is a stream that is being captured)
+    const auto last = (hipStream_t)w.order.last;
+    const auto before = w.order.before(s);
+    if (before != LaunchOrder::Before::NOTHING) {
+        const bool live = g.owned.count(last) && !capturing(last);
+        const bool idle = live && hipStreamQuery(last) == hipSuccess;
+        if (idle) {
+            // it is done
+        } else if (before == LaunchOrder::Before::GATE) {
+            FF_HIP(hipStreamWaitEvent(s, w.mark, 0));
+            launch_wait_started(w.word, w.order.target + awaited.bias, awaited.spin_limit, awaited.timeouts,
+                                (unsigned*)w.gave_up, s);
+            check_launch("WaitingLaunch");
+        } else if (live) {
+            FF_HIP(hipEventRecord(w.mark, last));
+            FF_HIP(hipStreamWaitEvent(s, w.mark, 0));
+        } else {
+            FF_HIP(hipDeviceSynchronize());
+        }
+        if (!idle) w.order.switched();
+    }
+    // (whatever the event marked so far, this launch's stream is past it)
+    marked_ = w.order.mark();
+    if (marked_) FF_HIP(hipEventRecord(w.mark, s));
     lk.release();  // held until the destructor
     word_ = w.word;
     locked_ = true;
@@ -509,7 +554,7 @@ WaitingLaunch::WaitingLaunch(hipStream_t s, int awaited) : s_(s), awaited_(await
 }
 
 void WaitingLaunch::launched() const {
-    if (outer_ && outer_->locked_) waiting().dev[outer_->dev_].order.launched(outer_->s_, awaited_);
+    if (outer_ && outer_->locked_) waiting().dev[outer_->dev_].order.launched(outer_->s_, awaited_, outer_->marked_);
 }
 
 WaitingLaunch::~WaitingLaunch() {
@@ -517,17 +562,15 @@ WaitingLaunch::~WaitingLaunch() {
     if (locked_) waiting().mu.unlock();
 }
 
-bool wait_order_state(unsigned* expected, unsigned* started) {
+WaitOrderState wait_order_state() {
     int dev = 0;
     FF_HIP(hipGetDevice(&dev));
     FF_HIP(hipDeviceSynchronize());
     Waiting& g = waiting();
     std::lock_guard<std::mutex> lk(g.mu);
-    *expected = *started = 0;
-    if ((int)g.dev.size() <= dev || !g.dev[dev].word) return false;
-    *expected = g.dev[dev].order.target;
-    FF_HIP(hipMemcpy(started, g.dev[dev].word, sizeof(unsigned), hipMemcpyDeviceToHost));
-    return true;
+    if ((int)g.dev.size() <= dev || !g.dev[dev].word) return {};
+    const WaitingState& w = g.dev[dev];
+    return {w.order.target, w.read(), w.times};
 }
 
 // ------------------------------------------------------------- InputFrames

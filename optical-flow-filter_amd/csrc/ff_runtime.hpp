@@ -203,6 +203,15 @@ private:
     std::vector<std::shared_ptr<StreamBox>> others_;
 };
 
+// Tiles of a fused frame launch that other tiles of it wait for, and where and
+// when a wait for them gives up.
+struct AwaitedTiles {
+    int count = 0;
+    unsigned* timeouts = nullptr;  // counts the waits that gave up (device)
+    int spin_limit = 0;
+    unsigned bias = 0;  // added to what is waited for (0, or a test's unreachable value)
+};
+
 // Around a fused frame launch in which some tiles wait for others of the same
 // launch (a pyramid's second level for its top level's tiles), a graph launch
 // included. Inside one launch the awaited tiles' blocks come first, and each
@@ -211,12 +220,20 @@ private:
 // awaited tiles are queued behind them there. So such a launch starts only
 // when every awaited tile of the one before it, whatever stream that was on,
 // has started (awaited tiles never wait, so from then on that launch drains
-// by itself): the tiles count themselves in one device word (started()), and
-// when the launch before was on another stream, which has not finished, a
-// kernel of one wave goes before this launch and polls that word. The end of
-// one launch and the start of the next overlap then. (With an event that
-// marked the end of the launch before, three filters on streams of their own
-// took 81 us per 2048x1088 two-level frame, for a launch of 55 us.)
+// by itself). When the launch before was on another stream, which has not
+// finished, this one's stream first waits for an event recorded right before
+// that launch, and then a kernel of one wave polls a device word in which the
+// awaited tiles count themselves (started()). The end of one launch and the
+// start of the next overlap then. (With an event that marked the end of the
+// launch before instead, three filters on streams of their own took 81 us per
+// 2048x1088 two-level frame, for a launch of 55 us.)
+//
+// The poll alone would have no bound: what its stream has queued before a
+// launch may take any time (a caller's stream with work of its own). With the
+// event it spans the launch's start only. It still gives up after the waits'
+// spin limit of 2 s, when other kernels have held the GPU all that time; the
+// launch behind it then goes, its filter's next check is an error, and the
+// next launch of any filter waits for the device.
 //
 // Constructed under a process-wide lock that is held until destruction, so
 // that launches are numbered in the order in which they are enqueued, and
@@ -225,7 +242,7 @@ private:
 // counted nor ordered, since its replays are not seen.
 class WaitingLaunch {
 public:
-    WaitingLaunch(hipStream_t s, int awaited);
+    WaitingLaunch(hipStream_t s, const AwaitedTiles& awaited);
     ~WaitingLaunch();
     WaitingLaunch(const WaitingLaunch&) = delete;
     WaitingLaunch& operator=(const WaitingLaunch&) = delete;
@@ -241,13 +258,16 @@ private:
     int awaited_ = 0, dev_ = 0;
     const WaitingLaunch* outer_ = nullptr;  // this one, or the one it is nested in
     unsigned* word_ = nullptr;
-    bool locked_ = false;
+    bool locked_ = false, marked_ = false;
 };
 
-// Test hook: the awaited tiles that the current device's launches should have
-// started, and that have, after waiting for the device. Returns false (zeros)
-// before the first such launch.
-bool wait_order_state(unsigned* expected, unsigned* started);
+// Test hook, after waiting for the device: the awaited tiles that its launches
+// should have started, those that have, and how many times a launch found that
+// a poll before it had given up (all 0 before the first such launch).
+struct WaitOrderState {
+    unsigned expected = 0, started = 0, gave_up = 0;
+};
+WaitOrderState wait_order_state();
 
 // Host frames for a filter's own input image, double buffered: load()
 // copies a host frame into a pinned host buffer (on a few threads), then

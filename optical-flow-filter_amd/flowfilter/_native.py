@@ -232,7 +232,7 @@ SIGNATURES = {
     "ff_filter_get_graphs": [_S, _pi],
     "ff_filter_get_wait_timeouts": [_S, ctypes.POINTER(ctypes.c_ulonglong)],
     "ff_filter_set_wait_test": [_S, _i],
-    "ff_wait_order_state": [ctypes.POINTER(ctypes.c_uint), ctypes.POINTER(ctypes.c_uint)],
+    "ff_wait_order_state": [ctypes.POINTER(ctypes.c_uint)] * 3,
     "ff_filter_set_tile_waves": [_S, _i],
     "ff_filter_get_tile_waves": [_S, _pi],
     "ff_filter_set_tile_top_rows": [_S, _i],

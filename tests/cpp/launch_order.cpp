@@ -3,6 +3,9 @@
 #include "ff_launch_order.hpp"
 
 #include <cstdio>
+#include <deque>
+#include <random>
+#include <vector>
 
 using ffamd::LaunchOrder;
 
@@ -17,25 +20,142 @@ using ffamd::LaunchOrder;
 // Only launches that were enqueued count, and a failed one is not the launch
 // that the next follows.
 static int failed_launches() {
+    using Before = LaunchOrder::Before;
     int streams[3];
     const void *a = &streams[0], *b = &streams[1], *c = &streams[2];
     LaunchOrder o;
-    CHECK(!o.follows(a));
-    o.launched(a, 10);
-    CHECK(o.target == 10 && !o.follows(a) && o.follows(b));
+    CHECK(o.before(a) == Before::NOTHING);
+    o.launched(a, 10, false);
+    CHECK(o.target == 10 && o.before(a) == Before::NOTHING && o.before(b) == Before::END);
     // (a launch on b fails: nothing is noted)
-    CHECK(o.follows(b) && o.follows(c) && !o.follows(a) && o.target == 10);
-    o.launched(c, 5);
-    CHECK(o.target == 15 && o.follows(a) && !o.follows(c));
+    CHECK(o.before(b) == Before::END && o.before(c) == Before::END && o.target == 10);
+    o.switched();
+    CHECK(o.mark());
+    o.launched(c, 5, true);
+    CHECK(o.target == 15 && o.before(a) == Before::GATE && o.before(c) == Before::NOTHING);
     o.finished(a);
-    CHECK(o.follows(a));
+    CHECK(o.before(a) == Before::GATE);
     o.finished(c);
-    CHECK(!o.follows(a) && o.target == 15);
-    // modulo 2^32
+    CHECK(o.before(a) == Before::NOTHING && o.target == 15);
+    // marks stop on one stream alone
+    for (int k = 0; k < LaunchOrder::kMarks; ++k) o.launched(a, 1, o.mark());
+    CHECK(!o.mark() && o.before(b) == Before::END);
+    // modulo 2^32, and from the device's count
     o.target = 0xfffffffeu;
-    o.launched(a, 5);
+    o.launched(a, 5, false);
     CHECK(o.target == 3u);
+    o.restart(7);
+    CHECK(o.target == 7u && o.before(b) == Before::NOTHING);
     return 0;
 }
 
-int main() { return failed_launches(); }
+// A model of streams whose launches wait as WaitingLaunch has them wait. Time
+// goes in steps; a launch's awaited tiles start up to kDispatch steps after its
+// turn comes, a poll gives up after kPoll, and what else a stream holds takes
+// up to 100 times that. No poll may give up, and no launch may start before the
+// awaited tiles of every launch enqueued earlier have.
+static const int kDispatch = 5, kPoll = 50;
+struct Op {
+    enum Kind { WORK, MARK, WAIT, POLL, LAUNCH } kind;
+    long arg;    // WORK: steps; MARK, WAIT: the event's record; POLL: the count; LAUNCH: its number
+    long spent;  // steps so far
+};
+static int model(unsigned seed, int nstreams, int launches) {
+    std::mt19937 rng(seed);
+    auto rnd = [&](long n) { return (long)(rng() % (unsigned long)n); };
+    std::vector<std::deque<Op>> q(nstreams);
+    std::vector<int> names(nstreams);
+    std::vector<char> recorded;  // per record of the event: reached
+    std::vector<long> delay;     // of each launch's start
+    std::vector<char> started;
+    LaunchOrder o;
+    unsigned word = 0;
+    long mark = -1;
+    int enqueued = 0;
+    auto record = [&](int s) {
+        mark = (long)recorded.size();
+        recorded.push_back(0);
+        q[s].push_back({Op::MARK, mark, 0});
+    };
+    for (long t = 0;; ++t) {
+        // the host: now and then a launch, mostly in bursts without a look at the device
+        while (enqueued < launches && rnd(40) < 20) {
+            const int s = rnd(10) == 0 ? 0 : (int)rnd(nstreams);
+            if (rnd(6) == 0) q[s].push_back({Op::WORK, rnd(100 * kPoll), 0});
+            const auto before = o.before(&names[s]);
+            if (before != LaunchOrder::Before::NOTHING) {
+                const int last = (int)((const int*)o.last - names.data());
+                const bool idle = q[last].empty();
+                if (idle) {
+                    // it is done
+                } else if (before == LaunchOrder::Before::GATE) {
+                    q[s].push_back({Op::WAIT, mark, 0});
+                    q[s].push_back({Op::POLL, (long)o.target, 0});
+                } else {
+                    record(last);
+                    q[s].push_back({Op::WAIT, mark, 0});
+                }
+                if (!idle) o.switched();
+            }
+            const bool with_mark = o.mark();
+            if (with_mark) record(s);
+            if (rnd(8) == 0) continue;  // the launch fails
+            q[s].push_back({Op::LAUNCH, enqueued++, 0});
+            delay.push_back(1 + rnd(kDispatch));
+            started.push_back(0);
+            o.launched(&names[s], 3, with_mark);
+            // (a run on one stream, past the marks)
+            if (rnd(50) == 0)
+                for (int k = 0; k < LaunchOrder::kMarks + 2 && enqueued < launches; ++k) {
+                    const bool m = o.mark();
+                    if (m) record(s);
+                    q[s].push_back({Op::LAUNCH, enqueued++, 0});
+                    delay.push_back(1 + rnd(kDispatch));
+                    started.push_back(0);
+                    o.launched(&names[s], 3, m);
+                }
+        }
+        bool idle = true;
+        for (auto& st : q) {
+            if (st.empty()) continue;
+            idle = false;
+            Op& op = st.front();
+            ++op.spent;
+            bool done = false;
+            switch (op.kind) {
+            case Op::WORK: done = op.spent > op.arg; break;
+            case Op::MARK:
+                recorded[op.arg] = 1;
+                done = true;
+                break;
+            case Op::WAIT: done = recorded[op.arg] != 0; break;
+            case Op::POLL:
+                done = (int)(word - (unsigned)op.arg) >= 0;
+                CHECK(done || op.spent <= kPoll);
+                break;
+            case Op::LAUNCH:
+                if (op.spent == delay[op.arg]) {
+                    for (long k = 0; k < op.arg; ++k) CHECK(started[k]);
+                    started[op.arg] = 1;
+                    word += 3;
+                }
+                done = op.spent >= delay[op.arg] + 10;
+                break;
+            }
+            if (done) st.pop_front();
+        }
+        if (idle && enqueued == launches) break;
+    }
+    CHECK(word == o.target && word == 3u * (unsigned)launches);
+    return 0;
+}
+
+int main() {
+    if (failed_launches()) return 1;
+    for (unsigned seed = 0; seed < 60; ++seed)
+        if (model(seed, 2 + (int)seed % 7, 400)) {
+            std::printf("seed %u\n", seed);
+            return 1;
+        }
+    return 0;
+}

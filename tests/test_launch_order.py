@@ -36,9 +36,9 @@ def _frames(h, w, n, seed):
 
 def _order_state():
     from flowfilter import _native as N
-    a, b = ctypes.c_uint(), ctypes.c_uint()
-    N.call("ff_wait_order_state", ctypes.byref(a), ctypes.byref(b))
-    return a.value, b.value
+    v = [ctypes.c_uint() for _ in range(3)]
+    N.call("ff_wait_order_state", *[ctypes.byref(x) for x in v])
+    return [x.value for x in v]
 
 
 def _hip_runtime():
@@ -119,3 +119,109 @@ def test_timeouts_of_replayed_frames_are_reported():
     f.setWaitTest(0)
     step(0)
     f.elapsedTime()
+
+
+def _backlog(stream, seconds):
+    """About that much work on a torch stream, of one wave."""
+    import torch
+    e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    with torch.cuda.stream(stream):
+        for _ in range(2):  # (the first loads the kernel)
+            e[0].record()
+            torch.cuda._sleep(10 ** 7)
+            e[1].record()
+            e[1].synchronize()
+        ms = e[0].elapsed_time(e[1])
+        print("10^7 cycles of it: %.2f ms" % ms, flush=True)
+        torch.cuda._sleep(int(10 ** 7 * min(seconds * 1e3 / ms, 1e3)))
+
+
+def _two_filters(ffo, h, w):
+    """Two filters that have taken turns, one of them on a torch stream, and
+    the oracle after the same frames."""
+    import torch
+    side = torch.cuda.Stream()
+    a, b = _pyr(h, w), _pyr(h, w)
+    a.stream = side.cuda_stream
+    o = ffo.PyramidalFlowFilter(h, w, 2)
+    o.configure_like([10.0, 30.0], 4.0, [2, 2])
+    frames = _frames(h, w, 6, 9)
+    for img in frames[:4]:
+        for f in (a, b):
+            f.loadImage(img)
+            f.compute()
+        o.compute(img)
+    a.getFlow(), b.getFlow()
+    return side, a, b, o, frames
+
+
+@pytest.mark.gpu
+def test_a_launch_behind_a_backlog_is_waited_for(ffo):
+    """A filter's launch is queued behind a second of other work of its stream:
+    a launch of a filter on another stream comes after it, however long that
+    takes."""
+    import time
+
+    import torch
+    h, w = 272, 512
+    side, a, b, o, frames = _two_filters(ffo, h, w)
+    own = torch.cuda.ExternalStream(b.stream)
+    for t, img in enumerate(frames[4:]):
+        print("backlog", t, flush=True)
+        for f in (a, b):
+            f.loadImage(img)
+        _backlog(side, 1.0)
+        busy = torch.cuda.Event()
+        busy.record(side)
+        a.compute()
+        b.compute()
+        time.sleep(0.6)
+        assert not busy.query(), "the backlog is too short for this test"
+        assert not own.query()
+        o.compute(img)
+        for f in (a, b):
+            assert np.array_equal(f.getFlow(), o.downloadFlow())
+            assert f.waitTimeouts() == 0
+    st = _order_state()
+    assert st[0] == st[1]
+
+
+@pytest.mark.gpu
+def test_a_wait_for_another_streams_launch_that_gives_up_is_an_error(ffo):
+    """Forced by the test hook (a few polls, for a count that no launch
+    reaches): the wait is counted and reported, the next launch finds the
+    device idle, and the other filter's frames stay right."""
+    from flowfilter import errors
+    h, w = 272, 512
+    side, a, b, o, frames = _two_filters(ffo, h, w)
+    gave_up = _order_state()[2]
+    img = frames[4]
+    b.loadImage(img)
+    b.compute()  # (in a state of its own from here on)
+    b.elapsedTime()
+    n = b.waitTimeouts()
+    b.setWaitTest(4)
+    b.compute()
+    with pytest.raises(errors.FilterError, match="spin limit"):
+        b.elapsedTime()
+    alone = b.waitTimeouts() - n  # of a launch without another before it
+    for f in (a, b):
+        f.loadImage(img)
+    _backlog(side, 0.2)
+    a.compute()
+    b.compute()
+    with pytest.raises(errors.FilterError, match="spin limit"):
+        b.elapsedTime()
+    assert b.waitTimeouts() - n == 2 * alone + 1
+    b.setWaitTest(0)
+    o.compute(img)
+    assert np.array_equal(a.getFlow(), o.downloadFlow())
+    for f in (b, a):
+        f.loadImage(frames[5])
+        f.compute()
+    b.elapsedTime()
+    o.compute(frames[5])
+    assert np.array_equal(a.getFlow(), o.downloadFlow())
+    assert a.waitTimeouts() == 0
+    st = _order_state()
+    assert st[0] == st[1] and st[2] == gave_up + 1
