@@ -1458,14 +1458,19 @@ namespace ad {
 void image_model(const float* I, float* a0, float* g, int B, int H, int W, hipStream_t s) {
     hipLaunchKernelGGL(k_ad_image_model, grid3(B, H, W), dim3(BX, BY), 0, s, I, a0, (float2*)g, Dims{H, W});
 }
+// Whether na floats at a and nb floats at b share memory.
+bool overlap(const float* a, size_t na, const float* b, size_t nb) {
+    const auto pa = (uintptr_t)a, pb = (uintptr_t)b;
+    return pa < pb + nb * sizeof(float) && pb < pa + na * sizeof(float);
+}
 void image_model_bwd(const float* ga0, const float* gg, float* gI, float* work, int B, int H, int W, int acc,
                      hipStream_t s) {
-    // a result that replaces an input goes through the work buffer, since the
+    // a result that overlaps an input goes through the work buffer, since the
     // adjoint reads neighbours
-    const bool inplace = gI == ga0 || gI == gg;
+    const size_t n = (size_t)B * H * W;
+    const bool inplace = overlap(gI, n, ga0, n) || overlap(gI, n, gg, 2 * n);
     launch_image_model_adjoint(ga0, gg, inplace ? work : gI, B, H, W, inplace ? 0 : acc, s);
     if (inplace) {
-        const size_t n = (size_t)B * H * W;
         hipLaunchKernelGGL(k_ad_put, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, work, gI, n, acc);
     }
 }
@@ -1473,14 +1478,10 @@ void smooth_steps_bwd(const float* gout, const float* gout2, float* gin, int n, 
                       hipStream_t s) {
     launch_smooth_adjoint(gout, gout2, gin, n, B, H, W, acc, s);
 }
-// (a result that overlaps the image goes through the work buffer)
-bool overlap(const float* a, size_t na, const float* b, size_t nb) {
-    const auto pa = (uintptr_t)a, pb = (uintptr_t)b;
-    return pa < pb + nb * sizeof(float) && pb < pa + na * sizeof(float);
-}
 void down(const float* I, float* O, float* work, int B, int H, int W, hipStream_t s) {
     const Dims d{H, W}, h{H / 2, W / 2};
     const size_t n = (size_t)B * h.H * h.W;
+    // (as above)
     const bool inplace = overlap(I, (size_t)B * H * W, O, n);
     hipLaunchKernelGGL(k_ad_down, grid3(B, h.H, h.W), dim3(BX, BY), 0, s, I, inplace ? work : O, d, h);
     if (inplace)

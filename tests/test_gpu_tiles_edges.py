@@ -1,0 +1,42 @@
+"""Calls that the tile kernels (ff_tiles.hip) take, at the edges of what they
+accept: results that overlap inputs, sizes beyond 32-bit offsets, many
+iterations, and what the profile counts of them."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _stream():
+    import torch
+    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def _p(t):
+    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+
+
+@pytest.mark.parametrize("B,h,w", [(1, 5, 7), (2, 33, 65), (3, 130, 200)])
+@pytest.mark.parametrize("acc", [0, 1])
+def test_image_model_adjoint_that_overlaps_its_inputs(B, h, w, acc):
+    """The result anywhere in the gradients it is computed from is bitwise the
+    result beside them: at the start, inside and in the second half of the
+    image gradient's, and one row into the brightness'."""
+    import torch
+    from flowfilter import _native as N
+    print("image model adjoint", (B, h, w), acc, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(h)
+    n = B * h * w
+    ga = torch.randn(n, generator=g, device="cuda")
+    gg = torch.randn(2 * n, generator=g, device="cuda")
+    work = torch.empty(B, 2 * h, w, device="cuda")
+    call = lambda a, d, o: N.call("ff_ad_image_model_backward", _p(a), _p(d), _p(o), _p(work), B, h, w, acc, _stream())
+    for base, off in (("gg", 0), ("gg", 2 * w), ("gg", n - 1), ("gg", n), ("gg", 2 * n - 2), ("ga", w), ("ga", n - 1)):
+        buf = {"ga": torch.cat([ga, ga[:n]]), "gg": torch.cat([gg, gg[:n]])}
+        out = buf[base][off:off + n]
+        want = out.clone()
+        call(ga, gg, want)
+        call(buf["ga"][:n], buf["gg"][:2 * n], out)
+        assert torch.equal(out, want), (base, off)
