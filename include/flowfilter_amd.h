@@ -682,9 +682,12 @@ FF_API ff_status ff_ad_photometric_backward(const float* frames, const float* fl
  * stages only, src/gpu/pipeline.cu:63-89). Between begin and end, every
  * kernel launch whose name contains `filter` is bracketed by HIP events on
  * its stream; end waits for them and returns the summed milliseconds and
- * the number of launches. Kernel names: image_model, propagate_x/_y,
- * propagate_payload_x/_y, update, delta_update, smooth_x/_y, down_x/_y,
- * scale_f2, copy2d, fused_top, fused_delta. */
+ * the number of launches. Kernel names: image_model, propagate_tile,
+ * propagate_payload_tile, smooth_tile and lax_wendroff_tile (iterations of an
+ * X and a Y pass each) or the single passes propagate_x/_y,
+ * propagate_payload_x/_y, smooth_x/_y and lax_wendroff_x/_y where the tile
+ * kernels do not apply; update, delta_update, down_x/_y, scale_f2,
+ * rotational_flow, flow_to_color, copy2d, copy_regions, fused_frame. */
 FF_API ff_status ff_profile_begin(const char* filter);
 FF_API ff_status ff_profile_end(double* total_ms, long long* count);
 

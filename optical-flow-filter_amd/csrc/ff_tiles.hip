@@ -755,6 +755,7 @@ bool launch_propagate(const PropFields& in, const PropFields& x, const PropField
     PropFields from = in;
     in_chunks(n, kMaxPropIters, [&](bool, int k, bool to_y) {
         const PropFields& to = to_y ? y : x;
+        ProfileScope ps(in.s ? "propagate_payload_tile" : "propagate_tile", s);
         launch_propagate_tile(from, PropFields{}, 0, to, k, 1, H, W, dt, border, s);
         from = to;
     });
@@ -766,10 +767,10 @@ bool launch_smooth(const DevImg& in, const DevImg& x, const DevImg& y, int n, hi
     if (!smooth_tile_supported((int)in.pitch, (int)y.pitch, H, W) || !smooth_tile_supported((int)x.pitch, (int)y.pitch, H, W) ||
         in.data == x.data || in.data == y.data)
         return false;
-    ProfileScope ps("smooth_tile", s);
     DevImg from = in;
     in_chunks(n, kMaxSmoothIters, [&](bool, int k, bool to_y) {
         const DevImg& to = to_y ? y : x;
+        ProfileScope ps("smooth_tile", s);
         launch_smooth_tile(from.data, (int)from.pitch, to.data, (int)to.pitch, k, 1, H, W, s);
         from = to;
     });
@@ -784,13 +785,13 @@ bool launch_lax_wendroff(const DevImg& flow, const DevImg& in, const DevImg& x, 
         if (!fits((long long)d->pitch, H)) return false;
     for (const DevImg* d : {&x, &y})
         if (in.data == d->data || flow.data == d->data) return false;
-    ProfileScope ps("lax_wendroff_tile", s);
     constexpr int kMost = 8;  // 48 of the buffer's 64 columns are output
     DevImg from = in;
     in_chunks(n, kMost, [&](bool, int k, bool last) {
         const DevImg& to = last ? x : y;  // the propagated image is the X pass's buffer
         const int nw = waves_for(1, H, W, k);
         const Tiling tl = tiling(H, W, k, nw * kTileRows);
+        ProfileScope ps("lax_wendroff_tile", s);
         hipLaunchKernelGGL(k_lax_wendroff_tile, dim3(tl.tiles_x * tl.tiles_y), dim3(nw * LANES),
                            (size_t)2 * nw * 2 * LANES * sizeof(float), s, flow, from, to, tl, k, dt);
         from = to;

@@ -40,3 +40,33 @@ def test_image_model_adjoint_that_overlaps_its_inputs(B, h, w, acc):
         call(ga, gg, want)
         call(buf["ga"][:n], buf["gg"][:2 * n], out)
         assert torch.equal(out, want), (base, off)
+
+
+@pytest.mark.parametrize("n", [1, 4, 9])
+def test_profile_counts_every_launch(n):
+    """Launches of several iterations are bracketed and counted one by one,
+    under the names that the header lists; the single passes under theirs."""
+    from flowfilter import _native as N
+    from flowfilter.gpu.flowsmoothing import FlowSmoother
+    from flowfilter.gpu.image import GPUImage
+    from flowfilter.gpu.propagation import FlowPropagator, FlowPropagatorPayload, LaxWendroffPropagator
+    print("profile", n, flush=True)
+    h, w = 70, 150
+
+    def img(*shape):
+        g = GPUImage(shape, 4)
+        g.upload(np.full(shape, 0.25, np.float32))
+        return g
+
+    flow, one = img(h, w, 2), img(h, w)
+    lw = LaxWendroffPropagator(flow, one)
+    lw.iterations = n
+    stages = [(FlowPropagator(flow, n), "propagate_tile", 4), (FlowPropagatorPayload(flow, one, flow, n), "propagate_payload_tile", 4),
+              (FlowSmoother(flow, n), "smooth_tile", 4), (lw, "lax_wendroff_tile", 8)]
+    passes = FlowPropagatorPayload(flow, one, flow, n)
+    passes.border = 0
+    for st, name, most in stages + [(passes, "propagate_payload_x", 1), (passes, "propagate_payload_y", 1)]:
+        N.profile_begin(name)
+        st.compute()
+        ms, launches = N.profile_end()
+        assert launches == -(-n // most) and ms > 0.0, name
