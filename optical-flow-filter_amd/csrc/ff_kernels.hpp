@@ -75,7 +75,6 @@ constexpr int kMaxPropIters = 4, kMaxSmoothIters = 4;
 bool propagate_tile_supported(const PropFields& in, const PropFields& out, int H, int W, int border);
 void launch_propagate_tile(const PropFields& in, const PropFields& mid, int after, const PropFields& out, int n, int B,
                            int H, int W, float dt, int border, hipStream_t s);
-bool smooth_tile_supported(int in_pitch, int out_pitch, int H, int W);
 void launch_smooth_tile(const void* in, int in_pitch, void* out, int out_pitch, int n, int B, int H, int W,
                         hipStream_t s);
 // Adjoints (ff_tiles.hip) of the image model, and of n <= kMaxSmoothIters

@@ -19,14 +19,16 @@ void require_shape(const Image& a, const Image& b, const char* who) {
 }
 
 PropFields prop_fields(const DevImg& f, const DevImg* s = nullptr, const DevImg* v = nullptr) {
+    // (a row of 2 GiB keeps a pitch that no tile kernel takes)
+    auto pitch = [](const DevImg& d) { return (int)std::min<size_t>(d.pitch, 0x7fffffff); };
     PropFields p;
     p.f = (float2*)f.data;
-    p.fp = (int)f.pitch;
+    p.fp = pitch(f);
     if (s) {
         p.s = (float*)s->data;
-        p.sp = (int)s->pitch;
+        p.sp = pitch(*s);
         p.v = (float2*)v->data;
-        p.vp = (int)v->pitch;
+        p.vp = pitch(*v);
     }
     return p;
 }

@@ -690,10 +690,6 @@ void launch_level_tile(const LevelFields& f, int B, int H, int W, int Hu, int Wu
     else f.grad ? form(no, yes) : form(no, no);
 }
 
-bool smooth_tile_supported(int in_pitch, int out_pitch, int H, int W) {
-    return H > 0 && W > 0 && fits(in_pitch, H) && fits(out_pitch, H);
-}
-
 void launch_smooth_tile(const void* in, int in_pitch, void* out, int out_pitch, int n, int B, int H, int W,
                         hipStream_t s) {
     if (n < 1 || n > kMaxSmoothIters) throw logic_error("smoothing: iterations of one launch out of range");
@@ -764,9 +760,9 @@ bool launch_propagate(const PropFields& in, const PropFields& x, const PropField
 
 bool launch_smooth(const DevImg& in, const DevImg& x, const DevImg& y, int n, hipStream_t s) {
     const int H = in.h, W = in.w;
-    if (!smooth_tile_supported((int)in.pitch, (int)y.pitch, H, W) || !smooth_tile_supported((int)x.pitch, (int)y.pitch, H, W) ||
-        in.data == x.data || in.data == y.data)
-        return false;
+    if (H <= 0 || W <= 0 || in.data == x.data || in.data == y.data) return false;
+    for (const DevImg* d : {&in, &x, &y})
+        if (!fits((long long)d->pitch, H)) return false;
     DevImg from = in;
     in_chunks(n, kMaxSmoothIters, [&](bool, int k, bool to_y) {
         const DevImg& to = to_y ? y : x;

@@ -70,3 +70,38 @@ def test_profile_counts_every_launch(n):
         st.compute()
         ms, launches = N.profile_end()
         assert launches == -(-n // most) and ms > 0.0, name
+
+
+def test_rows_of_two_gib(ffo):
+    """Rows longer than 32-bit offsets reach run in the single passes, with
+    64-bit offsets: bitwise the oracle's on crops at both ends and in the
+    middle (their edges left out)."""
+    import torch
+    from flowfilter.gpu.flowsmoothing import FlowSmoother
+    from flowfilter.gpu.image import GPUImage
+    from flowfilter.gpu.propagation import FlowPropagator
+    h, w = 3, 2 ** 28 + 70
+    print("rows of 2 GiB", (h, w), flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    img = GPUImage((h, w, 2), 4)
+    flow = torch.from_dlpack(img)
+    for row in flow:
+        row.uniform_(-1.0, 1.0, generator=g)
+    torch.cuda.synchronize()
+    starts = (0, w // 2 - 100, w - 200)
+
+    def check(got, oracle):
+        got = torch.from_dlpack(got)
+        for x in starts:
+            want = oracle(flow[:, x:x + 200].cpu().numpy())
+            inner = slice(0 if x == 0 else 10, 200 if x == starts[-1] else 190)
+            assert np.array_equal(got[:, x:x + 200].cpu().numpy()[:, inner], want[:, inner]), x
+
+    p = FlowPropagator(img, 2)
+    p.border = 1
+    p.compute()
+    check(p.getPropagatedFlow(), lambda a: ffo.propagate(a, 2, border=1))
+    del p
+    m = FlowSmoother(img, 2)
+    m.compute()
+    check(m.getSmoothedFlow(), lambda a: ffo.smooth(a, 2))
