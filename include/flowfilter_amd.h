@@ -561,7 +561,7 @@ typedef struct ff_ad_level {
  * below 64). */
 FF_API ff_status ff_ad_level_supported(int H, int W, int iterations, int smooth_iterations, int* supported);
 /* No output may be an input. gamma, maxflow: as for ff_ad_update (top level)
- * and ff_ad_delta_update; border >= 1. */
+ * and ff_ad_delta_update; border >= 1; the upper flow image below 2 GiB. */
 FF_API ff_status ff_ad_level_forward(const ff_ad_level* level, int iterations, int smooth_iterations, int B, int H,
                                      int W, int Hu, int Wu, float dt, int border, float gamma, float maxflow,
                                      void* stream);

@@ -997,6 +997,7 @@ ff_status ff_ad_level_forward(const ff_ad_level* level, int iterations, int smoo
             need(p, "argument");
         if (delta) {
             dims(B, Hu, Wu);
+            if (!ad::steps_supported(Hu, Wu)) throw invalid_argument("the upper flow image must be smaller than 2 GiB");
             for (const void* p : {(const void*)l.upper, (const void*)l.xmap, (const void*)l.ymap,
                                   (const void*)l.dflow_out})
                 need(p, "argument of a delta level");
