@@ -113,9 +113,9 @@ class FilterSpec(object):
 
     @property
     def tiled(self):
-        """Whether each level of a frame can run in one launch: image size and
-        iterations (also of a spec that was copied, loaded or changed)."""
-        return all(N.get_int("ff_ad_level_supported", lv["H"], lv["W"], lv["N"], lv["K"]) for lv in self.levels)
+        """Whether the levels of a frame can run in the tile kernels: image sizes
+        (also of a spec that was copied, loaded or changed)."""
+        return all(_tiled(lv["H"], lv["W"]) for lv in self.levels)
 
 
 # Iterations that one launch of the tile kernels takes, and whether they
@@ -189,22 +189,41 @@ def _propagate(fields, iterations, dt, border, B, h, w, save, s):
     return (f, sc, vc), passes
 
 
-def _last_iterations(pixels, n, save):
-    """Propagation iterations of a level that run in the launch of its image
-    model, update and smoothing; those before run in launches of their own.
+def _level_tiles(B, h, w, n, K):
+    """Workgroups of a level's launch with n propagation and K smoothing
+    iterations: buffers of 64 x 64 pixels with a halo of max(n, 2) + 2 K."""
+    inner = 64 - 2 * (max(n, 2) + 2 * K)
+    if inner <= 0:
+        return 1 << 31  # no launch takes them
+    across, down = (1 if size <= 64 else -(-size // inner) for size in (w, h))
+    return B * across * down
 
-    Iterations widen the halo of the tiles (2 + 2 K without any), which the
-    smoothing's passes then cover too, but save a pass over the fields. Of 8
-    at 3840x2160, two smoothing iterations: all in the launch 338 us, 4 of them
-    116 + 193, none 2 x 116 + 95, 2 of them 361; of 4 at 16 x 512x512: all 101,
-    none 70 + 47. With what the adjoints read written as well, none is best
-    (2 x 140 + 117 us, and 4 of 8 in the launch 140 + 340), except on images so
-    small that a launch costs more than its work."""
-    if pixels < 1 << 18:
-        return n
+
+def _in_launch(B, h, w, n, K, save):
+    """How many of a level's n propagation and K smoothing iterations run in the
+    launch of its image model and update (the last and the first of them); the
+    others run in launches of their own, up to four each.
+
+    Each widens the halo of that launch's tiles but saves a pass over the fields.
+    While the workgroups, however much they overlap, find place on the 256 CUs
+    at once (two a CU), the halo costs nothing: all. Past that the work grows
+    with it, from 2.6 times the pixels at a halo of 12 to 256 times at 30 (one
+    600x400 frame, n = 28, K = 1: 1620 us with all in the launch, 135 with 8
+    iterations; 3840x2160, n = 4, K = 12: 6.6 ms and 0.46). Images so small that
+    launches cost more than their work then take a halo of 16 (600x400, n = 16,
+    K = 6: 104 us, 120 with 4 and 2). On larger ones 4 iterations and 2 are best
+    (3840x2160, n = 16, K = 6: 675 us, 734 with 4 and 4, 832 with 8 and 4, 692
+    with none and 2; with n up to 6, all of them instead of 4: n = 4, K = 2: 277
+    us, 305 with none); with what the adjoints read written as well, no
+    propagation (forward and backward of n = 4, K = 4: 1450 us a frame, 1505
+    with 4 and 2)."""
+    if _level_tiles(B, h, w, n, K) <= 512:
+        return n, K
+    if B * h * w < 1 << 18:
+        return min(n, 8), min(K, 4)
     if save:
-        return 0
-    return n if n <= 6 else 4
+        return 0, min(K, 4)
+    return (n if n <= 6 else 4), min(K, 2)
 
 
 class _Level(ctypes.Structure):  # ff_ad_level
@@ -215,9 +234,9 @@ class _Level(ctypes.Structure):  # ff_ad_level
 
 
 def _level_forward(spec, l, image, state, upper, gamma, save, want_upd, s):
-    """One level of a frame after the first: the propagation's first
-    iterations in launches of their own, the rest of them and all that follows
-    in one. Returns the new state, the unsmoothed flow (top level, want_upd),
+    """One level of a frame after the first: the propagation's first iterations
+    and the smoothing's last in launches of their own, the rest of them and all
+    between in one. Returns the new state, the unsmoothed flow (top level, want_upd),
     and with `save` the image gradient, the propagated fields and the
     propagation's inputs as _frame_forward keeps them."""
     B, h, w = image.shape
@@ -226,7 +245,7 @@ def _level_forward(spec, l, image, state, upper, gamma, save, want_upd, s):
     new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=image.device)
     vec, sca = (lambda: new(B, h, w, 2)), (lambda: new(B, h, w))
     ptrs = lambda ts: [t.data_ptr() if t is not None else None for t in ts]
-    n = _last_iterations(B * h * w, lv["N"], save)
+    n, K = _in_launch(B, h, w, lv["N"], lv["K"], save)
     fields = (state["f"], state["a0"] if delta else None, state["d"] if delta else None)
     passes = []
     if n < lv["N"]:
@@ -258,8 +277,8 @@ def _level_forward(spec, l, image, state, upper, gamma, save, want_upd, s):
                 passes.append((min(2, n - 2 * (k + 1)),) + tuple(t[k] if t is not None else None for t in mid))
             fields = (None, sca(), vec()) if delta else (vec(), None, None)
             a.prop_flow, a.prop_scalar, a.prop_vector = ptrs(fields)
-    N.call("ff_ad_level_forward", ctypes.byref(a), n, lv["K"], B, h, w, hu, wu, lv["dt"], spec.border, gamma,
-           lv["maxflow"], s)
+    N.call("ff_ad_level_forward", ctypes.byref(a), n, K, B, h, w, hu, wu, lv["dt"], spec.border, gamma, lv["maxflow"], s)
+    st["f"] = _smooth(st["f"], lv["K"] - K, B, h, w, s)
     return st, upd, grad, fields, passes
 
 
