@@ -98,9 +98,9 @@ struct LevelJob {
     int delta, img_mode, first_block;
     // wait_job >= 0: wait for tiles of that job of the table, which has
     // wait_tx tiles across and its first tile's flags at wait_flags. Which
-    // of them: the first and last row (low and high half of the word
-    // wait_rows + r of the block map) for this job's tile row r, and the
-    // columns (word wait_rows + tiles_y + c) for its tile column c. flags
+    // of them: the first and last row (words wait_rows + 2 r and + 2 r + 1 of
+    // the block map) for this job's tile row r, and the first and last column
+    // (from word wait_rows + 2 (tiles_y + c)) for its tile column c. flags
     // >= 0: the job's tiles are waited for; tile t's flags are at flags + t.
     // frame_slot >= 0: the level's image is a filter's input frame, which a
     // launch may pass in place as its frame frame_slot (read where the
@@ -181,11 +181,11 @@ struct UpperTiles {
 };
 __device__ __forceinline__ UpperTiles upper_tiles(const LevelJob& p, int t) {
     const int ty = t / p.tiles_x, tx = t - ty * p.tiles_x;
-    const auto* w = (const FF_CONSTANT unsigned*)launch_args().block_job + p.wait_rows;
-    const unsigned rows = w[ty], cols = w[p.tiles_y + tx];
-    const int ty0 = (int)(rows & 0xffffu), tx0 = (int)(cols & 0xffffu);
-    const int nx = (int)(cols >> 16) - tx0 + 1;
-    return UpperTiles{ty0 * p.wait_tx + tx0, nx, ((int)(rows >> 16) - ty0 + 1) * nx};
+    const auto* w = (const FF_CONSTANT int*)launch_args().block_job + p.wait_rows;
+    const auto *rows = w + 2 * ty, *cols = w + 2 * (p.tiles_y + tx);
+    const int ty0 = rows[0], ty1 = rows[1], tx0 = cols[0], tx1 = cols[1];
+    const int nx = tx1 - tx0 + 1;
+    return UpperTiles{ty0 * p.wait_tx + tx0, nx, (ty1 - ty0 + 1) * nx};
 }
 
 // Wait for the tiles u of the upper level. Waiting for these few alone lets a
@@ -880,7 +880,8 @@ int FusedFrame::Impl::table(const std::vector<LevelArgs>& jobs, int nw, int rtop
         auto ranges = [&](int tiles, int size, int n, int nu, int upper_size) {
             for (int i = 0; i < tiles; ++i) {
                 const int lo = std::max(i * size - 2 * c.K, 0), hi = std::min(std::min(i * size + size, n) - 1 + 2 * c.K, n - 1);
-                map.push_back(upper_index(lo, n, nu) / upper_size | (upper_index(hi, n, nu) / upper_size) << 16);
+                map.push_back(upper_index(lo, n, nu) / upper_size);
+                map.push_back(upper_index(hi, n, nu) / upper_size);
             }
         };
         ranges(c.tiles_y, c.TH, c.H, q.H, q.TH);
