@@ -65,6 +65,7 @@
 
 #include "ff_device.hpp"
 #include "ff_kernels.hpp"
+#include "ff_per_device.hpp"
 #include "ff_runtime.hpp"
 #include "ff_tile.hpp"
 
@@ -955,19 +956,15 @@ void FusedFrame::Impl::run(int ti, hipStream_t s, const FrameRef* frames, int nf
     const int si = ti & 1;
     const Table& t = slot[si];
     if (!t.blocks) throw logic_error("fused frame: launch of an unprepared table");
-    static const hipError_t lds_ok4 = hipFuncSetAttribute(
-        (const void*)k_fused_frame<4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(kMaxWaves));
-    static const hipError_t lds_ok8 = hipFuncSetAttribute(
-        (const void*)k_fused_frame<8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(kMaxWaves));
-    static const hipError_t lds_ok44 = hipFuncSetAttribute(
-        (const void*)k_fused_frame<4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(kMaxWaves));
-    static const hipError_t lds_ok44i = hipFuncSetAttribute((const void*)k_fused_frame<4, 4, true>,
-                                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                            (int)lds_bytes(kMaxWaves));
-    if (lds_ok4 != hipSuccess) throw_hip(lds_ok4, "hipFuncSetAttribute", __FILE__, __LINE__);
-    if (lds_ok8 != hipSuccess) throw_hip(lds_ok8, "hipFuncSetAttribute", __FILE__, __LINE__);
-    if (lds_ok44 != hipSuccess) throw_hip(lds_ok44, "hipFuncSetAttribute", __FILE__, __LINE__);
-    if (lds_ok44i != hipSuccess) throw_hip(lds_ok44i, "hipFuncSetAttribute", __FILE__, __LINE__);
+    // (the limit of the dynamic LDS is a device's)
+    int dev = 0;
+    FF_HIP(hipGetDevice(&dev));
+    static OncePerDevice once;
+    once.run(dev, [] {
+        for (const void* k : {(const void*)k_fused_frame<4>, (const void*)k_fused_frame<8>,
+                              (const void*)k_fused_frame<4, 4>, (const void*)k_fused_frame<4, 4, true>})
+            FF_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(kMaxWaves)));
+    });
     // Sequence number of this launch for its slot's flags. A launch recorded
     // into a graph clears them itself and counts as the first, so every
     // replay is self-contained; direct launches count up from the last

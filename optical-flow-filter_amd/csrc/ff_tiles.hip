@@ -17,6 +17,7 @@
 
 #include "ff_device.hpp"
 #include "ff_kernels.hpp"
+#include "ff_per_device.hpp"
 #include "ff_runtime.hpp"
 #include "ff_tile.hpp"
 
@@ -606,12 +607,16 @@ __global__ void __launch_bounds__(1024, 8) k_lax_wendroff_tile(DevImg flow, DevI
 
 size_t exchange_bytes(int nw) { return (size_t)2 * nw * 10 * LANES * sizeof(float); }
 
-// The dynamic LDS of a launch is above the default limit.
-template <class K>
-void allow_lds(K kernel) {
-    const hipError_t e =
-        hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)exchange_bytes(16));
-    if (e != hipSuccess) throw_hip(e, "hipFuncSetAttribute", __FILE__, __LINE__);
+// The dynamic LDS of a launch is above the default limit, which is lifted for
+// each kernel on each device.
+template <class... K>
+void allow_lds(OncePerDevice& once, K... kernels) {
+    int dev = 0;
+    FF_HIP(hipGetDevice(&dev));
+    once.run(dev, [&] {
+        for (const void* k : {(const void*)kernels...})
+            FF_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)exchange_bytes(16)));
+    });
 }
 
 bool fits(long long pitch, int H) { return pitch * H < 0x7fffffffLL; }
@@ -626,12 +631,8 @@ bool propagate_tile_supported(const PropFields& in, const PropFields& out, int H
 void launch_propagate_tile(const PropFields& in, const PropFields& mid, int after, const PropFields& out, int n, int B,
                            int H, int W, float dt, int border, hipStream_t s) {
     if (n < 1 || n > kMaxPropIters) throw logic_error("propagation: iterations of one launch out of range");
-    static const bool once = [] {
-        allow_lds(k_propagate_tile<true>);
-        allow_lds(k_propagate_tile<false>);
-        return true;
-    }();
-    (void)once;
+    static OncePerDevice once;
+    allow_lds(once, k_propagate_tile<true>, k_propagate_tile<false>);
     const int nw = waves_for(B, H, W, n);
     const Tiling tl = tiling(H, W, n, nw * kTileRows);
     const dim3 grid(tl.tiles_x * tl.tiles_y, B), blk(nw * LANES);
@@ -661,18 +662,10 @@ bool level_tile_supported(int H, int W, int n, int K) {
 void launch_level_tile(const LevelFields& f, int B, int H, int W, int Hu, int Wu, int n, int K, int border, float dt,
                        float gamma, float maxflow, hipStream_t s) {
     if (!level_tile_supported(H, W, n, K)) throw logic_error("level: iterations or size of one launch out of range");
-    static const bool once = [] {
-        allow_lds(k_level_tile<true, true, true>);
-        allow_lds(k_level_tile<true, false, true>);
-        allow_lds(k_level_tile<false, true, true>);
-        allow_lds(k_level_tile<false, false, true>);
-        allow_lds(k_level_tile<true, true, false>);
-        allow_lds(k_level_tile<true, false, false>);
-        allow_lds(k_level_tile<false, true, false>);
-        allow_lds(k_level_tile<false, false, false>);
-        return true;
-    }();
-    (void)once;
+    static OncePerDevice once;
+    allow_lds(once, k_level_tile<true, true, true>, k_level_tile<true, false, true>, k_level_tile<false, true, true>,
+              k_level_tile<false, false, true>, k_level_tile<true, true, false>, k_level_tile<true, false, false>,
+              k_level_tile<false, true, false>, k_level_tile<false, false, false>);
     const int halo = level_halo(n, K), nw = level_waves(B, H, W, halo);
     const Tiling tl = tiling(H, W, halo, nw * kTileRows);
     const dim3 grid(tl.tiles_x * tl.tiles_y, B), blk(nw * LANES);
@@ -693,11 +686,8 @@ void launch_level_tile(const LevelFields& f, int B, int H, int W, int Hu, int Wu
 void launch_smooth_tile(const void* in, int in_pitch, void* out, int out_pitch, int n, int B, int H, int W,
                         hipStream_t s) {
     if (n < 1 || n > kMaxSmoothIters) throw logic_error("smoothing: iterations of one launch out of range");
-    static const bool once = [] {
-        allow_lds(k_smooth_tile);
-        return true;
-    }();
-    (void)once;
+    static OncePerDevice once;
+    allow_lds(once, k_smooth_tile);
     const int nw = waves_for(B, H, W, 2 * n);
     const Tiling tl = tiling(H, W, 2 * n, nw * kTileRows);
     hipLaunchKernelGGL(k_smooth_tile, dim3(tl.tiles_x * tl.tiles_y, B), dim3(nw * LANES), exchange_bytes(nw), s,
@@ -715,11 +705,8 @@ void launch_image_model_adjoint(const float* ga0, const float* gg, float* gI, in
 void launch_smooth_adjoint(const float* gout, const float* gout2, float* gin, int n, int B, int H, int W, int acc,
                            hipStream_t s) {
     if (n < 1 || n > kMaxSmoothIters) throw logic_error("smoothing adjoint: iterations of one launch out of range");
-    static const bool once = [] {
-        allow_lds(k_smooth_adjoint);
-        return true;
-    }();
-    (void)once;
+    static OncePerDevice once;
+    allow_lds(once, k_smooth_adjoint);
     const int nw = waves_for(B, H, W, 2 * n);
     const Tiling tl = tiling(H, W, 2 * n, nw * kTileRows);
     hipLaunchKernelGGL(k_smooth_adjoint, dim3(tl.tiles_x * tl.tiles_y, B), dim3(nw * LANES),

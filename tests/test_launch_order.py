@@ -1,5 +1,6 @@
-"""Order of fused launches on several streams: the bookkeeping on the CPU, and
-on the GPU what it counts against what the launches did."""
+"""Order of fused launches on several streams: the bookkeeping on the CPU (also
+that of set-up once per device), and on the GPU what it counts against what the
+launches did."""
 import ctypes
 import os
 import shutil
@@ -11,14 +12,15 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_bookkeeping(tmp_path):
+@pytest.mark.parametrize("program", ["launch_order", "per_device"])
+def test_bookkeeping(tmp_path, program):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
-    exe = str(tmp_path / "launch_order")
-    subprocess.check_call([gxx, "-std=c++17", "-O1", "-Wall", "-Werror",
+    exe = str(tmp_path / program)
+    subprocess.check_call([gxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-pthread",
                            "-I" + os.path.join(ROOT, "optical-flow-filter_amd", "csrc"),
-                           os.path.join(ROOT, "tests", "cpp", "launch_order.cpp"), "-o", exe])
+                           os.path.join(ROOT, "tests", "cpp", program + ".cpp"), "-o", exe])
     subprocess.check_call([exe], timeout=60)
 
 
