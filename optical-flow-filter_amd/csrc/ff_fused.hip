@@ -393,9 +393,7 @@ __device__ __forceinline__ void finish_image(const ImageRegs<MODE, R>& ir, float
 // first). Other tiles choose per wave.
 // t: the tile, row by row from the top.
 template <bool DELTA, int MODE, int R, bool ALLOW_INNER, bool INNER = false>
-__device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch, int nw,
-                                           ImgSrc frame) {
-    
+__device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch, int nw, ImgSrc frame) {
     Geo g;
     // the lane from the hardware's count, so that threadIdx.x takes no
     // register beyond the next line
@@ -469,7 +467,6 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
 
     int slot = 0;
 
-    {
     // ---------------------------------------------------------- propagation
     // N iterations of an X and a Y pass; the last one separately, since on
     // a delta level part of its flow output is dead
@@ -489,14 +486,11 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
     for (int it = 0; it + 1 < p.N; ++it) iteration(std::false_type{});
     iteration(std::true_type{});
 
-    }
     // ------------------------------------------------ image model + update
-    {
     if (DELTA && p.wait_job >= 0) wait_upper(p, u, g);
     float aold[R];  // unused (and removed) on delta levels
     float2 up[R];
     int offa[R], offf[R];
-    const Rsrc rai = rsrc(p.a0_in, p.a0_in_pitch * p.H);
     const Rsrc rao = rsrc(p.a0_out, p.a0_out_pitch * p.H);
     const Rsrc rdf = rsrc(p.dflow_out, p.dflow_out_pitch * p.H);
     const Rsrc rfu = rsrc(p.flow_upd, p.flow_upd_pitch * p.H);
@@ -514,7 +508,8 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
             aold[r] = 0.f;
         } else {
             offf[r] = out ? y * p.flow_upd_pitch + g.x * 8 : OOB;
-            aold[r] = ld1(rai, yl * p.a0_in_pitch + g.xl * 4);
+            // (looked up anew: held from the start it spills)
+            aold[r] = ld1(rsrc(p.a0_in, p.a0_in_pitch * p.H), yl * p.a0_in_pitch + g.xl * 4);
             up[r] = make_float2(0.f, 0.f);
         }
     }
@@ -524,7 +519,6 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
     if (!INNER && xedge) model_update<DELTA, true, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf, none);
     else model_update<DELTA, false, R>(s, im, aold, up, p, rao, rdf, rfu, offa, offf, none);
 
-    }
     // ------------------------------------------------------------ smoothing
     // flowSmoothX_k / flowSmoothY_k (flowsmoothing_k.cu:21-87), K times.
     for (int it = 0; it < p.K; ++it) {
@@ -537,9 +531,8 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
         else smooth_y<false, R>(s.fu, s.fv, e, rlast);
     }
 
-    {
-    const Rsrc rfo = rsrc(p.flow_out, p.flow_out_pitch * p.H);
     // ------------------------------------------------- write the new state
+    const Rsrc rfo = rsrc(p.flow_out, p.flow_out_pitch * p.H);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int y = g.yw + r;
@@ -547,7 +540,6 @@ __device__ __forceinline__ void level_tile(const LevelJob& p, int t, float* xch,
         st2(rfo, out ? y * p.flow_out_pitch + g.x * 8 : OOB, s.fu[r], s.fv[r]);
     }
     if (!DELTA && p.flags >= 0) signal_done(p, t, g);
-    }
 }
 
 // Rows per thread of a tile body: RLOW, except for top levels reduced on

@@ -4,7 +4,7 @@
 //
 // One launch per X or Y pass reads and writes every field once per pass, 2 n
 // times for n iterations, with a launch's latency each. Here a workgroup loads
-// a buffer of 64 columns by waves * 4 rows once, runs up to kMaxIters
+// a buffer of 64 columns by waves * 4 rows once, runs the
 // iterations in registers, and writes the tile inside it that neighbouring
 // pixels beyond the buffer cannot have reached. The iterations cost VALU
 // instructions and a barrier each (plus those of the halo), so a launch is
@@ -82,7 +82,6 @@ __device__ __forceinline__ TilePos tile_pos(const Tiling& t, int nw, int border)
     g.xlast = t.W - 1 - p.x0;
     g.yw = p.y0 + g.wave * R;
     g.xin = g.x >= border && g.x < t.W - border;
-    g.wave_in = p.x0 >= border && p.x0 + LANES - 1 < t.W - border && g.yw >= border && g.yw + R - 1 < t.H - border;
     p.xedge = p.x0 == 0 || p.x0 + LANES >= t.W;
     p.xinside = g.xlast < LANES - 1;
     p.yinside = p.y0 + nw * R > t.H;
