@@ -746,6 +746,7 @@ bool launch_propagate(const PropFields& in, const PropFields& x, const PropField
 
 bool launch_smooth(const DevImg& in, const DevImg& x, const DevImg& y, int n, hipStream_t s) {
     const int H = in.h, W = in.w;
+    // (FlowSmoother's buffers are new with every input, so none is its input)
     if (H <= 0 || W <= 0 || in.data == x.data || in.data == y.data) return false;
     for (const DevImg* d : {&in, &x, &y})
         if (!fits((long long)d->pitch, H)) return false;

@@ -105,3 +105,26 @@ def test_rows_of_two_gib(ffo):
     m = FlowSmoother(img, 2)
     m.compute()
     check(m.getSmoothedFlow(), lambda a: ffo.smooth(a, 2))
+
+
+@pytest.mark.parametrize("n", [1, 3, 9])
+def test_lax_wendroff_of_its_own_output(ffo, n):
+    """A Lax-Wendroff propagator fed its own output buffer (set after it was
+    made) reads all of it before it is overwritten, frame after frame."""
+    from flowfilter.gpu.image import GPUImage
+    from flowfilter.gpu.propagation import LaxWendroffPropagator
+    print("own output", n, flush=True)
+    rng = np.random.default_rng(n)
+    h, w = 70, 150
+    f = (rng.standard_normal((h, w, 2)) * 0.3).astype(np.float32)
+    a = rng.random((h, w), np.float32)
+    flow, img = GPUImage((h, w, 2), 4), GPUImage((h, w), 4)
+    flow.upload(f)
+    img.upload(a)
+    p = LaxWendroffPropagator(flow, img)
+    p.iterations = n
+    for _ in range(3):
+        p.compute()
+        a = ffo.lax_wendroff(f, a, n)
+        assert np.array_equal(p.getPropagatedImage().download(np.float32), a)
+        p.setInputImage(p.getPropagatedImage())
