@@ -228,9 +228,9 @@ struct AwaitedTiles {
 // launch before instead, three filters on streams of their own took 81 us per
 // 2048x1088 two-level frame, for a launch of 55 us.)
 //
-// The poll alone would have no bound: what its stream has queued before a
-// launch may take any time (a caller's stream with work of its own). With the
-// event it spans the launch's start only. It still gives up after the waits'
+// The poll alone would have no bound: what lies before a launch may take any
+// time (work of the caller's on its stream, or on any stream that shares its
+// hardware queue). With the event it spans the launch's start only. It still gives up after the waits'
 // spin limit of 2 s, when other kernels have held the GPU all that time; the
 // launch behind it then goes, its filter's next check is an error, and the
 // next launch of any filter waits for the device.

@@ -106,7 +106,8 @@ struct PassParams {
 // payload; with a middle output, the fields after `mid` iterations are written
 // too. Needs border >= 1: the pixels next to an image edge then keep their
 // values, so the lanes and rows beyond the image are never read by others.
-// Four iterations with payloads at 3840x2160: see kMaxPropIters.
+// Four iterations with payloads at 3840x2160: 116 us for 332 MB (66 us at a
+// copy's rate; the rest is VALU), 138 us with the middle output's 166 MB.
 template <bool PAY>
 __global__ void __launch_bounds__(1024, 8) k_propagate_tile(PropFields in, PropFields mid, PropFields out, Tiling tl,
                                                             int n, int after, float dt, int border) {
