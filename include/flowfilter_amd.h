@@ -499,12 +499,14 @@ FF_API ff_status ff_batch_get_blocks(ff_stage* batch, int* out);
  * backwards' gamma gradient (g_gamma_partial holds B times this). */
 FF_API ff_status ff_ad_partial_count(int height, int width, int* out);
 /* Image model (imagemodel_k.cu:31-133): a0 and grad (gx, gy) of a float
- * image. Backward: work holds 2*B*H*W floats. */
+ * image. Backward: work holds 2*B*H*W floats, used only where
+ * g_image overlaps g_a0 or g_grad. */
 FF_API ff_status ff_ad_image_model(const float* image, float* a0, float* grad, int B, int H, int W, void* stream);
 FF_API ff_status ff_ad_image_model_backward(const float* g_a0, const float* g_grad, float* g_image, float* work, int B,
                                             int H, int W, int accumulate, void* stream);
 /* One float pyramid step (pyramid_k.cu:81-145): half is (H/2) x (W/2);
- * work holds B*H*(W/2) floats. */
+ * work holds B*H*(W/2) floats (ff_ad_down uses it only where half overlaps
+ * image). */
 FF_API ff_status ff_ad_down(const float* image, float* half, float* work, int B, int H, int W, void* stream);
 FF_API ff_status ff_ad_down_backward(const float* g_half, float* g_image, float* work, int B, int H, int W,
                                      int accumulate, void* stream);

@@ -309,8 +309,8 @@ def _frame_forward(spec, state, image, gammas, save):
     for l in range(1, L):
         h, w = spec.sizes[l - 1]
         out = _empty(B, h // 2, w // 2, like=image)
-        work = _empty(B, h, w // 2, like=image)
-        N.call("ff_ad_down", _p(imgs[-1]), _p(out), _p(work), B, h, w, s)
+        # (no work buffer: it is used only where the result overlaps the image)
+        N.call("ff_ad_down", _p(imgs[-1]), _p(out), _p(out), B, h, w, s)
         imgs.append(out)
     if state is not None and spec.tiled:
         return _frame_levels(spec, state, imgs, gammas, save)
@@ -517,8 +517,8 @@ def _frame_backward(spec, saved, g_new, g_out, gammas, g_image_out):
     for l in range(L):
         h, w = spec.sizes[l]
         gi = g_image_out if l == 0 else _empty(B, h, w, like=g_a0[l])
-        work = _empty(B, 2 * h, w, like=g_a0[l])
-        N.call("ff_ad_image_model_backward", _p(g_a0[l]), _p(g_g[l]), _p(gi), _p(work), B, h, w, 0, s)
+        # (no work buffer: it is used only where the result overlaps an input)
+        N.call("ff_ad_image_model_backward", _p(g_a0[l]), _p(g_g[l]), _p(gi), _p(gi), B, h, w, 0, s)
         g_img[l] = gi
     for l in range(L - 1, 0, -1):
         h, w = spec.sizes[l - 1]

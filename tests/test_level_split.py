@@ -52,3 +52,22 @@ def test_split_levels_match_the_stages(monkeypatch, B, h, w, levels, maxflow, sm
     want = run()
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_window_allocates_no_unused_work_buffers(monkeypatch):
+    """The image model's adjoint and the pyramid's reduction use a work buffer
+    only where a result overlaps an input, which a window never asks for: none is
+    allocated for them (the pyramid's adjoint does use its own)."""
+    import torch
+    from flowfilter import autograd as A
+    shapes, inner = [], A._empty
+    monkeypatch.setattr(A, "_empty", lambda *a, **k: shapes.append(a) or inner(*a, **k))
+    B, T, h, w = 2, 3, 64, 80
+    frames = torch.rand(B, T, h, w, device="cuda", requires_grad=True)
+    out = A.flow_window(frames, torch.tensor([10.0, 50.0], device="cuda"), A.FilterSpec(h, w, 2, maxflow=2.0))
+    forward, shapes[:] = list(shapes), []
+    assert (B, h, w // 2) not in forward and (B, h // 2, w // 2) in forward
+    out.sum().backward()
+    assert shapes.count((B, h, w // 2)) == T  # the pyramid's adjoint
+    assert (B, 2 * h, w) not in shapes and (B, h, w) in shapes
