@@ -528,9 +528,10 @@ WaitingLaunch::WaitingLaunch(hipStream_t s, const AwaitedTiles& awaited) : s_(s)
     const auto before = w.order.before(s);
     if (before != LaunchOrder::Before::NOTHING) {
         const bool live = g.owned.count(last) && !capturing(last);
-        const bool idle = live && hipStreamQuery(last) == hipSuccess;
+        // (a poll that gave up just now proves nothing about those before it)
+        const bool idle = live && hipStreamQuery(last) == hipSuccess && !*w.gave_up;
         if (idle) {
-            // it is done
+            // it is done, and so are those that it waited for
         } else if (before == LaunchOrder::Before::GATE) {
             FF_HIP(hipStreamWaitEvent(s, w.mark, 0));
             launch_wait_started(w.word, w.order.target + awaited.bias, awaited.spin_limit, awaited.timeouts,
