@@ -227,3 +227,32 @@ def test_a_wait_for_another_streams_launch_that_gives_up_is_an_error(ffo):
     assert a.waitTimeouts() == 0
     st = _order_state()
     assert st[0] == st[1] and st[2] == gave_up + 1
+
+
+@pytest.mark.gpu
+def test_backlogs_on_streams_that_share_hardware_queues(ffo):
+    """More filters on streams of their own than the process has hardware
+    queues, while other streams, which share those queues, hold half a second of
+    work each: no wait gives up and every flow is the oracle's."""
+    import torch
+    h, w = 272, 512
+    fs = [_pyr(h, w) for _ in range(10)]
+    o = ffo.PyramidalFlowFilter(h, w, 2)
+    o.configure_like([10.0, 30.0], 4.0, [2, 2])
+    gave_up = _order_state()[2]
+    others = [torch.cuda.Stream() for _ in range(6)]
+    for t, img in enumerate(_frames(h, w, 6, 21)):
+        if t in (3, 5):
+            print("backlogs at frame", t, flush=True)
+            for s in others:
+                _backlog(s, 0.5)
+        for f in fs:
+            f.loadImage(img)
+        for f in fs:
+            f.compute()
+        o.compute(img)
+    for k, f in enumerate(fs):
+        assert np.array_equal(f.getFlow(), o.downloadFlow()), k
+        assert f.waitTimeouts() == 0, k
+    st = _order_state()
+    assert st[0] == st[1] and st[2] == gave_up
